@@ -35,7 +35,7 @@ VERSION = 2
 COL_WIDTHS = (1, 2, 4, 8, 16, 32)
 GRAPH_CHUNKS = (0, 8, 16, 32)
 BATCH_GRIDS = ((2, 1), (4, 2), (8, 2), (4, 1), (8, 1), (8, 4), (16, 1))
-ROW_POINTS = (8, 16)
+ROW_POINTS = (0, 8, 16)
 
 
 def cache_path() -> str:

@@ -4,12 +4,15 @@
 // batch.
 //
 // Work units are uniform in size whatever the grid: a row unit is
-// 4096/NX rows of NX points (256 threads) and a column
-// unit is 8192/NY columns of NY points (256 threads, two columns each).  Every unit therefore
-// moves the same bytes and does the same FFT work per point, and a
-// persistent grid that strides over the unit list is balanced without a
-// work queue.  Each block reads its unit's instance descriptor (field
-// pointer, tables, parameters) and runs the sweep body of that line length.
+// 4096/NX rows of NX points (256 threads) and a column unit is 8192/NY
+// columns of NY points (512 threads).  Every unit therefore moves the same
+// bytes and does the same FFT work per point, and a persistent grid that
+// strides over the unit list is balanced without a work queue.  Each block
+// reads its unit's instance descriptor (field pointer, tables, parameters) and
+// runs the sweep body of that line length, in the plan (points per thread,
+// exchange precision) of the member's own single-field run: small members
+// (SMALL_FIELD) take the small-field plans, so every member gives bit for bit
+// the result of its own run.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,6 +31,7 @@ struct BatchInst {
   ColArgs col;
   const void* nl[3];  // NLParams1 of the three slots
   int nx, ny;
+  int small;  // SMALL_FIELD
   float inv_nx, inv_ny;
 };
 
@@ -43,98 +47,48 @@ struct BatchFlags {
 };
 
 constexpr int BROW_THREADS = 256;
-// A column unit of 8192/NY columns is 512 lines of work: 512 threads with
-// one column each, or (NLSE_BATCH_COL_PAIRED) 256 threads owning two
-// adjacent columns each, moved with 16-byte accesses.  With FP64 stages the
-// paired form needs all 256 VGPRs plus AGPRs (one wave per SIMD, one
-// 4-wave block per CU); one column per thread takes 206-232 VGPRs (two
-// waves per SIMD): the 64-field workload's column sweep 253 -> 224 us.
-#ifndef NLSE_BATCH_COL_PAIRED
-#define NLSE_BATCH_COL_PAIRED 0
-#endif
-constexpr int BCOL_UNIT = 512;
-constexpr int BCOL_G = NLSE_BATCH_COL_PAIRED ? 2 : 1;
-constexpr int BCOL_THREADS = BCOL_UNIT / BCOL_G;
+constexpr int BCOL_THREADS = 512;
 
-// Row units of 4096/NX rows run as PASSES row_body calls of LPB rows with
-// the per-thread set size of the single-field row kernel of that length
-// (LineCfg::PR), so a batch member is transformed in the same radix plan
-// and gives bit for bit the result of its own plan's run.
-template <int N>
+// Row units of 4096/NX rows run as PASSES row_body calls of LPB rows.
+template <int N, bool SMALL>
 struct BRow {
-  static constexpr int P = LineCfg<N>::PR;
+  using C = LineCfg<N>;
+  static constexpr int P = SMALL ? C::PRS : C::PR;
+  static constexpr int AR = SMALL ? C::ARS : F64;
   static constexpr int T = N / P;
-  static constexpr int LPB = BROW_THREADS / T;
+  static constexpr int LPB = BROW_THREADS / T < 4096 / N ? BROW_THREADS / T : 4096 / N;
+  static constexpr int THREADS = LPB * T;
   static constexpr int PASSES = (4096 / N) / LPB;
-  static constexpr int LDS = row_lds_size<N, LPB, 1>();
+  static constexpr int LDSB = row_lds_size<N, LPB, 1>() * (int)sizeof(xchg_t<AR>);
+  static_assert(THREADS == BROW_THREADS, "one block size for every length");
 };
 
-template <int N>
+// Column units of 8192/NY columns run as PASSES tiles of WT columns.
+template <int N, bool SMALL>
 struct BCol {
-  static constexpr int T = N / 16;
-  static constexpr int WT = BCOL_THREADS / T;  // threads across; W = WT * BCOL_G columns
-  static constexpr int LDS = col_lds_size<N, WT, BCOL_G>();
+  using C = LineCfg<N>;
+  static constexpr int P = SMALL ? C::PS : C::P;
+  static constexpr int AR = SMALL ? C::ARS : F64;
+  static constexpr int T = N / P;
+  static constexpr int W = 8192 / N;
+  static constexpr int WT = BCOL_THREADS / T < W ? BCOL_THREADS / T : W;
+  static constexpr int PASSES = W / WT;
+  static constexpr int LDSB = col_lds_size<N, WT, 1>() * (int)sizeof(xchg_t<AR>);
+  static_assert(WT * T == BCOL_THREADS, "one block size for every length");
 };
 
 static bool batch_len_ok(int64_t n) { return n == 128 || n == 256 || n == 512 || n == 1024 || n == 2048; }
-static int len_index(int64_t n) { return n == 128 ? 0 : n == 256 ? 1 : n == 512 ? 2 : n == 1024 ? 3 : 4; }
-constexpr int NLEN = 5;
-
-// One persistent kernel per line length: a single length per kernel keeps
-// the register footprint of the plain sweeps (a kernel holding every
-// length spills).
-template <int N>
-__global__ __launch_bounds__(BROW_THREADS) void k_batch_row(const BatchInst* __restrict__ inst,
-                                                            const BatchUnit* __restrict__ units, int64_t nunits,
-                                                            BatchFlags f) {
-  __shared__ float2 lds[BRow<N>::LDS];
-  for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
-    const BatchUnit un = units[u];
-    const BatchInst& I = inst[un.inst];
-    RowArgs a = I.row;
-    a.inverse_first = f.inverse_first;
-    a.forward_last = f.forward_last;
-    a.has_a = f.has_a;
-    a.has_b = f.has_b;
-    a.nlp_a = I.nl[f.slot_a];
-    a.nlp_b = I.nl[f.slot_b];
-    a.out_scale = f.timing ? I.inv_nx : 1.f;
-#pragma unroll
-    for (int k = 0; k < BRow<N>::PASSES; ++k) {
-      row_body<N, BRow<N>::P, BRow<N>::LPB, 1>(a, un.first + k * BRow<N>::LPB, lds);
-      __syncthreads();
-    }
-  }
+// unit groups: line length, small-field plans or not
+static int len_index(int64_t n, bool small) {
+  return 2 * (n == 128 ? 0 : n == 256 ? 1 : n == 512 ? 2 : n == 1024 ? 3 : 4) + (small ? 1 : 0);
 }
+constexpr int NLEN = 10;
 
-template <int N>
-__global__ __launch_bounds__(BCOL_THREADS) void k_batch_col(const BatchInst* __restrict__ inst,
-                                                            const BatchUnit* __restrict__ units, int64_t nunits,
-                                                            BatchFlags f) {
-  __shared__ double2 lds2[BCol<N>::LDS / 2];
-  float2* lds = reinterpret_cast<float2*>(lds2);
-  // XCD-aware order: consecutive list entries (neighbouring column tiles,
-  // which share 128-byte lines when narrow) go to blocks on the same XCD
-  const int64_t grid = gridDim.x;
-  const int64_t bb = (grid % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (grid / 8) + blockIdx.x / 8 : blockIdx.x;
-  for (int64_t u = bb; u < nunits; u += grid) {
-    const BatchUnit un = units[u];
-    const BatchInst& I = inst[un.inst];
-    ColArgs c = I.col;
-    if (f.timing) c.scale = I.inv_ny;
-    col_body<N, 16, BCol<N>::WT, BCOL_G, BCOL_G, PROP_SEP64>(c, un.first, lds);
-    __syncthreads();
-  }
-}
-
-// One persistent launch per sweep for the whole batch, whatever the line
-// lengths: each unit's length picks the body (a block-uniform branch).  The
-// bodies are separate (not inlined) functions, so the kernel's register
-// allocation is the largest body's, not that of one giant inlined switch
-// (which spilled), and the LDS array is the largest length's.
-template <int N>
-__device__ __noinline__ void batch_row_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f,
-                                            float2* lds) {
+// One unit of a row or column sweep.  GEN: some member's loss varies from
+// point to point (see nl1_block_I).
+template <int N, bool SMALL, bool GEN>
+__device__ __forceinline__ void row_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
+  using B = BRow<N, SMALL>;
   RowArgs a = I.row;
   a.inverse_first = f.inverse_first;
   a.forward_last = f.forward_last;
@@ -143,61 +97,116 @@ __device__ __noinline__ void batch_row_unit(const BatchInst& I, const BatchUnit&
   a.nlp_a = I.nl[f.slot_a];
   a.nlp_b = I.nl[f.slot_b];
   a.out_scale = f.timing ? I.inv_nx : 1.f;
-#pragma unroll
-  for (int k = 0; k < BRow<N>::PASSES; ++k) {
-    row_body<N, BRow<N>::P, BRow<N>::LPB, 1>(a, un.first + k * BRow<N>::LPB, lds);
-    __syncthreads();
+#pragma unroll 1
+  for (int k = 0; k < B::PASSES; ++k)
+    row_body<N, B::P, B::LPB, 1, GEN, B::AR>(a, un.first + k * B::LPB, reinterpret_cast<xchg_t<B::AR>*>(lds));
+}
+
+template <int N, bool SMALL>
+__device__ __forceinline__ void col_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
+  using B = BCol<N, SMALL>;
+  ColArgs c = I.col;
+  if (f.timing) c.scale = I.inv_ny;
+#pragma unroll 1
+  for (int k = 0; k < B::PASSES; ++k)
+    col_body<N, B::P, B::WT, 1, 1, PROP_SEP64, B::AR>(c, un.first * B::PASSES + k,
+                                                      reinterpret_cast<xchg_t<B::AR>*>(lds));
+}
+
+// One persistent kernel per line length: a single length per kernel keeps
+// the register footprint of the plain sweeps (a kernel holding every
+// length spills).
+template <int N, bool SMALL, bool GEN>
+__global__ __launch_bounds__(BROW_THREADS) void k_batch_row(const BatchInst* __restrict__ inst,
+                                                            const BatchUnit* __restrict__ units, int64_t nunits,
+                                                            BatchFlags f) {
+  __shared__ double2 lds[BRow<N, SMALL>::LDSB / 16 + 1];
+  for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
+    const BatchUnit un = units[u];
+    row_unit<N, SMALL, GEN>(inst[un.inst], un, f, lds);
   }
 }
 
-template <int N>
-__device__ __noinline__ void batch_col_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f,
-                                            float2* lds) {
-  ColArgs c = I.col;
-  if (f.timing) c.scale = I.inv_ny;
-  col_body<N, 16, BCol<N>::WT, BCOL_G, BCOL_G, PROP_SEP64>(c, un.first, lds);
+// XCD-aware order: consecutive list entries (neighbouring column tiles,
+// which share 128-byte lines when narrow) go to blocks on the same XCD
+__device__ __forceinline__ int64_t xcd_block() {
+  const int64_t grid = gridDim.x;
+  return (grid % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (grid / 8) + blockIdx.x / 8 : blockIdx.x;
+}
+
+template <int N, bool SMALL>
+__global__ __launch_bounds__(BCOL_THREADS) void k_batch_col(const BatchInst* __restrict__ inst,
+                                                            const BatchUnit* __restrict__ units, int64_t nunits,
+                                                            BatchFlags f) {
+  __shared__ double2 lds[BCol<N, SMALL>::LDSB / 16 + 1];
+  for (int64_t u = xcd_block(); u < nunits; u += gridDim.x) {
+    const BatchUnit un = units[u];
+    col_unit<N, SMALL>(inst[un.inst], un, f, lds);
+  }
+}
+
+// One persistent launch per sweep for the whole batch, whatever the line
+// lengths: each unit's length picks the body (a block-uniform branch).  The
+// bodies are separate (not inlined) functions, so the kernel's register
+// allocation is the largest body's, not that of one giant inlined switch
+// (which spilled), and the LDS array is the largest length's.
+template <int N, bool SMALL, bool GEN>
+__device__ __noinline__ void batch_row_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
+  row_unit<N, SMALL, GEN>(I, un, f, lds);
+}
+
+template <int N, bool SMALL>
+__device__ __noinline__ void batch_col_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
+  col_unit<N, SMALL>(I, un, f, lds);
 }
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
-constexpr int BROW_LDS_ALL =
-    cmax(cmax(cmax(BRow<128>::LDS, BRow<256>::LDS), cmax(BRow<512>::LDS, BRow<1024>::LDS)), BRow<2048>::LDS);
-constexpr int BCOL_LDS_ALL =
-    cmax(cmax(cmax(BCol<128>::LDS, BCol<256>::LDS), cmax(BCol<512>::LDS, BCol<1024>::LDS)), BCol<2048>::LDS);
+template <template <int, bool> class B>
+constexpr int lds_all() {
+  return cmax(cmax(cmax(B<128, false>::LDSB, B<128, true>::LDSB), cmax(B<256, false>::LDSB, B<256, true>::LDSB)),
+              cmax(cmax(B<512, false>::LDSB, B<512, true>::LDSB), cmax(B<1024, false>::LDSB, B<2048, false>::LDSB)));
+}
 
+template <bool GEN>
 __global__ __launch_bounds__(BROW_THREADS) void k_batch_row_all(const BatchInst* __restrict__ inst,
                                                                 const BatchUnit* __restrict__ units, int64_t nunits,
                                                                 BatchFlags f) {
-  __shared__ double2 lds2[(BROW_LDS_ALL + 1) / 2];
-  float2* lds = reinterpret_cast<float2*>(lds2);
+  __shared__ double2 lds[lds_all<BRow>() / 16 + 1];
   for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
     const BatchUnit un = units[u];
     const BatchInst& I = inst[un.inst];
-    switch (I.nx) {
-      case 128: batch_row_unit<128>(I, un, f, lds); break;
-      case 256: batch_row_unit<256>(I, un, f, lds); break;
-      case 512: batch_row_unit<512>(I, un, f, lds); break;
-      case 1024: batch_row_unit<1024>(I, un, f, lds); break;
-      default: batch_row_unit<2048>(I, un, f, lds); break;
+    switch (I.nx + (I.small ? 1 : 0)) {
+      case 128: batch_row_unit<128, false, GEN>(I, un, f, lds); break;
+      case 129: batch_row_unit<128, true, GEN>(I, un, f, lds); break;
+      case 256: batch_row_unit<256, false, GEN>(I, un, f, lds); break;
+      case 257: batch_row_unit<256, true, GEN>(I, un, f, lds); break;
+      case 512:
+      case 513: batch_row_unit<512, false, GEN>(I, un, f, lds); break;
+      case 1024:
+      case 1025: batch_row_unit<1024, false, GEN>(I, un, f, lds); break;
+      default: batch_row_unit<2048, false, GEN>(I, un, f, lds); break;
     }
+    __syncthreads();  // the lengths lay the LDS out differently
   }
 }
 
 __global__ __launch_bounds__(BCOL_THREADS) void k_batch_col_all(const BatchInst* __restrict__ inst,
                                                                 const BatchUnit* __restrict__ units, int64_t nunits,
                                                                 BatchFlags f) {
-  __shared__ double2 lds2[(BCOL_LDS_ALL + 1) / 2];
-  float2* lds = reinterpret_cast<float2*>(lds2);
-  const int64_t grid = gridDim.x;
-  const int64_t bb = (grid % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (grid / 8) + blockIdx.x / 8 : blockIdx.x;
-  for (int64_t u = bb; u < nunits; u += grid) {
+  __shared__ double2 lds[lds_all<BCol>() / 16 + 1];
+  for (int64_t u = xcd_block(); u < nunits; u += gridDim.x) {
     const BatchUnit un = units[u];
     const BatchInst& I = inst[un.inst];
-    switch (I.ny) {
-      case 128: batch_col_unit<128>(I, un, f, lds); break;
-      case 256: batch_col_unit<256>(I, un, f, lds); break;
-      case 512: batch_col_unit<512>(I, un, f, lds); break;
-      case 1024: batch_col_unit<1024>(I, un, f, lds); break;
-      default: batch_col_unit<2048>(I, un, f, lds); break;
+    switch (I.ny + (I.small ? 1 : 0)) {
+      case 128: batch_col_unit<128, false>(I, un, f, lds); break;
+      case 129: batch_col_unit<128, true>(I, un, f, lds); break;
+      case 256: batch_col_unit<256, false>(I, un, f, lds); break;
+      case 257: batch_col_unit<256, true>(I, un, f, lds); break;
+      case 512: batch_col_unit<512, false>(I, un, f, lds); break;
+      case 513: batch_col_unit<512, true>(I, un, f, lds); break;
+      case 1024:
+      case 1025: batch_col_unit<1024, false>(I, un, f, lds); break;
+      default: batch_col_unit<2048, false>(I, un, f, lds); break;
     }
     __syncthreads();
   }
@@ -216,6 +225,7 @@ struct nlse_batch {
   BatchUnit* d_row = nullptr;
   BatchUnit* d_col = nullptr;
   int64_t n_row = 0, n_col = 0;
+  bool general = false;  // some member's loss varies from point to point
   int64_t row_off[NLEN + 1] = {0}, col_off[NLEN + 1] = {0};
   int row_grid[NLEN] = {0}, col_grid[NLEN] = {0};
   // one launch per sweep for every line length (k_batch_*_all) instead of
@@ -259,15 +269,20 @@ static BatchFlags row_flags(int precision, int stage) {
   return f;
 }
 
-template <int N>
+template <int N, bool SMALL>
 static void launch_row_n(nlse_batch* b, int li, const BatchFlags& f, hipStream_t s) {
-  hipLaunchKernelGGL(k_batch_row<N>, dim3((unsigned)b->row_grid[li]), dim3(BROW_THREADS), 0, s, b->d_inst,
-                     b->d_row + b->row_off[li], b->row_off[li + 1] - b->row_off[li], f);
+  const dim3 grid((unsigned)b->row_grid[li]), block(BROW_THREADS);
+  const BatchUnit* units = b->d_row + b->row_off[li];
+  const int64_t n = b->row_off[li + 1] - b->row_off[li];
+  if (b->general)
+    hipLaunchKernelGGL((k_batch_row<N, SMALL, true>), grid, block, 0, s, b->d_inst, units, n, f);
+  else
+    hipLaunchKernelGGL((k_batch_row<N, SMALL, false>), grid, block, 0, s, b->d_inst, units, n, f);
 }
 
-template <int N>
+template <int N, bool SMALL>
 static void launch_col_n(nlse_batch* b, int li, const BatchFlags& f, hipStream_t s) {
-  hipLaunchKernelGGL(k_batch_col<N>, dim3((unsigned)b->col_grid[li]), dim3(BCOL_THREADS), 0, s, b->d_inst,
+  hipLaunchKernelGGL((k_batch_col<N, SMALL>), dim3((unsigned)b->col_grid[li]), dim3(BCOL_THREADS), 0, s, b->d_inst,
                      b->d_col + b->col_off[li], b->col_off[li + 1] - b->col_off[li], f);
 }
 
@@ -275,18 +290,23 @@ static void launch_col_n(nlse_batch* b, int li, const BatchFlags& f, hipStream_t
 // all lengths (b->single).
 static int batch_row(nlse_batch* b, const BatchFlags& f, hipStream_t s) {
   if (b->single) {
-    hipLaunchKernelGGL(k_batch_row_all, dim3((unsigned)b->row_grid_all), dim3(BROW_THREADS), 0, s, b->d_inst, b->d_row,
-                       b->n_row, f);
+    hipLaunchKernelGGL(b->general ? k_batch_row_all<true> : k_batch_row_all<false>, dim3((unsigned)b->row_grid_all),
+                       dim3(BROW_THREADS), 0, s, b->d_inst, b->d_row, b->n_row, f);
     return launch_status("k_batch_row_all");
   }
-  for (int li = 0; li < NLEN; ++li) {
+  // longest lines first
+  for (int li = NLEN - 1; li >= 0; --li) {
     if (b->row_off[li + 1] == b->row_off[li]) continue;
     switch (li) {
-      case 0: launch_row_n<128>(b, li, f, s); break;
-      case 1: launch_row_n<256>(b, li, f, s); break;
-      case 2: launch_row_n<512>(b, li, f, s); break;
-      case 3: launch_row_n<1024>(b, li, f, s); break;
-      default: launch_row_n<2048>(b, li, f, s); break;
+      case 0: launch_row_n<128, false>(b, li, f, s); break;
+      case 1: launch_row_n<128, true>(b, li, f, s); break;
+      case 2: launch_row_n<256, false>(b, li, f, s); break;
+      case 3: launch_row_n<256, true>(b, li, f, s); break;
+      case 4:
+      case 5: launch_row_n<512, false>(b, li, f, s); break;
+      case 6:
+      case 7: launch_row_n<1024, false>(b, li, f, s); break;
+      default: launch_row_n<2048, false>(b, li, f, s); break;
     }
     int rc = launch_status("k_batch_row");
     if (rc) return rc;
@@ -303,14 +323,18 @@ static int batch_col(nlse_batch* b, hipStream_t s, int timing = 0) {
                        b->n_col, f);
     return launch_status("k_batch_col_all");
   }
-  for (int li = 0; li < NLEN; ++li) {
+  for (int li = NLEN - 1; li >= 0; --li) {
     if (b->col_off[li + 1] == b->col_off[li]) continue;
     switch (li) {
-      case 0: launch_col_n<128>(b, li, f, s); break;
-      case 1: launch_col_n<256>(b, li, f, s); break;
-      case 2: launch_col_n<512>(b, li, f, s); break;
-      case 3: launch_col_n<1024>(b, li, f, s); break;
-      default: launch_col_n<2048>(b, li, f, s); break;
+      case 0: launch_col_n<128, false>(b, li, f, s); break;
+      case 1: launch_col_n<128, true>(b, li, f, s); break;
+      case 2: launch_col_n<256, false>(b, li, f, s); break;
+      case 3: launch_col_n<256, true>(b, li, f, s); break;
+      case 4: launch_col_n<512, false>(b, li, f, s); break;
+      case 5: launch_col_n<512, true>(b, li, f, s); break;
+      case 6:
+      case 7: launch_col_n<1024, false>(b, li, f, s); break;
+      default: launch_col_n<2048, false>(b, li, f, s); break;
     }
     int rc = launch_status("k_batch_col");
     if (rc) return rc;
@@ -355,6 +379,7 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
   b->count = count;
   int rc = NLSE_OK;
   int dev = 0, ncu = 256;
+  int64_t total = 0;
   if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   std::vector<BatchUnit> rows_n[NLEN], cols_n[NLEN];
   for (int64_t i = 0; i < count && !rc; ++i) {
@@ -363,6 +388,8 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
     std::memset(&I, 0, sizeof I);
     I.nx = (int)it.nx;
     I.ny = (int)it.ny;
+    I.small = it.nx * it.ny <= SMALL_FIELD;
+    total += it.nx * it.ny;
     I.inv_nx = (float)(1.0 / (double)it.nx);
     I.inv_ny = (float)(1.0 / (double)it.ny);
     const double2 *twx = nullptr, *twy = nullptr;
@@ -382,7 +409,9 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
       h[sl].gdz_i = (float)it.nl[sl].gdz_i;
       h[sl].vdz_i = (float)it.nl[sl].vdz_i;
       h[sl].cplx = it.nl[sl].adz_i != 0.0 || it.nl[sl].gdz_i != 0.0 || it.nl[sl].vdz_i != 0.0;
+      b->general = b->general || h[sl].cplx;
     }
+    b->general = b->general || loss_saturates || it.v_kind == V_CPLX;
     if ((rc = batch_alloc(b, &nl, h, sizeof h))) break;
     for (int sl = 0; sl < 3; ++sl) I.nl[sl] = (const NLParams1*)nl + sl;
     RowArgs& r = I.row;
@@ -407,21 +436,19 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
     b->h_inst.push_back(I);
     b->offsets.push_back(it.offset);
     const int64_t lpb = 4096 / it.nx, w = 8192 / it.ny;
-    for (int64_t y = 0; y < it.ny; y += lpb) rows_n[len_index(it.nx)].push_back(BatchUnit{(int)i, 0, y});
-    for (int64_t t = 0; t < it.nx / w; ++t) cols_n[len_index(it.ny)].push_back(BatchUnit{(int)i, 0, t});
+    for (int64_t y = 0; y < it.ny; y += lpb) rows_n[len_index(it.nx, I.small)].push_back(BatchUnit{(int)i, 0, y});
+    for (int64_t t = 0; t < it.nx / w; ++t) cols_n[len_index(it.ny, I.small)].push_back(BatchUnit{(int)i, 0, t});
   }
+  for (BatchInst& I : b->h_inst) I.row.through = I.col.through = total * 8 <= WRITE_THROUGH;
   std::vector<BatchUnit> rows, cols;
   for (int li = 0; li < NLEN; ++li) {
     b->row_off[li] = (int64_t)rows.size();
     b->col_off[li] = (int64_t)cols.size();
     rows.insert(rows.end(), rows_n[li].begin(), rows_n[li].end());
     cols.insert(cols.end(), cols_n[li].begin(), cols_n[li].end());
-    // persistent grids: row blocks 8 per CU (64-field workload: 211 -> 186
-    // us per row sweep against 4), column blocks one per CU (the 8-wave
-    // blocks' registers allow one resident block; a second per CU only
-    // queues behind it: 253 -> 225 us)
+    // persistent grids: 8 row blocks and 2 column blocks per CU
     b->row_grid[li] = (int)std::min<int64_t>((int64_t)rows_n[li].size(), (int64_t)ncu * 8);
-    b->col_grid[li] = (int)std::min<int64_t>((int64_t)cols_n[li].size(), (int64_t)ncu * 1);
+    b->col_grid[li] = (int)std::min<int64_t>((int64_t)cols_n[li].size(), (int64_t)ncu * 2);
   }
   b->row_off[NLEN] = (int64_t)rows.size();
   b->col_off[NLEN] = (int64_t)cols.size();

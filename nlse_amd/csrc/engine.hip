@@ -164,7 +164,7 @@ int nlse_fft_plan_create(int ndim, const int64_t* dims, int64_t batch, nlse_fft_
   for (int d = 0; d + 1 < ndim; ++d) {
     int64_t cols = 1;
     for (int e = d + 1; e < ndim; ++e) cols *= dims[e];
-    p.colw[d] = p.ops[d]->colw(cols, 0);
+    p.colw[d] = p.ops[d]->colw(cols, 0, false);
   }
   *out = new nlse_fft_plan(p);
   return NLSE_OK;
@@ -188,7 +188,7 @@ int nlse_fft_exec(nlse_fft_plan* p, void* a_dev, int inverse, void* stream) {
     a.inverse_first = inverse ? 1 : 0;
     a.forward_last = inverse ? 0 : 1;
     a.out_scale = (last == 0) ? scale : 1.f;
-    int rc = p->ops[last]->row(1, a, s);
+    int rc = p->ops[last]->row(p->ops[last]->p_row, 1, a, s);
     if (rc) return rc;
   }
   for (int d = last - 1; d >= 0; --d) {
@@ -203,7 +203,7 @@ int nlse_fft_exec(nlse_fft_plan* p, void* a_dev, int inverse, void* stream) {
     a.do_fwd = inverse ? 0 : 1;
     a.do_inv = inverse ? 1 : 0;
     a.out_scale = (d == 0) ? scale : 1.f;
-    int rc = p->ops[d]->col(p->colw[d], a, s);
+    int rc = p->ops[d]->col(p->colw[d], false, a, s);
     if (rc) return rc;
   }
   return NLSE_OK;
@@ -323,7 +323,7 @@ __global__ void k_mul_prop(float2* A, const void* P, int kind, int64_t items, in
     if (kind == 1)
       A[i] = prop_c64(A[i], reinterpret_cast<const float2*>(P)[pi], 1.f);
     else
-      A[i] = prop_c128(A[i], reinterpret_cast<const double2*>(P)[pi], 1.0);
+      A[i] = to_f32(prop_c128(to_f64(A[i]), reinterpret_cast<const double2*>(P)[pi], 1.0));
   }
 }
 
@@ -753,7 +753,11 @@ struct nlse_plan {
   const double2* twx = nullptr;
   const double2* twy = nullptr;
   const double2* twt = nullptr;
-  bool row_alt = false;           // row kernels with the alternative set size (radix plan)
+  int row_points = 0;             // row kernels' set size (radix plan) if given, else chosen (row_p)
+  bool small = false;             // small-field plans (SMALL_FIELD)
+  bool through = false;           // sweeps write through (WRITE_THROUGH)
+  bool cplx = false;              // any nonlinear record of a complex dz
+  bool cplx_slot[3] = {false, false, false};
   int colw = 1;                   // y-column tile
   int colw_x = 1;                 // x-column tile (3-D)
   double2* prop128 = nullptr;     // 1-D complex128 propagator [ncomp][nx]
@@ -908,34 +912,43 @@ int nlse_plan_create(const nlse_plan_desc* d, nlse_plan** out) {
     delete p;
     return rc;
   }
-  if (d->row_points != 0 && d->row_points != p->rops->p_row) {
-    if (d->row_points != p->rops->p_row_alt || d->ndim == 1) {
-      const int pr = p->rops->p_row, pa = p->rops->p_row_alt;
+  const int64_t points = d->items * d->ncomp * (d->ndim >= 2 ? d->ny : 1) * d->nx * (d->ndim == 3 ? d->nt : 1);
+  p->small = d->ndim == 2 && points <= SMALL_FIELD;
+  p->through = points * 8 <= WRITE_THROUGH;
+  if (d->row_points != 0) {
+    const int pr = p->rops->p_row, pa = p->rops->p_row_alt, ps = p->rops->p_row_small;
+    const bool ok = d->row_points == pr || (d->ndim != 1 && (d->row_points == pa || (p->small && d->row_points == ps)));
+    if (!ok) {
       delete p;
       return fail(NLSE_ERR_ARG, "row_points %d unsupported for rows of %lld (0, %d or %d)", d->row_points,
                   (long long)d->nx, pr, pa);
     }
-    p->row_alt = true;
+    p->row_points = d->row_points;
   }
   if (d->ndim == 2) {
-    // default tile: the widest of 8, 4, 2, 1 columns that still gives every
-    // CU a block (a single 1024^2 field at 8 columns fills half the CUs;
-    // measured column sweeps at W = 8 / 4 / 2: 1024^2 12.7 / 11.3 / 14.7 us,
-    // 512^2 8.2 / 7.2 / 6.9 us; 2048^2 keeps 8)
+    // default tile: the widest of 8, 4, 2, 1 columns that gives every CU a
+    // block, or every second CU one of at most 256 threads (wider tiles read
+    // longer row segments, see LineCfg::WDEF).  Local step at W = 8 / 4 / 2:
+    // 1024^2 24.9 / 21.3 / - us, 512^2 - / 10.6 / 11.4 us, 256^2 10.6 / 8.3 /
+    // 7.8 us
     int want = d->col_width;
     if (want == 0) {
       int dev = 0, cus = 256;
       if (hipGetDevice(&dev) != hipSuccess ||
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
         cus = 256;
+      const int64_t t = d->ny / (p->small ? p->cops->p_col_small : p->cops->p_col);
       want = 8;
-      while (want > 1 && d->items * d->ncomp * (d->nx / want) < cus) want >>= 1;
+      for (; want > 1; want >>= 1) {
+        const int64_t blocks = d->items * d->ncomp * (d->nx / want);
+        if (blocks >= cus || (2 * blocks >= cus && want * t <= 256)) break;
+      }
     }
-    p->colw = p->cops->colw(d->nx, want);
+    p->colw = p->cops->colw(d->nx, want, p->small);
   }
   if (d->ndim == 3) {
-    p->colw = p->cops->colw(d->nx * d->nt, d->col_width);
-    p->colw_x = p->rops->colw(d->nt, d->col_width);
+    p->colw = p->cops->colw(d->nx * d->nt, d->col_width, false);
+    p->colw_x = p->rops->colw(d->nt, d->col_width, false);
   }
   *out = p;
   return NLSE_OK;
@@ -956,15 +969,23 @@ int nlse_plan_destroy(nlse_plan* p) {
   return NLSE_OK;
 }
 
+// Points per thread of the x-row sweep.  With a nonlocal response only a
+// run's first sweep is one: it keeps the default plan.
+static int row_p(const nlse_plan* p) {
+  if (p->wide) return 8;
+  if (p->row_points) return p->row_points;
+  return p->small && !p->nlc.on ? p->rops->p_row_small : p->rops->p_row;
+}
+
 int nlse_plan_config(const nlse_plan* p, int* row_points, int* col_width) {
   // 3-D plans report their y-column tile
   if (!p) return fail(NLSE_ERR_ARG, "null plan");
   if (p->wide) {
-    if (row_points) *row_points = 8;
+    if (row_points) *row_points = row_p(p);
     if (col_width) *col_width = 0;
     return NLSE_OK;
   }
-  if (row_points) *row_points = p->row_alt ? p->rops->p_row_alt : p->rops->p_row;
+  if (row_points) *row_points = row_p(p);
   if (col_width) *col_width = p->colw;
   return NLSE_OK;
 }
@@ -1074,6 +1095,7 @@ int nlse_plan_set_nl1(nlse_plan* p, int slot, const nlse_nl1* prm) {
     return wide_upload_nl(p, slot);
   }
   std::vector<NLParams1> h(p->d.items);
+  bool cx = false;
   for (int64_t i = 0; i < p->d.items; ++i) {
     h[i].adz = (float)prm[i].adz;
     h[i].gdz = (float)prm[i].gdz;
@@ -1083,7 +1105,10 @@ int nlse_plan_set_nl1(nlse_plan* p, int slot, const nlse_nl1* prm) {
     h[i].gdz_i = (float)prm[i].gdz_i;
     h[i].vdz_i = (float)prm[i].vdz_i;
     h[i].cplx = prm[i].adz_i != 0.0 || prm[i].gdz_i != 0.0 || prm[i].vdz_i != 0.0;
+    cx = cx || h[i].cplx;
   }
+  p->cplx_slot[slot] = cx;
+  p->cplx = p->cplx_slot[0] || p->cplx_slot[1] || p->cplx_slot[2];
   return upload(p, &p->nl[slot], h.data(), h.size() * sizeof(NLParams1));
 }
 
@@ -1268,7 +1293,7 @@ static int nlc_setup_2d(nlse_plan* p, const double* kernel, int kw) {
     n.zops = line_ops(n.M);
     if (!n.zops) return fail(NLSE_ERR_ARG, "unsupported intensity column length %lld", (long long)n.M);
     if ((rc = n.zops->twiddles(&n.twz))) return rc;
-    n.colw = n.zops->colw(nx, p->d.col_width);
+    n.colw = n.zops->colw(nx, p->d.col_width, false);
     // spectrum of the kernel wrapped on the M x nx torus, centre at (0, 0):
     // real and even, K^(ky, kx) = sum_{u,v} K[u][v] cos(2pi ky (u-r)/M) cos(2pi kx (v-r)/nx)
     const int64_t hy = n.M / 2 + 1, hx = nx / 2 + 1;
@@ -1358,7 +1383,7 @@ int nlse_plan_set_nonlocal_spectrum(nlse_plan* p, const double* quad, int64_t qy
     nlc_free(p);
     return rc;
   }
-  n.colw = n.zops->colw(nx, p->d.col_width);
+  n.colw = n.zops->colw(nx, p->d.col_width, false);
   n.on = true;
   return NLSE_OK;
 }
@@ -1433,6 +1458,9 @@ static int check_ready(const nlse_plan* p, int precision) {
   return NLSE_OK;
 }
 
+// The loss of a nonlinear application varies from point to point.
+static int nl_general(const nlse_plan* p) { return p->d.loss_saturates || p->vkind == V_CPLX || p->cplx; }
+
 static RowArgs plan_row_args(const nlse_plan* p, void* A) {
   RowArgs r = row_defaults();
   r.A = (float2*)A;
@@ -1447,6 +1475,8 @@ static RowArgs plan_row_args(const nlse_plan* p, void* A) {
   r.drv_r0 = p->fr0;
   r.drv_r1 = p->fr1;
   r.drv_dz = p->drv_dz;
+  r.general = nl_general(p);
+  r.through = p->through;
   return r;
 }
 
@@ -1463,6 +1493,7 @@ static ColArgs plan_col_args(const nlse_plan* p, void* A) {
   c.py = p->py;
   c.ptab = p->ptab;
   c.scale = (float)(1.0 / ((double)p->d.nx * (double)p->d.ny));
+  c.through = p->through;
   return c;
 }
 
@@ -1508,6 +1539,7 @@ static NlcArgs plan_nlc_args(const nlse_plan* p, void* A) {
   a.r = n.r;
   a.direct = n.direct ? 1 : 0;
   a.full = n.full ? 1 : 0;
+  a.general = nl_general(p);
   return a;
 }
 
@@ -1586,7 +1618,7 @@ static int band_and_z(nlse_plan* p, const void* A, hipStream_t s, const ColArgs*
     if (rc <= 0) return rc;  // launched, or an error
   }
   if ((rc = band_launch(p, A, s))) return rc;
-  if (!n.direct) rc = n.zops->col(n.colw, cz, s);
+  if (!n.direct) rc = n.zops->col(n.colw, false, cz, s);
   return rc;
 }
 
@@ -1628,6 +1660,7 @@ static int run1d(nlse_plan* p, void* A, int64_t nsteps, int precision, hipStream
   a.vkind = p->vkind;
   a.nlk = p->nlc.on ? p->nlc.K : nullptr;
   a.nlr = p->nlc.r;
+  a.general = nl_general(p);
   return p->rops->line1d(p->d.ncomp, a, s);
 }
 
@@ -1659,6 +1692,8 @@ static RowArgs row3d_args(const nlse_plan* p, void* A) {
   r.V = p->V;
   r.vkind = p->vkind;
   r.v_item_stride = p->v_item_stride;
+  r.general = nl_general(p);
+  r.through = p->through;
   return r;
 }
 
@@ -1668,6 +1703,7 @@ static ColArgs colx3d_args(const nlse_plan* p, void* A) {
   cx.nslabs = p->d.items * p->d.ny;
   cx.NX = (int)p->d.nt;
   cx.tw = p->twx;
+  cx.through = p->through;
   return cx;
 }
 
@@ -1685,6 +1721,7 @@ static ColArgs coly3d_args(const nlse_plan* p, void* A) {
   cy.pt = p->pt;
   cy.nt = (int)p->d.nt;
   cy.scale = (float)(1.0 / ((double)p->d.nx * (double)p->d.ny * (double)p->d.nt));
+  cy.through = p->through;
   return cy;
 }
 
@@ -1891,7 +1928,7 @@ static int wrun1d(nlse_plan* p, void* A, int64_t nsteps, int precision, hipStrea
 
 // x-row sweep with the plan's row kernel (default or alternative radix plan)
 static int launch_rows(const nlse_plan* p, int G, const RowArgs& a, hipStream_t s) {
-  return (p->row_alt ? p->rops->row_alt : p->rops->row)(G, a, s);
+  return p->rops->row(row_p(p), G, a, s);
 }
 
 static int chain_first(nlse_plan* p, void* A, int precision, hipStream_t s) {
@@ -1902,10 +1939,10 @@ static int chain_first(nlse_plan* p, void* A, int precision, hipStream_t s) {
     a.forward_last = 1;
     a.has_b = precision == 1;
     a.nlp_b = p->nl[NLSE_SLOT_HALF_PRE];
-    if ((rc = p->tops->row(1, a, s))) return rc;
+    if ((rc = p->tops->row(p->tops->p_row, 1, a, s))) return rc;
     ColArgs c = colx3d_args(p, A);
     c.do_fwd = 1;
-    return p->rops->col(p->colw_x, c, s);
+    return p->rops->col(p->colw_x, false, c, s);
   }
   if (p->nlc.on && precision == 1) return nlc_apply(p, A, 0, 1, p->nl[NLSE_SLOT_HALF_PRE], false, -1, s);
   RowArgs a = plan_row_args(p, A);
@@ -1920,18 +1957,18 @@ static int chain_step(nlse_plan* p, void* A, int precision, bool last, int64_t a
   if (p->wide) return wchain_step(p, A, precision, last, abs_k, s);
   int rc;
   if (p->d.ndim == 3) {
-    if ((rc = p->cops->col(p->colw, coly3d_args(p, A), s))) return rc;
+    if ((rc = p->cops->col(p->colw, false, coly3d_args(p, A), s))) return rc;
     ColArgs ci = colx3d_args(p, A);
     ci.do_inv = 1;
-    if ((rc = p->rops->col(p->colw_x, ci, s))) return rc;
+    if ((rc = p->rops->col(p->colw_x, false, ci, s))) return rc;
     RowArgs a = mid_row(p, row3d_args(p, A), precision, last);
-    if ((rc = p->tops->row(1, a, s))) return rc;
+    if ((rc = p->tops->row(p->tops->p_row, 1, a, s))) return rc;
     if (last) return NLSE_OK;
     ColArgs cf = colx3d_args(p, A);
     cf.do_fwd = 1;
-    return p->rops->col(p->colw_x, cf, s);
+    return p->rops->col(p->colw_x, false, cf, s);
   }
-  if ((rc = p->cops->col(p->colw, plan_col_args(p, A), s))) return rc;
+  if ((rc = p->cops->col(p->colw, p->small, plan_col_args(p, A), s))) return rc;
   if (p->nlc.on) {
     const int64_t ds = p->drive ? abs_k : -1;
     if (precision == 0) {
@@ -1991,7 +2028,7 @@ int nlse_run(nlse_plan* p, void* A, int64_t nsteps, int precision, int64_t step0
 // graph replays, so setters that rewrite a table in place keep the graph.
 static std::vector<uint64_t> graph_key(const nlse_plan* p, const void* A, int precision, int64_t chunk) {
   std::vector<uint64_t> k = {(uint64_t)(uintptr_t)A, (uint64_t)precision, (uint64_t)chunk, (uint64_t)p->pkind,
-                             (uint64_t)p->row_alt,
+                             (uint64_t)row_p(p), (uint64_t)nl_general(p),
                              (uint64_t)(uintptr_t)p->px, (uint64_t)(uintptr_t)p->py,
                              (uint64_t)(uintptr_t)p->ptab, (uint64_t)(uintptr_t)p->ptab128,
                              (uint64_t)(uintptr_t)p->pt, (uint64_t)(uintptr_t)p->V, (uint64_t)p->vkind,
@@ -2081,7 +2118,7 @@ int nlse_run_pass(nlse_plan* p, void* A, int pass, int64_t count, int precision,
     for (int64_t k = 0; k < count && !rc; ++k) {
       if (pass == 2) rc = p->rops->nlc(1, a, s);
       else if (pass == 3) rc = band_launch(p, A, s);
-      else if (pass == 4) rc = p->nlc.unpack ? p->nlc.zops->colu(cz, s) : p->nlc.zops->col(p->nlc.colw, cz, s);
+      else if (pass == 4) rc = p->nlc.unpack ? p->nlc.zops->colu(cz, s) : p->nlc.zops->col(p->nlc.colw, false, cz, s);
       else if (pass == 6) rc = band_and_z(p, A, s, &cz);
       else rc = p->rops->nlc(2, a, s);
     }
@@ -2094,7 +2131,7 @@ int nlse_run_pass(nlse_plan* p, void* A, int pass, int64_t count, int precision,
   ColArgs c = plan_col_args(p, A);
   c.scale = (float)(1.0 / (double)p->d.ny);
   for (int64_t k = 0; k < count; ++k) {
-    rc = pass == 0 ? launch_rows(p, p->d.ncomp, r, s) : p->cops->col(p->colw, c, s);
+    rc = pass == 0 ? launch_rows(p, p->d.ncomp, r, s) : p->cops->col(p->colw, p->small, c, s);
     if (rc) return rc;
   }
   return NLSE_OK;

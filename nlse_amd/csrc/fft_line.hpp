@@ -299,24 +299,43 @@ __host__ __device__ constexpr int tw_union_size(int n) {
   return tw_size_np(n, 16) + tw_size_np(n, 8) + tw_size_np(n, 4);
 }
 
-// The natural sets of G lines at element offsets off[g] (zeros for an
-// inactive group): one branch for the whole set, so the loads issue back to
-// back.
-template <int G, int P, int T>
-__device__ __forceinline__ void load_lines(const float2* __restrict__ A, const int64_t* off, int t, bool active,
-                                           float2 (&v)[G][P]) {
-  if (active) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = A[off[g] + t + m * T];
-  } else {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = make_float2(0.f, 0.f);
+// Stores kept in the L2 until the kernel's end, or written through to memory
+// (sc1) while the kernel runs.
+enum : int { ST_BACK = 0, ST_THROUGH = 16 };
+
+// Memory seen from a uniform address: a buffer descriptor in scalar registers.
+// An access is one instruction at a per-lane 32-bit byte offset plus a uniform
+// one, without vector instructions for 64-bit addresses and without keeping
+// the addresses of a line's loads for its stores.
+struct Buf {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ explicit Buf(const void* p)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(uniform(p)), 0, -1, 0x00027000)) {}
+  static __device__ __forceinline__ const void* uniform(const void* p) {
+    const uint64_t q = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)q);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(q >> 32));
+    return reinterpret_cast<const void*>(((uint64_t)hi << 32) | lo);
   }
-}
+  template <typename T>
+  __device__ __forceinline__ T load(uint32_t lane, uint32_t uni) const {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8 || sizeof(T) == 16, "access width");
+    if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, lane, uni, 0));
+    else if constexpr (sizeof(T) == 8)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, lane, uni, 0));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, lane, uni, 0));
+  }
+  template <int ST = ST_BACK>
+  __device__ __forceinline__ void store(float2 x, uint32_t lane, uint32_t uni) const {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), r, lane, uni, ST);
+  }
+  template <int ST = ST_BACK>
+  __device__ __forceinline__ void store(float4 x, uint32_t lane, uint32_t uni) const {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, lane, uni, ST);
+  }
+};
 
 // Padding of the row kernels' LDS lines (one float2 every 2^NLSE_ROW_PADSH
 // entries); the column kernel passes its own.
@@ -333,7 +352,7 @@ struct LdsLine {
 };
 
 template <int PADSH>
-__device__ __forceinline__ int lds_pad(int i) { return i + (i >> PADSH); }
+__host__ __device__ __forceinline__ constexpr int lds_pad(int i) { return i + (i >> PADSH); }
 
 // Twiddle table of a line length: the FP64 records {c, s} of every stage
 // table (tw_union_size(n) entries), followed by the same records as
@@ -348,15 +367,167 @@ __host__ __device__ constexpr int tw_f32_offset(int n) { return tw_union_size(n)
 // phase through the convolved intensity, while a gain bias would not (it
 // multiplies the whole nonlinear phase of the run) -- compensation keeps
 // the gain unbiased at about half the FP64 cost.
-enum FftArith : int { F64 = 0, F32C = 1 };
+// F64X: FP64 as F64, and the exchanges carry FP64 too: one rounding per
+// transform and no conversions between stages, for twice the LDS traffic.
+enum FftArith : int { F64 = 0, F32C = 1, F64X = 2 };
 
-// One Stockham stage on G lines owned by the same thread.  Non-last stages
-// exchange through LDS in rounds of GR lines (the LDS region holds GR lines
-// per thread column: line g of round r lives at slot g - r*GR); the last
-// stage (Ns = N/R) writes its outputs back to the natural set in registers.
-template <int N, int P, int S, int G, int GR, int PADSH, int AR>
-__device__ __forceinline__ void fft_stage(float2 (&v)[G][P], int t, const double2* __restrict__ tw,
-                                          float2* lds, int lds_stride) {
+template <int AR>
+using xchg_t = typename std::conditional<AR == F64X, double2, float2>::type;
+
+// Who exchanges a line: the whole block (barriers), or one wave (the lines of
+// a wave use their own LDS; the LDS operations of a wave complete in order, so
+// a compiler fence is enough).
+enum : int { SYNC_BLOCK = 0, SYNC_WAVE = 1 };
+
+template <int SYNC>
+__device__ __forceinline__ void line_sync() {
+  if constexpr (SYNC == SYNC_BLOCK) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+__device__ __forceinline__ double2 to_f64(double2 a) { return a; }
+template <typename C>
+__device__ __forceinline__ C from_f64(double2 a) {
+  if constexpr (std::is_same<C, float2>::value) return to_f32(a);
+  else return a;
+}
+
+// The FP64 twiddles of a thread's stages: two powers of w = exp(-2 pi i jm /
+// (Ns R)) per twiddled stage, w and w^2 (radix 4) or w and w^4 (radix 8, 16);
+// the others are products of these (3 for radix 16's factored form, 5 for
+// radix 8, 1 for radix 4).  They are loaded once, beside the field, and serve
+// every transform of the kernel: 15 table loads per radix-16 stage kept the
+// vector L1 as busy as the VALU (11.6 us each of a 28 us 2048^2 column
+// sweep), and loads issued at each stage exposed their latency.
+template <int N, int P>
+struct Twid {
+  static constexpr int NT = Plan<N, P>::NSTAGES > 1 ? Plan<N, P>::NSTAGES - 1 : 1;
+  double2 w[NT][2];
+};
+
+// Forward radix-R butterfly in FP64: inputs ld(k) times w^k (TW; w1, wq: the
+// powers Twid holds), outputs st(k, x).  Radix 16 runs as 4 x 4, w^(4 n1 + n2)
+// applied as w^(4 n1) before the first layer and w^n2 after it, which keeps
+// the live set near the 16 FP64 points.
+template <int R, bool TW, class Load, class Store>
+__device__ __forceinline__ void dft_io(Load ld, double2 w1, double2 wq, Store st) {
+  if constexpr (R == 16) {
+    double2 y[16];
+    double2 w2, w3, w8, w12;
+    if constexpr (TW) {
+      w8 = cmul_tw(wq, wq);
+      w12 = cmul_tw(w8, wq);
+      w2 = cmul_tw(w1, w1);
+      w3 = cmul_tw(w2, w1);
+    }
+#pragma unroll
+    for (int n2 = 0; n2 < 4; ++n2) {
+      double2 a = ld(n2), b = ld(4 + n2), c = ld(8 + n2), d = ld(12 + n2);
+      if constexpr (TW) {
+        b = cmul_tw(b, wq);
+        c = cmul_tw(c, w8);
+        d = cmul_tw(d, w12);
+      }
+      dft4(a, b, c, d);
+      if constexpr (TW) {
+        if (n2 > 0) {
+          const double2 w = n2 == 1 ? w1 : n2 == 2 ? w2 : w3;
+          a = cmul_tw(a, w);
+          b = cmul_tw(b, w);
+          c = cmul_tw(c, w);
+          d = cmul_tw(d, w);
+        }
+      }
+      // W16^(n2 k1)
+      if (n2 == 1) { b = rot(b, K_C8, K_S8); c = mul_w8_1(c); d = rot(d, K_S8, K_C8); }
+      if (n2 == 2) { b = mul_w8_1(b); c = mul_mi(c); d = mul_w8_3(d); }
+      if (n2 == 3) { b = rot(b, K_S8, K_C8); c = mul_w8_3(c); d = rot(d, -K_C8, -K_S8); }
+      y[n2 * 4 + 0] = a; y[n2 * 4 + 1] = b; y[n2 * 4 + 2] = c; y[n2 * 4 + 3] = d;
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) {
+      dft4(y[k1], y[4 + k1], y[8 + k1], y[12 + k1]);
+      st(k1, y[k1]);
+      st(k1 + 4, y[4 + k1]);
+      st(k1 + 8, y[8 + k1]);
+      st(k1 + 12, y[12 + k1]);
+    }
+  } else {
+    double2 x[R], w[8];
+    if constexpr (TW) {
+      w[1] = w1;
+      if constexpr (R == 4) {
+        w[2] = wq;
+        w[3] = cmul_tw(w1, wq);
+      } else if constexpr (R == 8) {
+        w[4] = wq;
+        w[2] = cmul_tw(w1, w1);
+        w[3] = cmul_tw(w[2], w1);
+        w[5] = cmul_tw(wq, w1);
+        w[6] = cmul_tw(wq, w[2]);
+        w[7] = cmul_tw(wq, w[3]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      x[k] = ld(k);
+      if (TW && k > 0) x[k] = cmul_tw(x[k], w[k]);
+    }
+    dft<R>(x);
+#pragma unroll
+    for (int k = 0; k < R; ++k) st(k, x[k]);
+  }
+}
+
+// Byte offset of stage S in the twiddle table (FP64 and FP32 records have the
+// same size).
+template <int N, int P, int S, int AR>
+constexpr uint32_t stage_twiddles() {
+  return 16u * (uint32_t)((AR != F32C ? 0 : tw_f32_offset(N)) + tw_base(N, P) + Plan<N, P>::tw_offset(S));
+}
+
+// A value the compiler cannot see through: what is computed from it is
+// computed again (addresses, twiddle loads) instead of being kept in
+// registers from one stage or transform to the next.
+__device__ __forceinline__ uint32_t opaque(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+template <int N, int P, int S = 1>
+__device__ __forceinline__ void load_twiddles_from(Twid<N, P>& W, const Buf& tw, int t) {
+  using PL = Plan<N, P>;
+  if constexpr (S < PL::NSTAGES) {
+    constexpr int NS = PL::ns(S);
+    static_assert(PL::radix(S) == P, "only the first stage has another radix, and no twiddles");
+    constexpr uint32_t TW0 = stage_twiddles<N, P, S, F64>();
+    const uint32_t o = 16u * (uint32_t)(t & (NS - 1));
+    W.w[S - 1][0] = tw.load<double2>(o, TW0);
+    W.w[S - 1][1] = tw.load<double2>(o, TW0 + 16u * (uint32_t)(((P == 4 ? 2 : 4) - 1) * NS));
+    load_twiddles_from<N, P, S + 1>(W, tw, t);
+  }
+}
+
+template <int N, int P>
+__device__ __forceinline__ Twid<N, P> load_twiddles(const Buf& tw, int t) {
+  Twid<N, P> W;
+  if constexpr (Plan<N, P>::NSTAGES > 1 && P >= 4 && P < 16) load_twiddles_from<N, P>(W, tw, t);
+  return W;
+}
+
+// One Stockham stage on G lines owned by the same thread, natural sets v in,
+// w out (v and w may be the same registers).  Stages before the last exchange
+// through LDS in rounds of GR lines (the LDS region holds GR lines per thread
+// column: line g of round r lives at slot g - r*GR); the last stage (Ns = N/R)
+// lands on the natural set.
+template <int N, int P, int S, int G, int GR, int PADSH, int AR, int SYNC, typename CI, typename CO>
+__device__ __forceinline__ void fft_stage(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+                                          xchg_t<AR>* lds, int lds_stride) {
   using PL = Plan<N, P>;
   constexpr int R = PL::radix(S);
   constexpr int NS = PL::ns(S);
@@ -364,97 +535,110 @@ __device__ __forceinline__ void fft_stage(float2 (&v)[G][P], int t, const double
   constexpr bool LAST = (S == PL::NSTAGES - 1);
   constexpr int T = PL::T;
   static_assert(G % GR == 0, "lines per round must divide the lines per thread");
-  using TW = typename std::conditional<AR == F64, double2, float4>::type;
-  TW tws[NB][R > 1 ? R - 1 : 1];
-  if constexpr (NS > 1) {
-    const TW* twst = reinterpret_cast<const TW*>(AR == F64 ? (const void*)tw : (const void*)(tw + tw_f32_offset(N))) +
-                     tw_base(N, P) + PL::tw_offset(S);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int jm = (t + b * T) & (NS - 1);
-#pragma unroll
-      for (int k = 1; k < R; ++k) tws[b][k - 1] = twst[(k - 1) * NS + jm];
-    }
-  }
+  // T a multiple of the padding period: no carry in lds_pad(t + m T)
+  constexpr bool LDS_STEP = T % (1 << PADSH) == 0;
+  constexpr uint32_t TW0 = stage_twiddles<N, P, S, AR>();
 #pragma unroll
   for (int r = 0; r < G / GR; ++r) {
+    if constexpr (!LAST) line_sync<SYNC>();  // the exchange before this one has been read
+    const int ts = (int)opaque((uint32_t)t);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int j = t + b * T;
-      const int jm = j & (NS - 1);
+    for (int gg = 0; gg < GR; ++gg) {
+      const int g = r * GR + gg;
 #pragma unroll
-      for (int gg = 0; gg < GR; ++gg) {
-        const int g = r * GR + gg;
-        float2 y[R];
-        if constexpr (AR == F64) {
-          double2 x[R];
-#pragma unroll
-          for (int k = 0; k < R; ++k) x[k] = to_f64(v[g][b + k * NB]);
-          if constexpr (NS > 1) {
-#pragma unroll
-            for (int k = 1; k < R; ++k) x[k] = cmul_tw(x[k], tws[b][k - 1]);
+      for (int b = 0; b < NB; ++b) {
+        const int j = ts + b * T;
+        const int jm = j & (NS - 1);
+        // lds_pad(base + k NS) = lds_pad(base) + lds_pad(k NS): base mod
+        // 2^PADSH and k NS mod 2^PADSH add without a carry (NS >= 2^PADSH,
+        // or base mod NS R = jm < NS, or R divides 2^PADSH), so one address
+        // serves all outputs through instruction offsets
+        xchg_t<AR>* out = lds + gg * lds_stride + lds_pad<PADSH>((j / NS) * NS * R + jm);
+        if constexpr (AR != F32C) {
+          auto ld = [&](int k) { return to_f64(v[g][b + k * NB]); };
+          auto st = [&](int k, double2 x) {
+            if constexpr (LAST) w[g][b + k * NB] = from_f64<CO>(x);
+            else out[lds_pad<PADSH>(k * NS)] = from_f64<xchg_t<AR>>(x);
+          };
+          double2 w1{}, wq{};
+          if constexpr (NS > 1 && P == 16) {
+            const uint32_t o = 16u * opaque((uint32_t)jm);
+            w1 = tw.load<double2>(o, TW0);
+            wq = tw.load<double2>(o, TW0 + 16u * 3u * NS);
+          } else if constexpr (NS > 1) {
+            w1 = W.w[S - 1][0];
+            wq = W.w[S - 1][1];
           }
-          dft<R>(x);
-#pragma unroll
-          for (int k = 0; k < R; ++k) y[k] = to_f32(x[k]);
+          dft_io<R, (NS > 1)>(ld, w1, wq, st);
         } else {
+          float2 y[R];
 #pragma unroll
-          for (int k = 0; k < R; ++k) y[k] = v[g][b + k * NB];
-          if constexpr (NS > 1) {
-#pragma unroll
-            for (int k = 1; k < R; ++k) y[k] = cmul_tw(y[k], tws[b][k - 1]);
+          for (int k = 0; k < R; ++k) {
+            y[k] = v[g][b + k * NB];
+            if (NS > 1 && k > 0)
+              y[k] = cmul_tw(y[k], tw.load<float4>(16u * (uint32_t)jm, TW0 + 16u * (uint32_t)((k - 1) * NS)));
           }
           dft<R>(y);
-        }
-        if constexpr (LAST) {
 #pragma unroll
-          for (int k = 0; k < R; ++k) v[g][b + k * NB] = y[k];
-        } else {
-          const int base = (j / NS) * NS * R + jm;
-#pragma unroll
-          for (int k = 0; k < R; ++k) lds[gg * lds_stride + lds_pad<PADSH>(base + k * NS)] = y[k];
+          for (int k = 0; k < R; ++k) {
+            if constexpr (LAST) w[g][b + k * NB] = y[k];
+            else out[lds_pad<PADSH>(k * NS)] = y[k];
+          }
         }
       }
     }
     if constexpr (!LAST) {
-      __syncthreads();
+      line_sync<SYNC>();
 #pragma unroll
       for (int gg = 0; gg < GR; ++gg)
 #pragma unroll
-        for (int m = 0; m < P; ++m) v[r * GR + gg][m] = lds[gg * lds_stride + lds_pad<PADSH>(t + m * T)];
-      __syncthreads();
+        for (int m = 0; m < P; ++m)
+          w[r * GR + gg][m] = LDS_STEP ? lds[gg * lds_stride + lds_pad<PADSH>(ts) + lds_pad<PADSH>(m * T)]
+                                       : lds[gg * lds_stride + lds_pad<PADSH>(ts + m * T)];
     }
   }
 }
 
-template <int N, int P, int S, int G, int GR, int PADSH, int AR>
-__device__ __forceinline__ void fft_stages_from(float2 (&v)[G][P], int t, const double2* __restrict__ tw,
-                                                float2* lds, int lds_stride) {
-  if constexpr (S < Plan<N, P>::NSTAGES) {
-    fft_stage<N, P, S, G, GR, PADSH, AR>(v, t, tw, lds, lds_stride);
-    fft_stages_from<N, P, S + 1, G, GR, PADSH, AR>(v, t, tw, lds, lds_stride);
+template <int N, int P, int S, int G, int GR, int PADSH, int AR, int SYNC, typename CI, typename CO>
+__device__ __forceinline__ void fft_stages_from(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+                                                xchg_t<AR>* lds, int lds_stride) {
+  if constexpr (S == Plan<N, P>::NSTAGES - 1) {
+    fft_stage<N, P, S, G, GR, PADSH, AR, SYNC>(v, w, t, W, tw, lds, lds_stride);
+  } else {
+    xchg_t<AR> u[G][P];
+    fft_stage<N, P, S, G, GR, PADSH, AR, SYNC>(v, u, t, W, tw, lds, lds_stride);
+    fft_stages_from<N, P, S + 1, G, GR, PADSH, AR, SYNC>(u, w, t, W, tw, lds, lds_stride);
   }
 }
 
+template <int G, int P, typename C>
+__device__ __forceinline__ void swap_parts(C (&v)[G][P]) {
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      C z = v[g][m];
+      v[g][m].x = z.y;
+      v[g][m].y = z.x;
+    }
+}
+
 // Forward (INV=false) or unnormalised inverse (INV=true) DFT of G lines,
-// natural set in, natural set out.  The inverse is swap(F(swap(x))) with
-// swap(a + ib) = b + ia (= conj(F(conj x))), a register renaming.
-template <int N, int P, int G, bool INV, int GR = G, int PADSH = NLSE_ROW_PADSH, int AR = F64>
-__device__ __forceinline__ void fft_line(float2 (&v)[G][P], int t, const double2* __restrict__ tw,
-                                         float2* lds, int lds_stride) {
-  if constexpr (INV) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = make_float2(v[g][m].y, v[g][m].x);
-  }
-  fft_stages_from<N, P, 0, G, GR, PADSH, AR>(v, t, tw, lds, lds_stride);
-  if constexpr (INV) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = make_float2(v[g][m].y, v[g][m].x);
-  }
+// natural set v in, natural set w out.  The inverse is swap(F(swap(x))) with
+// swap(a + ib) = b + ia (= conj(F(conj x))), a register renaming.  An FP64
+// input or output set is taken or left without rounding.
+template <int N, int P, int G, bool INV, int GR, int PADSH, int AR, int SYNC, typename CI, typename CO>
+__device__ __forceinline__ void fft_line_io(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+                                            xchg_t<AR>* lds, int lds_stride) {
+  if constexpr (INV) swap_parts<G, P>(v);
+  fft_stages_from<N, P, 0, G, GR, PADSH, AR, SYNC>(v, w, t, W, tw, lds, lds_stride);
+  if constexpr (INV) swap_parts<G, P>(w);
+}
+
+template <int N, int P, int G, bool INV, int GR = G, int PADSH = NLSE_ROW_PADSH, int AR = F64, int SYNC = SYNC_BLOCK>
+__device__ __forceinline__ void fft_line(float2 (&v)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+                                         xchg_t<AR>* lds, int lds_stride) {
+  fft_line_io<N, P, G, INV, GR, PADSH, AR, SYNC>(v, v, t, W, tw, lds, lds_stride);
 }
 
 }  // namespace nlse

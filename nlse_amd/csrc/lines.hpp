@@ -14,37 +14,26 @@
 #include "common.hpp"
 #include "passes_2d.hpp"
 
-#ifndef NLSE_COL_PREFER_PAIRS
-#define NLSE_COL_PREFER_PAIRS 0
-#endif
-#ifndef NLSE_COL_THREADS
-#define NLSE_COL_THREADS 512  // threads of one column-sweep block at most
-#endif
-#ifndef NLSE_COL_LDS_KB
-#define NLSE_COL_LDS_KB 150  // LDS budget of one column-sweep block
-#endif
-
 namespace nlse {
 
-// Runtime-N dispatch table.
+// Runtime-N dispatch table.  p: points per thread (radix plan) of a sweep.
 struct LineOps {
   int (*twiddles)(const double2**);
-  int (*row)(int, const RowArgs&, hipStream_t);
-  // the row kernel with the other per-thread set size (radix plan), a
-  // choice of the autotuner: p_row_alt points per thread (= p_row when the
-  // length has no alternative)
-  int (*row_alt)(int, const RowArgs&, hipStream_t);
-  int p_row, p_row_alt;
+  // x rows (G = 1, or component pairs G = 2) with p points per thread: p_row
+  // by default, p_row_alt on request, p_row_small for small fields
+  int (*row)(int, int, const RowArgs&, hipStream_t);
+  int p_row, p_row_alt, p_row_small;
   int (*line1d)(int, const Line1DArgs&, hipStream_t);
   int (*nlc)(int, const NlcArgs&, hipStream_t);
-  int (*col)(int, const ColArgs&, hipStream_t);
-  int (*colw)(int64_t, int);
+  // columns: tile width, small-field plan or not
+  int (*col)(int, bool, const ColArgs&, hipStream_t);
+  int (*colw)(int64_t, int, bool);
+  int p_col, p_col_small;
   // intensity column sweep + band pass in one launch (1: not available for
   // this tile width, use the separate launches)
   int (*colz_band)(int, const ColArgs&, const BandArgs&, int, size_t, int64_t, hipStream_t);
   // full-torus intensity convolution of row-pair-packed spectra (k_colu)
   int (*colu)(const ColArgs&, hipStream_t);
-  int lpb1, lpb2, t;
 };
 
 // ------------------------------------------------------ twiddle tables
@@ -114,26 +103,12 @@ static int get_twiddles(const double2** out) {
 }
 
 // -------------------------------------------------- kernel dispatchers
-// Points per thread (P) of each kernel kind and line length: 16 by
-// default, 8 for lengths in [NLSE_P8_FROM_K, NLSE_P8_UPTO_K), 4 from
-// NLSE_P4_FROM_K.  A smaller P puts more waves on a line (latency hiding
-// for one-round sweeps), a larger P has fewer stages, i.e. fewer FP64
-// conversions and LDS exchanges.  Measured on MI355X with the FP64 stages:
-// k_row is faster at P = 16 for 2048 (35.6 -> 33.1 us) and at P = 8 for
-// 1024 and 512 (512^2 row sweep 9.9 -> 6.3 us: twice the waves on a field
-// that fills a quarter of the SIMDs at P = 16, the same three stages);
-// k_nlc_nl keeps P = 8 at 2048 (26.7 vs 29.6 us); k_nlc_z P = 8 at 512
-// and 1024 only (2048: 19.6 vs 20.4 us); at 512 both nonlocal row kernels
-// take P = 8 (512^2 nonlocal step 40.2 -> 30.2 us: k_nlc_z 8.7 -> 5.7,
-// k_nlc_nl 15.8 -> 9.6 us); the column kernel keeps P = 16 (the
-// uneven-batch column units are built on it).  The autotuner can switch
-// the x-row kernels to the other set size per plan.
-#ifndef NLSE_P8_FROM_COL
-#define NLSE_P8_FROM_COL (1 << 30)
-#endif
-#ifndef NLSE_P8_FROM_ROW
-#define NLSE_P8_FROM_ROW 512
-#endif
+// Points per thread (P) of each kernel kind and line length.  A smaller P puts
+// more lanes on a line (a shorter chain of instructions per lane, what a field
+// of few lines waits for), a larger P has fewer stages, i.e. fewer exchanges
+// and conversions.  Nonlocal row kernels (measured on MI355X): k_nlc_nl keeps
+// P = 8 at 2048 (26.7 vs 29.6 us); k_nlc_z P = 8 at 512 and 1024 only; at 512
+// both take P = 8.
 #ifndef NLSE_P8_FROM_NLZ
 #define NLSE_P8_FROM_NLZ 512
 #endif
@@ -143,109 +118,88 @@ static int get_twiddles(const double2** out) {
 #ifndef NLSE_P8_FROM_NLNL
 #define NLSE_P8_FROM_NLNL 512
 #endif
-#ifndef NLSE_P8_FROM_1D
-#define NLSE_P8_FROM_1D (1 << 30)
-#endif
-#ifndef NLSE_P8_UPTO_COL
-#define NLSE_P8_UPTO_COL (1 << 30)
-#endif
-#ifndef NLSE_P8_UPTO_ROW
-#define NLSE_P8_UPTO_ROW 2048
-#endif
 #ifndef NLSE_P8_UPTO_NLNL
 #define NLSE_P8_UPTO_NLNL (1 << 30)
 #endif
-#ifndef NLSE_P8_UPTO_1D
-#define NLSE_P8_UPTO_1D (1 << 30)
-#endif
-#ifndef NLSE_P4_FROM_COL
-#define NLSE_P4_FROM_COL (1 << 30)
-#endif
-#ifndef NLSE_P4_FROM_ROW
-#define NLSE_P4_FROM_ROW (1 << 30)
-#endif
-#ifndef NLSE_P4_FROM_NLZ
-#define NLSE_P4_FROM_NLZ (1 << 30)
-#endif
-#ifndef NLSE_P4_FROM_NLNL
-#define NLSE_P4_FROM_NLNL (1 << 30)
-#endif
-#ifndef NLSE_P4_FROM_1D
-#define NLSE_P4_FROM_1D (1 << 30)
-#endif
 
-constexpr int pick_p(int n, int p8_from, int p8_upto, int p4_from) {
-  return n >= p4_from && n >= 4 ? 4 : (n >= p8_from && n < p8_upto && n >= 8 ? 8 : (n >= 16 ? 16 : n));
+constexpr int pick_p(int n, int p8_from, int p8_upto) {
+  return n >= p8_from && n < p8_upto && n >= 8 ? 8 : (n >= 16 ? 16 : n);
 }
-#define NLSE_PICK_P(n, K) pick_p(n, NLSE_P8_FROM_##K, NLSE_P8_UPTO_##K, NLSE_P4_FROM_##K)
 constexpr int lines_per_block(int threads, int t) { return threads / t >= 1 ? threads / t : 1; }
+
+// Fields of at most this many points (all items and components) take the
+// small-field plans of LineCfg: their sweeps are a few waves per CU, bound by
+// the length of one lane's work.  One step (row + column sweep) of a local
+// field, default against small-field plan: 256^2 14.0 -> 7.8 us, 512^2 12.7 ->
+// 10.6 us; 18 fields of 256^2 (1.2 M points) 19.0 -> 20.2 us.
+constexpr int64_t SMALL_FIELD = 1 << 18;
+
+// Fields of at most this many bytes are written through to memory: a kernel's
+// end then has no dirty L2 lines left to write back before the next sweep,
+// whose reads come from other XCDs, may start.  Step of a local field, stores
+// back / through: 1024^2 25.2 -> 21.0 us, 2 x 1024^2 46.2 -> 31.8 us, 2048^2
+// 59.7 -> 56.4 us; 28 x 1024^2 (235 MB) 280 -> 298 us.
+constexpr int64_t WRITE_THROUGH = 48 << 20;
 
 template <int N>
 struct LineCfg {
-  // column kernel
-  static constexpr int P = NLSE_PICK_P(N, COL);
+  // column sweeps
+  static constexpr int P = N >= 16 ? 16 : N;
   static constexpr int T = N / P;
   static constexpr int LINE = LdsLine<N, 3, 3>::SIZE;  // column-pass lines
-  // row kernel: 256 threads for one component, 128 for pairs
-  static constexpr int PR = NLSE_PICK_P(N, ROW);
-  static constexpr int LPB1 = lines_per_block(256, N / PR);
-  static constexpr int LPB2 = lines_per_block(128, N / PR);
+  // small fields: up to 256 points 4 per thread, FP64 exchanges (one rounding
+  // per transform, so the extra stages round nothing); 512 points 8
+  static constexpr int PS = N <= 256 ? 4 : (N == 512 ? 8 : P);
+  static constexpr int ARS = N <= 256 ? F64X : F64;
+  // x rows
+  static constexpr int PR = (N == 512 || N == 1024) ? 8 : P;
+  static constexpr int PRS = N <= 256 ? 4 : PR;
   // nonlocal row kernels (one line pair per N/P threads, 128 per block)
-  static constexpr int PZ = NLSE_PICK_P(N, NLZ);
+  static constexpr int PZ = pick_p(N, NLSE_P8_FROM_NLZ, NLSE_P8_UPTO_NLZ);
   static constexpr int LPBZ = lines_per_block(128, N / PZ);
-  static constexpr int PN = NLSE_PICK_P(N, NLNL);
+  static constexpr int PN = pick_p(N, NLSE_P8_FROM_NLNL, NLSE_P8_UPTO_NLNL);
   static constexpr int LPBN = lines_per_block(128, N / PN);
   // whole 1-D runs
-  static constexpr int P1 = NLSE_PICK_P(N, 1D);
+  static constexpr int P1 = N >= 16 ? 16 : N;
   static constexpr int LPB1D1 = lines_per_block(256, N / P1);
   static constexpr int LPB1D2 = lines_per_block(128, N / P1);
-  // default column tile: 8 columns (64-byte row segments; wider tiles
-  // spill registers at 512 threads); 2-D plans narrow it when a sweep
-  // would have fewer blocks than CUs (nlse_plan_create)
+  // default column tile: 8 columns (64-byte row segments; narrower tiles
+  // read 32-byte segments: 12.9 us against 8.5 us for an in-place copy of
+  // a 2048^2 field); 2-D plans narrow it for small fields (nlse_plan_create)
   static constexpr int WDEF = 8;
 };
 
-// Column tile of W columns: WT threads across (<= 512 threads per block,
-// i.e. up to 256 VGPRs per lane), G = W/WT columns per thread, LDS rounds
-// of GR columns per thread column (<= 150 KiB of LDS).
-template <int N, int W>
+// Column tile of W columns with PC points per thread: WT threads across, G =
+// W/WT columns per thread, LDS rounds of GR columns per thread column.  One
+// column per thread needs at most 128 VGPRs and takes blocks of up to 1024
+// threads; several columns per thread take 512.
+template <int N, int W, int PC, int AR>
 struct ColCfg {
-  using C = LineCfg<N>;
-  static constexpr int WTMAX = (NLSE_COL_THREADS / C::T) >= 1 ? (NLSE_COL_THREADS / C::T) : 1;
-  // with NLSE_COL_PREFER_PAIRS every thread owns two adjacent columns
-  // (16-byte accesses) whenever the tile has two or more; measured slower
-  // where the tile fits one column per thread (1024^2 column sweep 11.7 ->
-  // 13.3 us, 3-D 512x512x64 workload 3.76k -> 3.49k steps/s), so pairs are used only when
-  // the tile is wider than WTMAX threads
-  static constexpr int WTP = (NLSE_COL_PREFER_PAIRS && W >= 2) ? W / 2 : W;
-  static constexpr int WT = WTP < WTMAX ? WTP : WTMAX;
+  static constexpr int T = N / PC;
+  static constexpr int LINEB = LineCfg<N>::LINE * (int)sizeof(xchg_t<AR>);  // bytes of a line
+  static constexpr bool ONE = W * T <= 1024 && W * LINEB <= 150 * 1024;
+  static constexpr int WTMAX = lines_per_block(512, T);
+  static constexpr int WT = ONE || W < WTMAX ? W : WTMAX;
   static constexpr int G = W / WT;
-  static constexpr int GRMAX = (NLSE_COL_LDS_KB * 1024) / (WT * C::LINE * 8);
+  static constexpr int GRMAX = (150 * 1024) / (WT * LINEB);
   static constexpr int gr(int g) { return (g <= GRMAX || g == 1) ? g : gr(g / 2); }
   static constexpr int GR = gr(G);
-  static constexpr bool OK = G >= 1 && G <= 4 && GR >= 1 && WT * GR * C::LINE * 8 <= 160 * 1024;
+  static constexpr bool OK = G >= 1 && G <= 4 && GR >= 1 && WT * GR * LINEB <= 160 * 1024;
 };
 
-// Row kernels with PR points per thread (256 threads for one component,
-// 128 for pairs, as in LineCfg).
-template <int N, int PR>
+// Row kernels with PR points per thread, 128 threads where a line has fewer.
+template <int N, int PR, int AR>
 static int row_launch_p(int G, const RowArgs& a, hipStream_t s) {
   constexpr int T = N / PR;
-  if (G == 1) {
-    constexpr int L = lines_per_block(256, T);
-    const int64_t blocks = (a.ngroups + L - 1) / L;
-    hipLaunchKernelGGL((k_row<N, PR, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-  } else {
-    constexpr int L = lines_per_block(128, T);
-    const int64_t blocks = (a.ngroups + L - 1) / L;
-    hipLaunchKernelGGL((k_row<N, PR, L, 2>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-  }
+  constexpr int L = lines_per_block(128, T);
+  const int64_t blocks = (a.ngroups + L - 1) / L;
+  if (G == 2)
+    hipLaunchKernelGGL((k_row<N, PR, L, 2, true, AR>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+  else if (a.general)
+    hipLaunchKernelGGL((k_row<N, PR, L, 1, true, AR>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_row<N, PR, L, 1, false, AR>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
   return launch_status("k_row");
-}
-
-template <int N>
-static int row_launch(int G, const RowArgs& a, hipStream_t s) {
-  return row_launch_p<N, LineCfg<N>::PR>(G, a, s);
 }
 
 // The alternative set size: 16 where the default is 8 and 8 where it is 16
@@ -256,8 +210,16 @@ constexpr int row_p_alt() {
 }
 
 template <int N>
-static int row_launch_alt(int G, const RowArgs& a, hipStream_t s) {
-  return row_launch_p<N, row_p_alt<N>()>(G, a, s);
+static int row_launch(int p, int G, const RowArgs& a, hipStream_t s) {
+  using C = LineCfg<N>;
+  if (p == C::PR) return row_launch_p<N, C::PR, F64>(G, a, s);
+  if constexpr (row_p_alt<N>() != C::PR) {
+    if (p == row_p_alt<N>()) return row_launch_p<N, row_p_alt<N>(), F64>(G, a, s);
+  }
+  if constexpr (C::PRS != C::PR) {
+    if (p == C::PRS) return row_launch_p<N, C::PRS, C::ARS>(G, a, s);
+  }
+  return fail(NLSE_ERR_ARG, "no row kernel of %d points per thread for length %d", p, N);
 }
 
 template <int N>
@@ -267,11 +229,14 @@ static int line1d_launch(int G, const Line1DArgs& a, hipStream_t s) {
   if (G == 1) {
     constexpr int L = C::LPB1D1;
     const int64_t blocks = (a.ngroups + L - 1) / L;
-    hipLaunchKernelGGL((k_line1d<N, C::P1, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    if (a.general)
+      hipLaunchKernelGGL((k_line1d<N, C::P1, L, 1, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_line1d<N, C::P1, L, 1, false>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
   } else {
     constexpr int L = C::LPB1D2;
     const int64_t blocks = (a.ngroups + L - 1) / L;
-    hipLaunchKernelGGL((k_line1d<N, C::P1, L, 2>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    hipLaunchKernelGGL((k_line1d<N, C::P1, L, 2, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
   }
   return launch_status("k_line1d");
 }
@@ -293,80 +258,92 @@ static int nlc_launch(int stage, const NlcArgs& a, hipStream_t s) {
     constexpr int L = C::LPBN, T = N / C::PN;
     const int64_t blocks = (a.ngroups + L - 1) / L;
     if (full)
-      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-    else if (a.ncomp == 1)
-      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1, 1, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    else if (a.ncomp != 1)
+      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 2, 0, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    else if (a.general)
+      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1, 0, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
     else
-      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 2>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
   }
   return launch_status(stage == 1 ? "k_nlc_z" : "k_nlc_nl");
 }
 
+template <int N, int W, int PK, int PC, int AR>
+static void col_launch_k(const ColArgs& a, hipStream_t s) {
+  using K = ColCfg<N, W, PC, AR>;
+  const int64_t blocks = a.nslabs * (a.NX / W);
+  hipLaunchKernelGGL((k_col<N, PC, K::WT, K::G, K::GR, PK, AR>), dim3((unsigned)blocks), dim3(K::WT * K::T), 0, s, a);
+}
+
 template <int N, int W>
-static bool col_launch_w(const ColArgs& a, hipStream_t s) {
+static bool col_launch_w(bool small, const ColArgs& a, hipStream_t s) {
   using C = LineCfg<N>;
-  using K = ColCfg<N, W>;
-  if constexpr (K::OK) {
-    const int64_t blocks = a.nslabs * (a.NX / W);
+  if constexpr (ColCfg<N, W, C::PS, C::ARS>::OK && C::PS != C::P) {
+    // small fields: the separable propagator's sweep
+    if (small && a.do_prop && a.pkind == PROP_SEP64) {
+      col_launch_k<N, W, PROP_SEP64, C::PS, C::ARS>(a, s);
+      return true;
+    }
+  }
+  if constexpr (ColCfg<N, W, C::P, F64>::OK) {
     // the separable 2-D and 3-D propagators, the real kernel spectrum of
     // the nonlocal response and the propagator-free transforms get their
     // own instances (fewer live registers than the run-time dispatch over
-    // every kind)
+    // every kind); slabs of 4 GiB and more take the PK = -1 instance
     const bool prop = a.do_prop != 0;
-    if (prop && a.pkind == PROP_SEP64)
-      hipLaunchKernelGGL((k_col<N, C::P, K::WT, K::G, K::GR, PROP_SEP64>), dim3((unsigned)blocks),
-                         dim3(K::WT * C::T), 0, s, a);
-    else if (prop && a.pkind == PROP_KREAL)
-      hipLaunchKernelGGL((k_col<N, C::P, K::WT, K::G, K::GR, PROP_KREAL>), dim3((unsigned)blocks),
-                         dim3(K::WT * C::T), 0, s, a);
-    else if (prop && a.pkind == PROP_SEP3D)
-      hipLaunchKernelGGL((k_col<N, C::P, K::WT, K::G, K::GR, PROP_SEP3D>), dim3((unsigned)blocks),
-                         dim3(K::WT * C::T), 0, s, a);
+    const bool big = (int64_t)N * a.NX * 8 > (int64_t)0xffffffff;
+    if (big || (prop && a.pkind != PROP_SEP64 && a.pkind != PROP_KREAL && a.pkind != PROP_SEP3D))
+      col_launch_k<N, W, -1, C::P, F64>(a, s);
     else if (!prop)
-      hipLaunchKernelGGL((k_col<N, C::P, K::WT, K::G, K::GR, PK_NONE>), dim3((unsigned)blocks),
-                         dim3(K::WT * C::T), 0, s, a);
+      col_launch_k<N, W, PK_NONE, C::P, F64>(a, s);
+    else if (a.pkind == PROP_SEP64)
+      col_launch_k<N, W, PROP_SEP64, C::P, F64>(a, s);
+    else if (a.pkind == PROP_KREAL)
+      col_launch_k<N, W, PROP_KREAL, C::P, F64>(a, s);
     else
-      hipLaunchKernelGGL((k_col<N, C::P, K::WT, K::G, K::GR>), dim3((unsigned)blocks), dim3(K::WT * C::T), 0, s,
-                         a);
+      col_launch_k<N, W, PROP_SEP3D, C::P, F64>(a, s);
     return true;
-  } else {
-    return false;
   }
+  return false;
 }
 
 template <int N>
-static bool col_ok(int w) {
+static bool col_ok(int w, bool small) {
+  using C = LineCfg<N>;
+#define NLSE_COL_OK(W) (ColCfg<N, W, C::P, F64>::OK && (!small || ColCfg<N, W, C::PS, C::ARS>::OK))
   switch (w) {
-    case 1: return ColCfg<N, 1>::OK;
-    case 2: return ColCfg<N, 2>::OK;
-    case 4: return ColCfg<N, 4>::OK;
-    case 8: return ColCfg<N, 8>::OK;
-    case 16: return ColCfg<N, 16>::OK;
-    case 32: return ColCfg<N, 32>::OK;
-    case 64: return ColCfg<N, 64>::OK;
+    case 1: return NLSE_COL_OK(1);
+    case 2: return NLSE_COL_OK(2);
+    case 4: return NLSE_COL_OK(4);
+    case 8: return NLSE_COL_OK(8);
+    case 16: return NLSE_COL_OK(16);
+    case 32: return NLSE_COL_OK(32);
+    case 64: return NLSE_COL_OK(64);
     default: return false;
   }
+#undef NLSE_COL_OK
 }
 
 template <int N>
-static int col_width_for(int64_t ncols, int want) {
+static int col_width_for(int64_t ncols, int want, bool small) {
   int w = want > 0 ? want : LineCfg<N>::WDEF;
   if (w > 64) w = 64;
-  while (w > 1 && (w > ncols || (ncols % w) != 0 || !col_ok<N>(w))) w >>= 1;
+  while (w > 1 && (w > ncols || (ncols % w) != 0 || !col_ok<N>(w, small))) w >>= 1;
   return w;
 }
 
 template <int N>
-static int col_launch(int W, const ColArgs& a, hipStream_t s) {
+static int col_launch(int W, bool small, const ColArgs& a, hipStream_t s) {
   bool ok = false;
   switch (W) {
-    case 1: ok = col_launch_w<N, 1>(a, s); break;
-    case 2: ok = col_launch_w<N, 2>(a, s); break;
-    case 4: ok = col_launch_w<N, 4>(a, s); break;
-    case 8: ok = col_launch_w<N, 8>(a, s); break;
-    case 16: ok = col_launch_w<N, 16>(a, s); break;
-    case 32: ok = col_launch_w<N, 32>(a, s); break;
-    case 64: ok = col_launch_w<N, 64>(a, s); break;
+    case 1: ok = col_launch_w<N, 1>(small, a, s); break;
+    case 2: ok = col_launch_w<N, 2>(small, a, s); break;
+    case 4: ok = col_launch_w<N, 4>(small, a, s); break;
+    case 8: ok = col_launch_w<N, 8>(small, a, s); break;
+    case 16: ok = col_launch_w<N, 16>(small, a, s); break;
+    case 32: ok = col_launch_w<N, 32>(small, a, s); break;
+    case 64: ok = col_launch_w<N, 64>(small, a, s); break;
     default: break;
   }
   if (!ok) return fail(NLSE_ERR_ARG, "unsupported column width %d for length %d", W, N);
@@ -460,12 +437,10 @@ static int colu_launch(const ColArgs& a, hipStream_t s) {
 template <int N>
 LineOps make_ops() {
   using C = LineCfg<N>;
-  return LineOps{&get_twiddles<N>,    &row_launch<N>,       &row_launch_alt<N>, C::PR,
-                 row_p_alt<N>(),      &line1d_launch<N>,    &nlc_launch<N>,     &col_launch<N>,
-                 &col_width_for<N>,   &colz_band_launch<N>, &colu_launch<N>,    C::LPB1,
-                 C::LPB2,             N / C::PR};
+  return LineOps{&get_twiddles<N>,  &row_launch<N>, C::PR,          row_p_alt<N>(), C::PRS,
+                 &line1d_launch<N>, &nlc_launch<N>, &col_launch<N>, &col_width_for<N>,
+                 C::P,              C::PS,          &colz_band_launch<N>, &colu_launch<N>};
 }
-
 
 // Dispatch table entry of a line length (engine.hip), or null.
 const LineOps* line_ops_public(int64_t n);

@@ -53,6 +53,7 @@ struct NlcArgs {
   float2 drv_t1;
   float drv_dz;
   float out_scale;
+  int general;            // the loss varies from point to point (see nl1_block_I)
   // band values of the convolved intensity
   const int* rowmap;      // [NY] band row index, or -1
   const float* rowband;   // [slabs][nb][NX]
@@ -66,30 +67,39 @@ struct NlcArgs {
   int full;
 };
 
-// Geometry of line group gi: the two field lines it owns and their slabs.
+// Line groups of a block (see RowLines): a uniform base of the block's first
+// group and this lane's 32-bit offset from there; the group's second line
+// lies cs elements after its first.
 struct NlcLines {
-  int64_t item, yp;
-  int64_t off[2];
-  int64_t slab[2];
-  int64_t y[2];
+  int64_t base;          // uniform
+  uint32_t d;
+  int64_t cs;            // uniform
+  uint32_t item, yp;
+  uint32_t item0, yp0;   // uniform: the block's first group
+  uint32_t slab[2], y[2];
 };
 
-__device__ __forceinline__ NlcLines nlc_lines(const NlcArgs& a, int64_t gi, int n) {
+__device__ __forceinline__ NlcLines nlc_lines(const NlcArgs& a, uint32_t g0, uint32_t gi, uint32_t n) {
   NlcLines L;
-  L.item = gi / a.M;
-  L.yp = gi - L.item * a.M;
+  const uint32_t M = (uint32_t)a.M, ny = (uint32_t)a.ny;
+  const bool one = a.M >= a.ngroups;
+  L.item0 = one ? 0u : g0 / M;
+  L.yp0 = g0 - L.item0 * M;
+  L.item = one ? 0u : gi / M;
+  L.yp = gi - L.item * M;
+  const uint32_t rows = ny * (uint32_t)a.ncomp;  // field rows of an item
+  L.base = ((int64_t)L.item0 * rows + L.yp0) * n;
+  L.d = ((L.item - L.item0) * rows + L.yp - L.yp0) * n;
   if (a.ncomp == 1) {
     L.slab[0] = L.slab[1] = L.item;
     L.y[0] = L.yp;
-    L.y[1] = L.yp + a.M;
-    L.off[0] = (L.item * a.ny + L.yp) * n;
-    L.off[1] = L.off[0] + a.M * n;
+    L.y[1] = L.yp + M;
+    L.cs = (int64_t)M * n;
   } else {
     L.slab[0] = 2 * L.item;
     L.slab[1] = 2 * L.item + 1;
     L.y[0] = L.y[1] = L.yp;
-    L.off[0] = (L.slab[0] * a.ny + L.yp) * n;
-    L.off[1] = L.off[0] + a.ny * n;
+    L.cs = (int64_t)ny * n;
   }
   return L;
 }
@@ -102,17 +112,26 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_z(NlcArgs a) {
   constexpr int T = PL::T;
   constexpr int LINE = LdsLine<N, NLSE_ROW_PADSH, 0>::SIZE;
   __shared__ float2 lds[LPB * LINE];
-  const int li = threadIdx.x / T;
-  const int t = threadIdx.x % T;
-  const int64_t gi = (int64_t)blockIdx.x * LPB + li;
-  const bool active = gi < a.ngroups;
-  const NlcLines L = nlc_lines(a, active ? gi : 0, N);
+  constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
+  const int li = LPB == 1 ? 0 : threadIdx.x / T;
+  const int t = LPB == 1 ? threadIdx.x : threadIdx.x % T;
+  // groups past the end work on the last group and store nothing
+  const uint32_t g0 = blockIdx.x * LPB, last = (uint32_t)a.ngroups - 1;
+  const bool active = g0 + li <= last;
+  const uint32_t gi = active ? g0 + li : last;
+  const NlcLines L = nlc_lines(a, g0, gi, N);
   float2* lline = lds + li * LINE;
+  const Buf A0(a.A + L.base), Z0(a.Z + (int64_t)g0 * N), tw(a.tw);
+  const uint32_t d = 8u * (L.d + t), cs = 8u * (uint32_t)L.cs, zd = 8u * ((gi - g0) * N + t);
 
   float2 v[2][P];
-  load_lines<2, P, T>(a.A, L.off, t, active, v);
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int m = 0; m < P; ++m) v[g][m] = A0.load<float2>(d, g * cs + 8u * m * T);
+  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
   if (a.inverse_first) {
-    fft_line<N, P, 2, true, 1>(v, t, a.tw, lline, LINE);
+    fft_line<N, P, 2, true, 1, NLSE_ROW_PADSH, F64, SYNC>(v, t, W, tw, lline, LINE);
     if (a.out_scale != 1.f) {
 #pragma unroll
       for (int g = 0; g < 2; ++g)
@@ -123,7 +142,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_z(NlcArgs a) {
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int m = 0; m < P; ++m) a.A[L.off[g] + t + m * T] = v[g][m];
+        for (int m = 0; m < P; ++m) A0.store(v[g][m], d, g * cs + 8u * m * T);
     }
   }
   if constexpr (FULL) {
@@ -132,33 +151,23 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_z(NlcArgs a) {
     for (int g = 0; g < 2; ++g)
 #pragma unroll
       for (int m = 0; m < P; ++m) v[g][m] = make_float2(sqmag(v[g][m]), 0.f);
-    fft_line<N, P, 2, false, 1, NLSE_ROW_PADSH, F32C>(v, t, a.tw, lline, LINE);
+    fft_line<N, P, 2, false, 1, NLSE_ROW_PADSH, F32C, SYNC>(v, t, W, tw, lline, LINE);
     if (active) {
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int m = 0; m < P; ++m) a.Z[(L.item * a.ny + L.y[g]) * N + t + m * T] = v[g][m];
+        for (int m = 0; m < P; ++m) a.Z[((int64_t)L.item * a.ny + L.y[g]) * N + t + m * T] = v[g][m];
     }
   } else if (a.write_z) {
     float2 z[1][P];
 #pragma unroll
     for (int m = 0; m < P; ++m) z[0][m] = make_float2(sqmag(v[0][m]), sqmag(v[1][m]));
-    fft_line<N, P, 1, false, 1, NLSE_ROW_PADSH, F32C>(z, t, a.tw, lline, LINE);
+    fft_line<N, P, 1, false, 1, NLSE_ROW_PADSH, F32C, SYNC>(z, t, W, tw, lline, LINE);
     if (active) {
 #pragma unroll
-      for (int m = 0; m < P; ++m) a.Z[gi * N + t + m * T] = z[0][m];
+      for (int m = 0; m < P; ++m) Z0.store(z[0][m], zd, 8u * m * T);
     }
   }
-}
-
-// Convolved intensity of point x of a line in row y of slab `slab`: the
-// band value where (y, x) is a band point, else the circular value.
-__device__ __forceinline__ float nlc_band(const NlcArgs& a, int bi, int64_t slab, int64_t y, int x, int n,
-                                          float circ) {
-  if (bi >= 0) return a.rowband[(slab * a.nb + bi) * n + x];
-  if (x < a.r) return a.colband[(slab * a.ny + y) * 2 * a.r + x];
-  if (x >= n - a.r) return a.colband[(slab * a.ny + y) * 2 * a.r + (x - n + 2 * a.r)];
-  return circ;
 }
 
 // Stage 2: the nonlinear operator with the convolved intensities, then
@@ -169,67 +178,72 @@ __device__ __forceinline__ float nlc_band(const NlcArgs& a, int bi, int64_t slab
 // every point and are transformed one line after the other.
 // Both rows of a one-component pair transformed by one two-line F_x
 // (measured 27.9 -> 27.0 us at 2048^2) rather than one after the other.
-#ifndef NLSE_NLNL_PAIR_FX
-#define NLSE_NLNL_PAIR_FX 1
-#endif
 
-template <int N, int P, int LPB, int NC, int FULL = 0>
+template <int N, int P, int LPB, int NC, int FULL = 0, bool GEN = false>
 __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
   constexpr int LINE = LdsLine<N, NLSE_ROW_PADSH, 0>::SIZE;
   __shared__ float2 lds[LPB * LINE];
-  const int li = threadIdx.x / T;
-  const int t = threadIdx.x % T;
-  const int64_t gi = (int64_t)blockIdx.x * LPB + li;
-  const bool active = gi < a.ngroups;
-  const int64_t gs = active ? gi : 0;
-  const NlcLines L = nlc_lines(a, gs, N);
+  constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
+  const int li = LPB == 1 ? 0 : threadIdx.x / T;
+  const int t = LPB == 1 ? threadIdx.x : threadIdx.x % T;
+  // groups past the end work on the last group and store nothing
+  const uint32_t g0 = blockIdx.x * LPB, last = (uint32_t)a.ngroups - 1;
+  const bool active = g0 + li <= last;
+  const uint32_t gi = active ? g0 + li : last;
+  const NlcLines L = nlc_lines(a, g0, gi, N);
   float2* lline = lds + li * LINE;
+  const Buf A0(a.A + L.base), Z0(a.Z + (int64_t)g0 * N), tw(a.tw);
+  const uint32_t d = 8u * (L.d + t), cs = 8u * (uint32_t)L.cs, zd = 8u * ((gi - g0) * N + t);
 
   float2 z[1][P];
 #pragma unroll
   for (int m = 0; m < P; ++m) z[0][m] = make_float2(0.f, 0.f);
   if (!a.direct) {
-    const int64_t zrow = FULL ? L.item * a.ny + L.y[0] : gs;
+    // full: row y of an item's ny, else group g's row
 #pragma unroll
-    // unconditional: lines past the end read line 0 (gs) and store nothing;
-    // a select per element would put each load behind a branch
-    for (int m = 0; m < P; ++m) z[0][m] = a.Z[zrow * N + t + m * T];
+    for (int m = 0; m < P; ++m)
+      z[0][m] = FULL ? a.Z[((int64_t)L.item * a.ny + L.y[0]) * N + t + m * T] : Z0.load<float2>(zd, 8u * m * T);
   }
   float2 v[NC][P];
-  load_lines<NC, P, T>(a.A, L.off, t, active, v);
-  if (!a.direct) fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F32C>(z, t, a.tw, lline, LINE);
-  // z.x: convolved intensity of line 0, z.y: of line 1
-  if (active) {
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const int bi = a.rowmap[L.y[g]];
+  for (int g = 0; g < NC; ++g)
 #pragma unroll
-      for (int m = 0; m < P; ++m) {
-        const float circ = g == 0 ? z[0][m].x : z[0][m].y;
-        const float val = nlc_band(a, bi, L.slab[g], L.y[g], t + m * T, N, circ);
-        if (g == 0)
-          z[0][m].x = val;
-        else
-          z[0][m].y = val;
-      }
+    for (int m = 0; m < P; ++m) v[g][m] = A0.load<float2>(d, g * cs + 8u * m * T);
+  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
+  if (!a.direct) fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F32C, SYNC>(z, t, W, tw, lline, LINE);
+  // z.x: convolved intensity of line 0, z.y: of line 1; band points take
+  // their band values: a band row from the row band, else the r points at
+  // either end from the column band (uniform tests skip the other points)
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int bi = a.rowmap[L.y[g]];
+    const float* rb = a.rowband + ((int64_t)L.slab[g] * a.nb + bi) * N + t;
+    const float* cb = a.colband + ((int64_t)L.slab[g] * a.ny + L.y[g]) * 2 * a.r + t;
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      float& c = g == 0 ? z[0][m].x : z[0][m].y;
+      if (bi >= 0) c = rb[m * T];
+      else if (m * T < a.r && t + m * T < a.r) c = cb[m * T];
+      else if ((m + 1) * T > N - a.r && t + m * T >= N - a.r) c = cb[m * T - N + 2 * a.r];
     }
   }
 
   float vr[P], vi[P];
-  auto load_row_v = [&](int64_t y) {
-    load_v_set<P, T>(a.V, a.vkind, L.item * a.v_item_stride + y * N + t, vr, vi);
+  auto load_row_v = [&](uint32_t y) {
+    load_v_set<P, T, GEN>(a.V, a.vkind, L.item0 * a.v_item_stride + (int64_t)L.yp0 * N,
+                     (L.item - L.item0) * (uint32_t)a.v_item_stride + (y - L.yp0) * N + t, vr, vi);
   };
-  auto finish_line = [&](float2 (&w)[1][P], int64_t off) {
-    if (a.forward_last) fft_line<N, P, 1, false>(w, t, a.tw, lline, LINE);
+  auto finish_line = [&](float2 (&w)[1][P], uint32_t c1) {
+    if (a.forward_last) fft_line<N, P, 1, false, 1, NLSE_ROW_PADSH, F64, SYNC>(w, t, W, tw, lline, LINE);
     if (a.out_scale != 1.f) {
 #pragma unroll
       for (int m = 0; m < P; ++m) w[0][m] = make_float2(w[0][m].x * a.out_scale, w[0][m].y * a.out_scale);
     }
     if (active) {
 #pragma unroll
-      for (int m = 0; m < P; ++m) a.A[off + t + m * T] = w[0][m];
+      for (int m = 0; m < P; ++m) A0.store(w[0][m], d, c1 + 8u * m * T);
     }
   };
 
@@ -242,27 +256,26 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
       float2 z2[1][P];
 #pragma unroll
       for (int m = 0; m < P; ++m)
-        z2[0][m] = a.Z[(L.item * a.ny + L.y[1]) * N + t + m * T];
-      fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F32C>(z2, t, a.tw, lline, LINE);
+        z2[0][m] = a.Z[((int64_t)L.item * a.ny + L.y[1]) * N + t + m * T];
+      fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F32C, SYNC>(z2, t, W, tw, lline, LINE);
 #pragma unroll
       for (int m = 0; m < P; ++m) z[0][m].y = z2[0][m].x;
     }
 #pragma unroll
     for (int m = 0; m < P; ++m) I[m] = z[0][m].x;
     load_row_v(L.y[0]);
-    nl1_block_I<P>(v[0], I, p, a.loss_sat, vr, vi);
-#if NLSE_NLNL_PAIR_FX
+    nl1_block_I<P, GEN>(v[0], I, p, a.loss_sat, a.vkind == V_CPLX, vr, vi);
     // both rows' F_x in one two-line transform
     float2 u[2][P];
 #pragma unroll
     for (int m = 0; m < P; ++m) {
       u[0][m] = v[0][m];
-      u[1][m] = a.A[L.off[1] + t + m * T];
+      u[1][m] = A0.load<float2>(d, cs + 8u * m * T);
       I[m] = z[0][m].y;
     }
     load_row_v(L.y[1]);
-    nl1_block_I<P>(u[1], I, p, a.loss_sat, vr, vi);
-    if (a.forward_last) fft_line<N, P, 2, false, 1>(u, t, a.tw, lline, LINE);
+    nl1_block_I<P, GEN>(u[1], I, p, a.loss_sat, a.vkind == V_CPLX, vr, vi);
+    if (a.forward_last) fft_line<N, P, 2, false, 1, NLSE_ROW_PADSH, F64, SYNC>(u, t, W, tw, lline, LINE);
     if (a.out_scale != 1.f) {
 #pragma unroll
       for (int g = 0; g < 2; ++g)
@@ -273,20 +286,8 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int m = 0; m < P; ++m) a.A[L.off[g] + t + m * T] = u[g][m];
+        for (int m = 0; m < P; ++m) A0.store(u[g][m], d, g * cs + 8u * m * T);
     }
-#else
-    finish_line(v, L.off[0]);
-    float2 w[1][P];
-#pragma unroll
-    for (int m = 0; m < P; ++m) {
-      w[0][m] = a.A[L.off[1] + t + m * T];
-      I[m] = z[0][m].y;
-    }
-    load_row_v(L.y[1]);
-    nl1_block_I<P>(w[0], I, p, a.loss_sat, vr, vi);
-    finish_line(w, L.off[1]);
-#endif
   } else {
     const NLParams2* pp = reinterpret_cast<const NLParams2*>(a.nlp) + 2 * L.item;
     const NLParams2 p1 = pp[0], p2 = pp[1];
@@ -306,7 +307,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
     if (a.has_drive) {
 #pragma unroll
       for (int m = 0; m < P; ++m) {
-        const int64_t ri = L.yp * N + t + m * T;
+        const int64_t ri = (int64_t)L.yp * N + t + m * T;
         float2 q = cmul(a.drv_r0[ri], a.drv_t0);
         q = make_float2(q.x * a.drv_dz, q.y * a.drv_dz);
         v[1][m] = make_float2(v[1][m].x + q.y, v[1][m].y - q.x);
@@ -318,10 +319,10 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
     float2 w[1][P];
 #pragma unroll
     for (int m = 0; m < P; ++m) w[0][m] = v[0][m];
-    finish_line(w, L.off[0]);
+    finish_line(w, 0);
 #pragma unroll
     for (int m = 0; m < P; ++m) w[0][m] = v[1][m];
-    finish_line(w, L.off[1]);
+    finish_line(w, cs);
   }
 }
 

@@ -52,56 +52,92 @@ struct RowArgs {
   float2 drv_t1;
   float drv_dz;
   float out_scale;        // applied to the stored result (1 or 1/N)
+  int general;            // the loss varies from point to point (see nl1_block_I)
+  int through;            // write the result through to memory (ST_THROUGH)
 };
 
-// LDS floats2 of one row block.
+// LDS entries of one row block.
 template <int N, int LPB, int G>
 constexpr int row_lds_size() {
   return LPB * G * LdsLine<N, NLSE_ROW_PADSH, 0>::SIZE;
 }
 
-// Row sweep body: LPB line groups starting at group `g0`.
-template <int N, int P, int LPB, int G>
-__device__ __forceinline__ void row_body(const RowArgs& a, int64_t g0, float2* lds) {
+// Line groups of a row block: a uniform element offset of the block's first
+// group and 32-bit per-lane offsets from there (a block's groups span less
+// than 2^29 elements: at most two items' worth of one component pair).
+template <int N, int G>
+struct RowLines {
+  int64_t base;   // uniform: element offset of the first group's first line
+  uint32_t d;     // this lane's group, relative to base
+  int64_t cs;     // uniform: offset from line 0 to line 1 of a group (G = 2)
+  uint32_t item;
+  uint32_t item0, y0;  // uniform: item and row of the block's first group
+  uint32_t y;
+};
+
+template <int N, int G>
+__device__ __forceinline__ RowLines<N, G> row_lines(uint32_t g0, uint32_t g, uint32_t rows, bool one_item) {
+  RowLines<N, G> L;
+  L.item0 = one_item ? 0u : g0 / rows;
+  L.item = one_item ? 0u : g / rows;
+  L.y0 = g0 - L.item0 * rows;
+  L.y = g - L.item * rows;
+  L.cs = (int64_t)rows * N;
+  if constexpr (G == 1) {
+    L.base = (int64_t)g0 * N;
+    L.d = (g - g0) * N;
+  } else {
+    L.base = ((int64_t)L.item0 * 2 * rows + L.y0) * N;
+    L.d = ((L.item - L.item0) * 2 * rows + L.y - L.y0) * N;
+  }
+  return L;
+}
+
+// Row sweep body: LPB line groups starting at group `g0`.  Groups past the
+// end work on the last group and store nothing.
+template <int N, int P, int LPB, int G, bool GEN, int AR = F64>
+__device__ __forceinline__ void row_body(const RowArgs& a, int64_t g0, xchg_t<AR>* lds) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
   constexpr int LINE = LdsLine<N, NLSE_ROW_PADSH, 0>::SIZE;
+  // the lanes of a line are one wave's or fewer: no block barriers
+  constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
 
-  const int li = threadIdx.x / T;
-  const int t = threadIdx.x % T;
-  const int64_t gi = g0 + li;
-  const bool active = gi < a.ngroups;
-  const int64_t gsafe = active ? gi : 0;
-  const int64_t item = gsafe / a.rows_per_item;
-  const int64_t y = gsafe - item * a.rows_per_item;
-  int64_t off[G];
-  if constexpr (G == 1) {
-    off[0] = gsafe * N;
-  } else {
-    off[0] = ((item * 2) * a.rows_per_item + y) * N;
-    off[1] = off[0] + a.rows_per_item * N;
-  }
-  float2* lline = lds + li * G * LINE;
+  const int li = LPB == 1 ? 0 : threadIdx.x / T;
+  const int t = LPB == 1 ? threadIdx.x : threadIdx.x % T;
+  const uint32_t gi = (uint32_t)g0 + li, last = (uint32_t)a.ngroups - 1;
+  const bool active = gi <= last;
+  const RowLines<N, G> L =
+      row_lines<N, G>((uint32_t)g0, active ? gi : last, (uint32_t)a.rows_per_item, a.rows_per_item >= a.ngroups);
+  const uint32_t item = L.item;
+  xchg_t<AR>* lline = lds + li * G * LINE;
+  const Buf A0(a.A + L.base), tw(a.tw);
+  const uint32_t d = 8u * (L.d + t), cs = 8u * (uint32_t)L.cs;
 
   float2 v[G][P];
-  load_lines<G, P, T>(a.A, off, t, active, v);
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int m = 0; m < P; ++m) v[g][m] = A0.load<float2>(d, g * cs + 8u * m * T);
+  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
 
   // side inputs of the real-space step, fetched with the field so that
   // their latency overlaps the inverse transform
   const bool has_nl = a.has_a || a.has_b;
   float vr[P], vi[P];
-  load_v_set<P, T>(a.V, has_nl ? a.vkind : V_NONE, item * a.v_item_stride + y * N + t, vr, vi);
+  load_v_set<P, T, GEN>(a.V, has_nl ? a.vkind : V_NONE, L.item0 * a.v_item_stride + (int64_t)L.y0 * N,
+                   (item - L.item0) * (uint32_t)a.v_item_stride + (L.y - L.y0) * N + t, vr, vi);
 
-  if (a.inverse_first) fft_line<N, P, G, true>(v, t, a.tw, lline, LINE);
+  if (a.inverse_first) fft_line<N, P, G, true, G, NLSE_ROW_PADSH, AR, SYNC>(v, t, W, tw, lline, LINE);
 
   if constexpr (G == 1) {
-    if (a.has_a) {
-      const NLParams1 pa = reinterpret_cast<const NLParams1*>(a.nlp_a)[item];
-      nl1_block<P>(v[0], pa, a.loss_sat, vr, vi);
-    }
-    if (a.has_b) {
-      const NLParams1 pb = reinterpret_cast<const NLParams1*>(a.nlp_b)[item];
-      nl1_block<P>(v[0], pb, a.loss_sat, vr, vi);
+    // one copy of the code for both applications
+#pragma unroll 1
+    for (int k = 0; k < 2; ++k) {
+      if (k == 0 ? a.has_a : a.has_b) {
+        const NLParams1 q = reinterpret_cast<const NLParams1*>(k == 0 ? a.nlp_a : a.nlp_b)[item];
+        nl1_block<P, GEN>(v[0], q, a.loss_sat, a.vkind == V_CPLX, vr, vi);
+      }
     }
   } else {
     if (a.has_a) {
@@ -117,7 +153,7 @@ __device__ __forceinline__ void row_body(const RowArgs& a, int64_t g0, float2* l
     if (a.has_drive) {
 #pragma unroll
       for (int m = 0; m < P; ++m) {
-        const int64_t ri = y * N + t + m * T;
+        const int64_t ri = (int64_t)L.y * N + t + m * T;
         float2 q = cmul(a.drv_r0[ri], a.drv_t0);
         q = make_float2(q.x * a.drv_dz, q.y * a.drv_dz);
         v[1][m] = make_float2(v[1][m].x + q.y, v[1][m].y - q.x);
@@ -133,7 +169,7 @@ __device__ __forceinline__ void row_body(const RowArgs& a, int64_t g0, float2* l
     }
   }
 
-  if (a.forward_last) fft_line<N, P, G, false>(v, t, a.tw, lline, LINE);
+  if (a.forward_last) fft_line<N, P, G, false, G, NLSE_ROW_PADSH, AR, SYNC>(v, t, W, tw, lline, LINE);
 
   if (a.out_scale != 1.f) {
 #pragma unroll
@@ -142,17 +178,24 @@ __device__ __forceinline__ void row_body(const RowArgs& a, int64_t g0, float2* l
       for (int m = 0; m < P; ++m) v[g][m] = make_float2(v[g][m].x * a.out_scale, v[g][m].y * a.out_scale);
   }
   if (active) {
+    if (a.through) {
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+      for (int g = 0; g < G; ++g)
 #pragma unroll
-      for (int m = 0; m < P; ++m) a.A[off[g] + t + m * T] = v[g][m];
+        for (int m = 0; m < P; ++m) A0.store<ST_THROUGH>(v[g][m], d, g * cs + 8u * m * T);
+    } else {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int m = 0; m < P; ++m) A0.store(v[g][m], d, g * cs + 8u * m * T);
+    }
   }
 }
 
-template <int N, int P, int LPB, int G>
+template <int N, int P, int LPB, int G, bool GEN = false, int AR = F64>
 __global__ __launch_bounds__(LPB*(N / P)) void k_row(RowArgs a) {
-  __shared__ float2 lds[row_lds_size<N, LPB, G>()];
-  row_body<N, P, LPB, G>(a, (int64_t)blockIdx.x * LPB, lds);
+  __shared__ xchg_t<AR> lds[row_lds_size<N, LPB, G>()];
+  row_body<N, P, LPB, G, GEN, AR>(a, (int64_t)blockIdx.x * LPB, lds);
 }
 
 struct ColArgs {
@@ -174,6 +217,7 @@ struct ColArgs {
   int nt;              // columns = NX * NT for PROP_SEP3D
   float scale;         // 1/(NX NY) folded into the propagator
   float out_scale;     // applied to the stored result when no propagator
+  int through;         // write the result through to memory (ST_THROUGH)
 };
 
 // Column sweep.  A block covers W = WT*G adjacent columns of one slab:
@@ -189,112 +233,170 @@ constexpr int col_lds_size() {
   return WT * GR * LdsLine<N, 3, 3>::SIZE;
 }
 
+// The propagator on the natural sets w of G columns c0 + g*CS: complex64
+// products (float2 sets) for the complex64 propagators, FP64 products
+// (double2) for the complex128 ones.
+template <int KIND>
+using prop_t = typename std::conditional<KIND == PROP_SEP3D || KIND == PROP_C128, double2, float2>::type;
+
+template <int N, int P, int G, int CS, int KIND>
+__device__ __forceinline__ void col_prop(const ColArgs& a, prop_t<KIND> (&w)[G][P], int comp, int t, int c0) {
+  constexpr int T = N / P;
+  if constexpr (KIND == PROP_SEP64) {
+    const Buf pyb(a.py + comp * N);
+    double2 px[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) px[g] = a.px[comp * a.NX + c0 + g * CS];
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      const double2 py = pyb.load<double2>(16u * t, 16u * m * T);
+#pragma unroll
+      for (int g = 0; g < G; ++g) w[g][m] = prop_sep_c64(w[g][m], px[g], py, a.scale);
+    }
+  } else if constexpr (KIND == PROP_SEP3D) {
+    // column c = x*NT + t of an (NY, NX, NT) field: complex64(px*py)
+    // times the complex128 temporal factor
+    const Buf pyb(a.py);
+    double2 px[G], pt[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int col = c0 + g * CS;
+      px[g] = a.px[col / a.nt];
+      pt[g] = a.pt[col % a.nt];
+      pt[g].x *= (double)a.scale;
+      pt[g].y *= (double)a.scale;
+    }
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      const double2 py = pyb.load<double2>(16u * t, 16u * m * T);
+#pragma unroll
+      for (int g = 0; g < G; ++g) w[g][m] = prop_sep3d(w[g][m], px[g], py, pt[g]);
+    }
+  } else if constexpr (KIND == PROP_C128) {
+    const double2* pt = a.ptab128 + c0;
+#pragma unroll
+    for (int m = 0; m < P; ++m)
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        w[g][m] = prop_c128(w[g][m], pt[(int64_t)(t + m * T) * a.NX + g * CS], (double)a.scale);
+  } else {
+    const float2* pt = a.ptab + (int64_t)comp * N * a.NX + c0;
+#pragma unroll
+    for (int m = 0; m < P; ++m)
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        w[g][m] = prop_c64(w[g][m], pt[(int64_t)(t + m * T) * a.NX + g * CS], a.scale);
+  }
+}
+
 // Column sweep body for tile `b` (tile index over slabs x tiles per slab).
 // PK >= 0 compiles only that propagator kind (fewer live registers); -1
 // dispatches on a.pkind.
-template <int N, int P, int WT, int G, int GR, int PK = -1>
-__device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, float2* lds) {
+template <int N, int P, int WT, int G, int GR, int PK = -1, int FA = F64>
+__device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>* lds) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
   constexpr int LINE = LdsLine<N, 3, 3>::SIZE;
-  constexpr int W = WT * G;
+  constexpr int TILE = WT * G;
 
   const int cw = threadIdx.x % WT;
   const int t = threadIdx.x / WT;
-  const int tiles = a.NX / W;
-  const int64_t slab = b / tiles;
+  const uint32_t tiles = (uint32_t)a.NX / TILE;
+  const uint32_t slab = (uint32_t)b / tiles;
   // column of line g: c0 + g * CS.  Two lines per thread take adjacent
   // columns (PAIRED, CS = 1), so a thread moves 16 bytes per row and a
   // wave's load covers whole 64-byte row segments; otherwise lines are WT
   // apart (a one-column tile, WT = G = 1, also has CS = 1 but is not paired)
   constexpr bool PAIRED = G == 2 && NLSE_COL_PAIRED;
   constexpr int CS = PAIRED ? 1 : WT;
-  const int c0 = (int)(b % tiles) * W + (PAIRED ? G * cw : cw);
-  const int64_t base = slab * (int64_t)N * a.NX + c0;
-  float2* lline = lds + cw * GR * LINE;
+  const int u0 = (int)((uint32_t)b - slab * tiles) * TILE;  // uniform: first column of the tile
+  const int c0 = u0 + (PAIRED ? G * cw : cw);
+  // slabs below 4 GiB are addressed from a uniform descriptor; the PK = -1
+  // instance takes any size (the launcher chooses)
+  constexpr bool WIDE = PK == -1;
+  float2* const A0 = a.A + (int64_t)slab * N * a.NX + u0;
+  const Buf AB(A0), tw(a.tw);
+  const uint32_t rs = 8u * (uint32_t)T * (uint32_t)a.NX;
+  const uint32_t d = 8u * ((uint32_t)t * (uint32_t)a.NX + (uint32_t)(c0 - u0));
+  xchg_t<FA>* lline = lds + cw * GR * LINE;
 
   float2 v[G][P];
 #pragma unroll
   for (int m = 0; m < P; ++m) {
-    if constexpr (PAIRED) {
-      const float4 q = *reinterpret_cast<const float4*>(a.A + base + (int64_t)(t + m * T) * a.NX);
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) v[g][m] = A0[(int64_t)(t + m * T) * a.NX + (c0 - u0) + g * CS];
+    } else if constexpr (PAIRED) {
+      const float4 q = AB.load<float4>(d, m * rs);
       v[0][m] = make_float2(q.x, q.y);
       v[1][m] = make_float2(q.z, q.w);
     } else {
 #pragma unroll
-      for (int g = 0; g < G; ++g) v[g][m] = a.A[base + (int64_t)(t + m * T) * a.NX + g * WT];
+      for (int g = 0; g < G; ++g) v[g][m] = AB.load<float2>(d, m * rs + 8u * g * WT);
     }
   }
+  Twid<N, P> W;
+  if constexpr (PK != PROP_KREAL) W = load_twiddles<N, P>(tw, t);
 
-  // the real spectrum multiplies an intensity (nonlocal response): its
-  // transforms are FP32 (see FftArith); field transforms are FP64
-  constexpr int AR = PK == PROP_KREAL ? F32C : F64;
-  if (a.do_fwd) fft_line<N, P, G, false, GR, 3, AR>(v, t, a.tw, lline, LINE);
-  const int pkind = PK >= 0 ? PK : a.pkind;
-  if (PK != PK_NONE && a.do_prop) {
-    const int comp = (int)(slab % a.ncomp);
-    if ((PK < 0 || PK == PROP_SEP64) && pkind == PROP_SEP64) {
-      double2 px[G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) px[g] = a.px[comp * a.NX + c0 + g * CS];
-#pragma unroll
-      for (int m = 0; m < P; ++m) {
-        const double2 py = a.py[comp * N + t + m * T];
-#pragma unroll
-        for (int g = 0; g < G; ++g) v[g][m] = prop_sep_c64(v[g][m], px[g], py, a.scale);
-      }
-    } else if ((PK < 0 || PK == PROP_SEP3D) && pkind == PROP_SEP3D) {
-      // column c = x*NT + t of an (NY, NX, NT) field: complex64(px*py)
-      // times the complex128 temporal factor, applied in FP64
-      double2 px[G], pt[G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int col = c0 + g * CS;
-        px[g] = a.px[col / a.nt];
-        pt[g] = a.pt[col % a.nt];
-      }
-#pragma unroll
-      for (int m = 0; m < P; ++m) {
-        const double2 py = a.py[t + m * T];
-#pragma unroll
-        for (int g = 0; g < G; ++g) v[g][m] = prop_sep3d(v[g][m], px[g], py, pt[g], (double)a.scale);
-      }
-    } else if ((PK < 0 || PK == PROP_KREAL) && pkind == PROP_KREAL) {
-      // even real spectrum: entry (ky, kx) of the quadrant table at
-      // (min(ky, N-ky), min(kx, NX-kx))
-      const int hx = a.NX / 2 + 1;
-      int kx[G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int col = c0 + g * CS;
-        kx[g] = col <= a.NX / 2 ? col : a.NX - col;
-      }
-#pragma unroll
-      for (int m = 0; m < P; ++m) {
-        const int ky = t + m * T;
-        const int kyq = ky <= N / 2 ? ky : N - ky;
+  constexpr int PADSH = 3;
+  if constexpr (PK >= 0 && PK != PK_NONE && PK != PROP_KREAL) {
+    // F_y, propagator, I_y; with a complex128 propagator the field stays in
+    // FP64 from the last forward stage to the first inverse one
+    prop_t<PK> w[G][P];
+    fft_line_io<N, P, G, false, GR, PADSH, FA, SYNC_BLOCK>(v, w, t, W, tw, lline, LINE);
+    const int comp = (int)(slab % (uint32_t)a.ncomp);
+    col_prop<N, P, G, CS, PK>(a, w, comp, t, c0);
+    fft_line_io<N, P, G, true, GR, PADSH, FA, SYNC_BLOCK>(w, v, t, W, tw, lline, LINE);
+  } else {
+    // the real spectrum multiplies an intensity (nonlocal response): its
+    // transforms are FP32 (see FftArith); field transforms are FP64
+    constexpr int AR = PK == PROP_KREAL ? F32C : FA;
+    static_assert(PK != PROP_KREAL || FA != F64X, "FP32 exchange");
+    if (a.do_fwd) fft_line<N, P, G, false, GR, PADSH, AR>(v, t, W, tw, lline, LINE);
+    if (PK != PK_NONE && a.do_prop) {
+      const int comp = (int)(slab % (uint32_t)a.ncomp);
+      if (PK == PROP_KREAL || a.pkind == PROP_KREAL) {
+        // even real spectrum: entry (ky, kx) of the quadrant table at
+        // (min(ky, N-ky), min(kx, NX-kx))
+        const int hx = a.NX / 2 + 1;
+        int kx[G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          const float f = a.kq[kyq * hx + kx[g]] * a.scale;
-          v[g][m] = make_float2(v[g][m].x * f, v[g][m].y * f);
+          const int col = c0 + g * CS;
+          kx[g] = col <= a.NX / 2 ? col : a.NX - col;
+        }
+#pragma unroll
+        for (int m = 0; m < P; ++m) {
+          const int ky = t + m * T;
+          const int kyq = ky <= N / 2 ? ky : N - ky;
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            const float f = a.kq[kyq * hx + kx[g]] * a.scale;
+            v[g][m] = make_float2(v[g][m].x * f, v[g][m].y * f);
+          }
+        }
+      } else if constexpr (PK < 0) {
+        if (a.pkind == PROP_SEP64) {
+          col_prop<N, P, G, CS, PROP_SEP64>(a, v, comp, t, c0);
+        } else if (a.pkind == PROP_C64) {
+          col_prop<N, P, G, CS, PROP_C64>(a, v, comp, t, c0);
+        } else {
+          double2 w[G][P];
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int m = 0; m < P; ++m) w[g][m] = to_f64(v[g][m]);
+          if (a.pkind == PROP_SEP3D) col_prop<N, P, G, CS, PROP_SEP3D>(a, w, comp, t, c0);
+          else col_prop<N, P, G, CS, PROP_C128>(a, w, comp, t, c0);
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int m = 0; m < P; ++m) v[g][m] = to_f32(w[g][m]);
         }
       }
-    } else if ((PK < 0 || PK == PROP_C128) && pkind == PROP_C128) {
-      const double2* pt = a.ptab128 + c0;
-#pragma unroll
-      for (int m = 0; m < P; ++m)
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-          v[g][m] = prop_c128(v[g][m], pt[(int64_t)(t + m * T) * a.NX + g * CS], (double)a.scale);
-    } else if (PK < 0 || PK == PROP_C64) {
-      const float2* pt = a.ptab + (int64_t)comp * N * a.NX + c0;
-#pragma unroll
-      for (int m = 0; m < P; ++m)
-#pragma unroll
-        for (int g = 0; g < G; ++g) v[g][m] = prop_c64(v[g][m], pt[(int64_t)(t + m * T) * a.NX + g * CS], a.scale);
     }
+    if (a.do_inv) fft_line<N, P, G, true, GR, PADSH, AR>(v, t, W, tw, lline, LINE);
   }
-  if (a.do_inv) fft_line<N, P, G, true, GR, 3, AR>(v, t, a.tw, lline, LINE);
 
   if (a.out_scale != 1.f) {
 #pragma unroll
@@ -302,29 +404,36 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, float2* ld
 #pragma unroll
       for (int m = 0; m < P; ++m) v[g][m] = make_float2(v[g][m].x * a.out_scale, v[g][m].y * a.out_scale);
   }
+  auto put = [&](auto st) {
+    constexpr int ST = decltype(st)::value;
 #pragma unroll
-  for (int m = 0; m < P; ++m) {
-    if constexpr (PAIRED) {
-      *reinterpret_cast<float4*>(a.A + base + (int64_t)(t + m * T) * a.NX) =
-          make_float4(v[0][m].x, v[0][m].y, v[1][m].x, v[1][m].y);
-    } else {
+    for (int m = 0; m < P; ++m) {
+      if constexpr (WIDE) {
 #pragma unroll
-      for (int g = 0; g < G; ++g) a.A[base + (int64_t)(t + m * T) * a.NX + g * WT] = v[g][m];
+        for (int g = 0; g < G; ++g) A0[(int64_t)(t + m * T) * a.NX + (c0 - u0) + g * CS] = v[g][m];
+      } else if constexpr (PAIRED) {
+        AB.template store<ST>(make_float4(v[0][m].x, v[0][m].y, v[1][m].x, v[1][m].y), d, m * rs);
+      } else {
+#pragma unroll
+        for (int g = 0; g < G; ++g) AB.template store<ST>(v[g][m], d, m * rs + 8u * g * WT);
+      }
     }
-  }
+  };
+  if (!WIDE && a.through) put(std::integral_constant<int, ST_THROUGH>{});
+  else put(std::integral_constant<int, ST_BACK>{});
 }
 
 // PK: the propagator kind compiled in (-1: any kind, chosen at run time).
-template <int N, int P, int WT, int G, int GR, int PK = -1>
+template <int N, int P, int WT, int G, int GR, int PK = -1, int FA = F64>
 __global__ __launch_bounds__(WT*(N / P)) void k_col(ColArgs a) {
-  __shared__ float2 lds[col_lds_size<N, WT, GR>()];
+  __shared__ xchg_t<FA> lds[col_lds_size<N, WT, GR>()];
   // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs,
   // so block b runs on XCD b % 8; give each XCD a contiguous range of
   // tiles so that the two 64-byte halves of a 128-byte line are fetched
   // by neighbouring tiles on the same XCD (one L2 fill instead of two)
   const int64_t nblk = (int64_t)gridDim.x;
   const int64_t b = (nblk % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8 : blockIdx.x;
-  col_body<N, P, WT, G, GR, PK>(a, b, lds);
+  col_body<N, P, WT, G, GR, PK, FA>(a, b, lds);
 }
 
 // Intensity convolution over the full NY-row torus (a response given by
@@ -360,6 +469,8 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
   const int ca = j, cb = j == 0 ? 0 : a.NX - j;
   float2* Z = a.A + slab * (int64_t)(N / 2) * a.NX;
   float2* lline = lds + cw * LINE;
+  const Buf tw(a.tw);
+  const Twid<N, P> W{};  // (FP64 twiddles: none here)
 
   float2 v[1][P];
 #pragma unroll
@@ -369,7 +480,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
     v[0][m] = make_float2(0.5f * (za.x + zb.x), 0.5f * (za.y - zb.y));
     v[0][m + H] = make_float2(0.5f * (za.y + zb.y), 0.5f * (zb.x - za.x));
   }
-  fft_line<N, P, 1, false, 1, 3, F32C>(v, t, a.tw, lline, LINE);
+  fft_line<N, P, 1, false, 1, 3, F32C>(v, t, W, tw, lline, LINE);
   const int hx = a.NX / 2 + 1;
 #pragma unroll
   for (int m = 0; m < P; ++m) {
@@ -378,7 +489,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
     const float f = a.kq[kyq * hx + j] * a.scale;
     v[0][m] = make_float2(v[0][m].x * f, v[0][m].y * f);
   }
-  fft_line<N, P, 1, true, 1, 3, F32C>(v, t, a.tw, lline, LINE);
+  fft_line<N, P, 1, true, 1, 3, F32C>(v, t, W, tw, lline, LINE);
   if (act) {
 #pragma unroll
     for (int m = 0; m < H; ++m) {
@@ -449,13 +560,15 @@ struct Line1DArgs {
   int vkind;
   const double* nlk;      // nonlocal kernel [2*nlr+1] (null: local response)
   int nlr;
+  int general;            // the loss varies from point to point (see nl1_block_I)
 };
 
-template <int N, int P, int LPB, int G>
+template <int N, int P, int LPB, int G, bool GEN = false>
 __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
   constexpr int LINE = LdsLine<N, NLSE_ROW_PADSH, 0>::SIZE;
+  constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
   __shared__ float2 lds[LPB * G * LINE];
   const int li = threadIdx.x / T;
   const int t = threadIdx.x % T;
@@ -473,7 +586,9 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
 #pragma unroll
     for (int m = 0; m < P; ++m) v[g][m] = active ? a.A[off[g] + t + m * T] : make_float2(0.f, 0.f);
   float vr[P], vi[P];
-  load_v_set<P, T>(a.V, a.vkind, t, vr, vi);
+  load_v_set<P, T, GEN>(a.V, a.vkind, 0, (uint32_t)t, vr, vi);
+  const Buf tw(a.tw);
+  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
   double2 pr[G][P];
 #pragma unroll
   for (int g = 0; g < G; ++g)
@@ -487,7 +602,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
       conv1d_intensity<N, P, G>(v, I, reinterpret_cast<float*>(lline), t, a.nlk, a.nlr);
       if constexpr (G == 1) {
         const NLParams1 p = reinterpret_cast<const NLParams1*>(prm)[item];
-        nl1_block_I<P>(v[0], I[0], p, a.loss_sat, vr, vi);
+        nl1_block_I<P, GEN>(v[0], I[0], p, a.loss_sat, a.vkind == V_CPLX, vr, vi);
       } else {
         const NLParams2* pp = reinterpret_cast<const NLParams2*>(prm) + 2 * item;
         const NLParams2 p1 = pp[0], p2 = pp[1];
@@ -495,7 +610,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
       }
     } else if constexpr (G == 1) {
       const NLParams1 p = reinterpret_cast<const NLParams1*>(prm)[item];
-      nl1_block<P>(v[0], p, a.loss_sat, vr, vi);
+      nl1_block<P, GEN>(v[0], p, a.loss_sat, a.vkind == V_CPLX, vr, vi);
     } else {
       const NLParams2* pp = reinterpret_cast<const NLParams2*>(prm) + 2 * item;
       const NLParams2 p1 = pp[0], p2 = pp[1];
@@ -505,12 +620,13 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
 
   for (int64_t s = 0; s < a.nsteps; ++s) {
     if (a.precision == 1) apply_nl(a.nl_pre);
-    fft_line<N, P, G, false>(v, t, a.tw, lline, LINE);
+    double2 w[G][P];
+    fft_line_io<N, P, G, false, G, NLSE_ROW_PADSH, F64, SYNC>(v, w, t, W, tw, lline, LINE);
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = prop_c128(v[g][m], pr[g][m], a.scale);
-    fft_line<N, P, G, true>(v, t, a.tw, lline, LINE);
+      for (int m = 0; m < P; ++m) w[g][m] = prop_c128(w[g][m], pr[g][m], a.scale);
+    fft_line_io<N, P, G, true, G, NLSE_ROW_PADSH, F64, SYNC>(w, v, t, W, tw, lline, LINE);
     if (a.precision == 1) {
       apply_nl(a.nl_post);
     } else {

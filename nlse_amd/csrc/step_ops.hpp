@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fft_line.hpp"
+
 namespace nlse {
 
 // A complex step dz = dr + i di (imaginary-time evolution, nlse.py:505-508)
@@ -86,30 +88,40 @@ __device__ __forceinline__ float recip(float d) {
   return fmaf(r, fmaf(-d, r, 1.0f), r);
 }
 
-// Library evaluation for arguments outside the polynomial range (kept out
-// of line: it is rarely taken and large).
-__device__ __noinline__ void sincos_expm1_lib(float h, float a, float* s, float* c, float* em) {
-  *em = expm1f(-a);
-  sincosf(h, s, c);
+__device__ __forceinline__ bool wave_all(bool c) {
+  return __builtin_amdgcn_read_exec() == __builtin_amdgcn_ballot_w64(c);
+}
+__device__ __forceinline__ bool wave_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
+
+// A *= exp(-a + i th) for n points in memory with the library functions, for
+// arguments outside the series' ranges (a strided by `as`: 0 for one loss).
+// Out of line and on a copy of the points: rarely taken, and a call amid the
+// points would tie up the registers of the common path.
+__device__ __noinline__ void phase_loss_lib(float2* A, const float* a, int as, const float* th, int n) {
+  for (int m = 0; m < n; ++m) {
+    float s2, c2;
+    const float em = expm1f(-a[m * as]);
+    sincosf(0.5f * th[m], &s2, &c2);
+    const float cm1 = -2.0f * s2 * s2;
+    const float dr = fmaf(em, 1.0f + cm1, cm1);
+    const float di = (1.0f + em) * (2.0f * s2 * c2);
+    A[m] = make_float2(A[m].x + fmaf(A[m].x, dr, -A[m].y * di), A[m].y + fmaf(A[m].y, dr, A[m].x * di));
+  }
 }
 
-__device__ __forceinline__ float2 apply_phase_loss(float2 A, float a, float theta) {
-  const float h = 0.5f * theta;
-  float em, s2, c2;
-  // wave-uniform choice: the polynomial range covers the physical steps
-  // (|theta| <= pi/2 and |a| <= 1/8 per step); otherwise the library calls
-  if (__builtin_amdgcn_read_exec() == __builtin_amdgcn_ballot_w64(fabsf(h) <= 0.78539816f && fabsf(a) <= 0.125f)) {
-    em = expm1_small(-a);
-    sincos_small(h, s2, c2);
-  } else {
-    sincos_expm1_lib(h, a, &s2, &c2, &em);
+template <int P>
+__device__ __forceinline__ void phase_loss_slow(float2* A, const float* a, int as, const float* th) {
+  float2 tA[P];
+  float ta[P], tt[P];
+#pragma unroll
+  for (int m = 0; m < P; ++m) {
+    tA[m] = A[m];
+    ta[m] = a[m * as];
+    tt[m] = th[m];
   }
-  const float cosm1 = -2.0f * s2 * s2;
-  const float dr = fmaf(em, 1.0f + cosm1, cosm1);
-  const float di = (1.0f + em) * (2.0f * s2 * c2);
-  const float cx = fmaf(A.x, dr, -A.y * di);
-  const float cy = fmaf(A.y, dr, A.x * di);
-  return make_float2(A.x + cx, A.y + cy);
+  phase_loss_lib(tA, ta, 1, tt, P);
+#pragma unroll
+  for (int m = 0; m < P; ++m) A[m] = tA[m];
 }
 
 // Apply exp(-a + i theta) to P points with one wave-uniform choice of the
@@ -119,7 +131,7 @@ __device__ __forceinline__ void apply_phase_loss_block(float2* A, const float* a
   bool small = true;
 #pragma unroll
   for (int m = 0; m < P; ++m) small = small && fabsf(0.5f * theta[m]) <= 0.78539816f && fabsf(a[m]) <= 0.125f;
-  if (__builtin_amdgcn_read_exec() == __builtin_amdgcn_ballot_w64(small)) {
+  if (wave_all(small)) {
 #pragma unroll
     for (int m = 0; m < P; ++m) {
       float s2, c2;
@@ -133,36 +145,101 @@ __device__ __forceinline__ void apply_phase_loss_block(float2* A, const float* a
       A[m] = make_float2(A[m].x + cx, A[m].y + cy);
     }
   } else {
+    phase_loss_slow<P>(A, a, 1, theta);
+  }
+}
+
+__device__ __forceinline__ float2 apply_phase_loss(float2 A, float a, float theta) {
+  apply_phase_loss_block<1>(&A, &a, &theta);
+  return A;
+}
+
+// sin(x) and cos(x) - 1 for |x| <= 1/4: Taylor series to x^7 and x^6 (next
+// terms: 4e-11 and 6e-9 relative).
+__device__ __forceinline__ void sincosm1_quarter(float x, float& s, float& cm1) {
+  const float x2 = x * x;
+  float ps = fmaf(x2, -1.98412698e-4f, 8.33333333e-3f);
+  ps = fmaf(x2, ps, -1.66666667e-1f);
+  s = fmaf(x * x2, ps, x);
+  float pc = fmaf(x2, -1.38888889e-3f, 4.16666667e-2f);
+  pc = fmaf(x2, pc, -0.5f);
+  cm1 = x2 * pc;
+}
+
+// A *= exp(-a + i th[m]) on P points with one loss `a` for all of them:
+// e^{-a} - 1 is evaluated once, and steps of small phase (the wave's largest
+// |th| <= 1/4) take the short series: about 17 operations per point against
+// 38 of apply_phase_loss_block.
+template <int P>
+__device__ __forceinline__ void apply_phase_block(float2* A, float a, const float* th) {
+  bool quarter = fabsf(a) <= 0.125f, half = quarter;
+#pragma unroll
+  for (int m = 0; m < P; ++m) {
+    quarter = quarter && fabsf(th[m]) <= 0.25f;
+    half = half && fabsf(th[m]) <= 1.5707963f;
+  }
+  const float em = expm1_small(-a), e1 = 1.0f + em;
+  if (wave_all(quarter)) {
+#pragma unroll
     for (int m = 0; m < P; ++m) {
-      float s2, c2, em;
-      sincos_expm1_lib(0.5f * theta[m], a[m], &s2, &c2, &em);
-      const float cosm1 = -2.0f * s2 * s2;
-      const float dr = fmaf(em, 1.0f + cosm1, cosm1);
-      const float di = (1.0f + em) * (2.0f * s2 * c2);
-      const float cx = fmaf(A[m].x, dr, -A[m].y * di);
-      const float cy = fmaf(A[m].y, dr, A[m].x * di);
-      A[m] = make_float2(A[m].x + cx, A[m].y + cy);
+      float sn, cm1;
+      sincosm1_quarter(th[m], sn, cm1);
+      const float dr = fmaf(e1, cm1, em), di = e1 * sn;
+      A[m] = make_float2(A[m].x + fmaf(A[m].x, dr, -A[m].y * di), A[m].y + fmaf(A[m].y, dr, A[m].x * di));
     }
+  } else if (wave_all(half)) {
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      float s2, c2;
+      sincos_small(0.5f * th[m], s2, c2);
+      const float cm1 = -2.0f * s2 * s2;
+      const float dr = fmaf(e1, cm1, em), di = e1 * (2.0f * s2 * c2);
+      A[m] = make_float2(A[m].x + fmaf(A[m].x, dr, -A[m].y * di), A[m].y + fmaf(A[m].y, dr, A[m].x * di));
+    }
+  } else {
+    phase_loss_slow<P>(A, &a, 0, th);
+  }
+}
+
+// nl_prop on P points with the intensity I given per point (|A|^2, or its
+// convolution for the nonlocal response) and the potential vr + i vi (has_vi,
+// uniform: a complex one).  GEN: instances that also take losses which vary
+// from point to point (saturated loss, complex V, complex dz).
+template <int P, bool GEN>
+__device__ __forceinline__ void nl1_block_I(float2* A, const float* I, const struct NLParams1& p, bool loss_sat,
+                                            bool has_vi, const float* vr, const float* vi) {
+  float th[P];
+  if (!GEN || !(loss_sat || has_vi || wave_any(p.cplx != 0))) {
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      const float sat = recip(fmaf(I[m], p.inv_isat, 1.0f));
+      th[m] = fmaf(p.gdz * I[m], sat, p.vdz * vr[m]);
+    }
+    apply_phase_block<P>(A, p.adz, th);
+  } else {
+    float a[P];
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      const float sat = recip(fmaf(I[m], p.inv_isat, 1.0f));
+      th[m] = fmaf(p.gdz * I[m], sat, p.vdz * vr[m]);
+      a[m] = fmaf(p.vdz, vi[m], loss_sat ? p.adz * sat : p.adz);
+      if (p.cplx) {
+        a[m] = fmaf(p.gdz_i * I[m], sat, fmaf(p.vdz_i, vr[m], a[m]));
+        th[m] -= fmaf(p.vdz_i, vi[m], loss_sat ? p.adz_i * sat : p.adz_i);
+      }
+    }
+    apply_phase_loss_block<P>(A, a, th);
   }
 }
 
 // nl_prop on P points (see nl1), potential values given per point.
-template <int P>
-__device__ __forceinline__ void nl1_block(float2* A, const struct NLParams1& p, bool loss_sat, const float* vr,
-                                          const float* vi) {
-  float a[P], th[P];
+template <int P, bool GEN>
+__device__ __forceinline__ void nl1_block(float2* A, const struct NLParams1& p, bool loss_sat, bool has_vi,
+                                          const float* vr, const float* vi) {
+  float I[P];
 #pragma unroll
-  for (int m = 0; m < P; ++m) {
-    const float I = A[m].x * A[m].x + A[m].y * A[m].y;
-    const float sat = recip(fmaf(I, p.inv_isat, 1.0f));
-    th[m] = fmaf(p.gdz * I, sat, p.vdz * vr[m]);
-    a[m] = fmaf(p.vdz, vi[m], loss_sat ? p.adz * sat : p.adz);
-    if (p.cplx) {
-      a[m] = fmaf(p.gdz_i * I, sat, fmaf(p.vdz_i, vr[m], a[m]));
-      th[m] -= fmaf(p.vdz_i, vi[m], loss_sat ? p.adz_i * sat : p.adz_i);
-    }
-  }
-  apply_phase_loss_block<P>(A, a, th);
+  for (int m = 0; m < P; ++m) I[m] = A[m].x * A[m].x + A[m].y * A[m].y;
+  nl1_block_I<P, GEN>(A, I, p, loss_sat, has_vi, vr, vi);
 }
 
 // The imaginary-dz terms of one two-component application (see NLParams2).
@@ -194,25 +271,6 @@ __device__ __forceinline__ void nl2_block(float2* A1, float2* A2, const struct N
   }
   apply_phase_loss_block<P>(A1, a1, t1);
   apply_phase_loss_block<P>(A2, a2, t2);
-}
-
-// nl_prop with a given intensity per point (the nonlocal response
-// replaces |A|^2 by its convolution with the kernel, nlse.py:444-447).
-template <int P>
-__device__ __forceinline__ void nl1_block_I(float2* A, const float* I, const struct NLParams1& p, bool loss_sat,
-                                            const float* vr, const float* vi) {
-  float a[P], th[P];
-#pragma unroll
-  for (int m = 0; m < P; ++m) {
-    const float sat = recip(fmaf(I[m], p.inv_isat, 1.0f));
-    th[m] = fmaf(p.gdz * I[m], sat, p.vdz * vr[m]);
-    a[m] = fmaf(p.vdz, vi[m], loss_sat ? p.adz * sat : p.adz);
-    if (p.cplx) {
-      a[m] = fmaf(p.gdz_i * I[m], sat, fmaf(p.vdz_i, vr[m], a[m]));
-      th[m] -= fmaf(p.vdz_i, vi[m], loss_sat ? p.adz_i * sat : p.adz_i);
-    }
-  }
-  apply_phase_loss_block<P>(A, a, th);
 }
 
 template <int P>
@@ -250,23 +308,24 @@ __device__ __forceinline__ void load_v(const void* V, int vkind, int64_t idx, fl
   }
 }
 
-// V at the P points base + m*T of a line (vr, vi zero without V).  The kind
-// is tested once for the whole set: with a per-point test the compiler
-// waits for each load at the branch join, serialising P load latencies.
-template <int P, int T>
-__device__ __forceinline__ void load_v_set(const void* V, int vkind, int64_t base, float* vr, float* vi) {
+// V at the P points base + d + m*T of a line (base uniform, d per lane; vr,
+// vi zero without V).  The kind is tested once for the whole set: with a
+// per-point test the compiler waits for each load at the branch join,
+// serialising P load latencies.
+template <int P, int T, bool CPLX = true>
+__device__ __forceinline__ void load_v_set(const void* V, int vkind, int64_t base, uint32_t d, float* vr, float* vi) {
   if (vkind == V_REAL) {
-    const float* p = reinterpret_cast<const float*>(V) + base;
+    const Buf p(reinterpret_cast<const float*>(V) + base);
 #pragma unroll
     for (int m = 0; m < P; ++m) {
-      vr[m] = p[m * T];
+      vr[m] = p.load<float>(4u * d, 4u * m * T);
       vi[m] = 0.f;
     }
-  } else if (vkind == V_CPLX) {
-    const float2* p = reinterpret_cast<const float2*>(V) + base;
+  } else if (CPLX && vkind == V_CPLX) {
+    const Buf p(reinterpret_cast<const float2*>(V) + base);
 #pragma unroll
     for (int m = 0; m < P; ++m) {
-      const float2 w = p[m * T];
+      const float2 w = p.load<float2>(8u * d, 8u * m * T);
       vr[m] = w.x;
       vi[m] = w.y;
     }
@@ -315,7 +374,11 @@ __device__ __forceinline__ void rabi(float2& A1, float2& A2, const RabiParams& r
 
 // A_c64 * P where P is the complex64 rounding of the FP64 product px*py
 // (the reference builds exp(-i(kx^2+ky^2) dz/2k) in FP64 and casts it to
-// complex64, nlse.py:194-197).  `scale` is an exact power of two (1/N).
+// complex64, nlse.py:194-197).  `scale` is an exact power of two (1/N).  The
+// product is a complex64 one, as the reference's: its FP32 roundings are not
+// free of bias (-2.8e-9 of the power per step in the speckle workload), and
+// an FP64 product, nearer to the exact result, would leave the complex64
+// reference by 5e-6 of the power over 2001 steps.
 __device__ __forceinline__ float2 prop_sep_c64(float2 A, double2 px, double2 py, float scale) {
   const double pr = fma(px.x, py.x, -px.y * py.y);
   const double pi = fma(px.x, py.y, px.y * py.x);
@@ -329,25 +392,22 @@ __device__ __forceinline__ float2 prop_c64(float2 A, float2 P, float scale) {
   return make_float2(fmaf(A.x, P.x, -A.y * P.y), fmaf(A.x, P.y, A.y * P.x));
 }
 
-// complex64 field times a complex128 propagator, computed in FP64 with one
-// rounding (numpy multiplies complex64 by complex128 in complex128 and casts
-// back, nlse_1d.py:104, nlse_3d.py:112).
-__device__ __forceinline__ float2 prop_c128(float2 A, double2 P, double scale) {
-  const double ax = A.x, ay = A.y;
+// A times a complex128 propagator (numpy multiplies complex64 by complex128
+// in complex128 and casts back, nlse_1d.py:104, nlse_3d.py:112).
+__device__ __forceinline__ double2 prop_c128(double2 A, double2 P, double scale) {
   const double px = P.x * scale, py = P.y * scale;
-  return make_float2((float)fma(ax, px, -ay * py), (float)fma(ax, py, ay * px));
+  return make_double2(fma(A.x, px, -A.y * py), fma(A.x, py, A.y * px));
 }
 
 // 3-D propagator (nlse_3d.py:105-114): P = complex64(px*py) (the 2-D part,
-// cast to complex64 by the reference) times the complex128 temporal
-// factor; the product and A*P are evaluated in FP64 and rounded once.
-__device__ __forceinline__ float2 prop_sep3d(float2 A, double2 px, double2 py, double2 pt, double scale) {
+// cast to complex64 by the reference) times the complex128 temporal factor
+// pt (scaled by 1/N).
+__device__ __forceinline__ double2 prop_sep3d(double2 A, double2 px, double2 py, double2 pt) {
   const double p2r = (double)(float)fma(px.x, py.x, -px.y * py.y);
   const double p2i = (double)(float)fma(px.x, py.y, px.y * py.x);
-  const double pr = fma(p2r, pt.x, -p2i * pt.y) * scale;
-  const double pi = fma(p2r, pt.y, p2i * pt.x) * scale;
-  const double ax = A.x, ay = A.y;
-  return make_float2((float)fma(ax, pr, -ay * pi), (float)fma(ax, pi, ay * pr));
+  const double pr = fma(p2r, pt.x, -p2i * pt.y);
+  const double pi = fma(p2r, pt.y, p2i * pt.x);
+  return make_double2(fma(A.x, pr, -A.y * pi), fma(A.x, pi, A.y * pr));
 }
 
 }  // namespace nlse
