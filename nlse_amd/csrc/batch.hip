@@ -46,10 +46,15 @@ struct BatchFlags {
   int timing;  // repeated sweeps: rescale by 1/N per sweep
 };
 
+// Row units of 4096/NX rows are PASSES row_body calls of LPB rows, column
+// units of 8192/NY columns PASSES tiles of WT columns.  The per-length kernels
+// deal out single passes, in blocks of THREADS threads: 256, or 512 for
+// 2048-point columns (tiles of 4 columns, 32-byte row segments, at least).
+// The kernels of all lengths (block sizes BROW_THREADS, BCOL_THREADS) deal out
+// whole units.
 constexpr int BROW_THREADS = 256;
 constexpr int BCOL_THREADS = 512;
 
-// Row units of 4096/NX rows run as PASSES row_body calls of LPB rows.
 template <int N, bool SMALL>
 struct BRow {
   using C = LineCfg<N>;
@@ -57,37 +62,41 @@ struct BRow {
   static constexpr int AR = SMALL ? C::ARS : F64;
   static constexpr int T = N / P;
   static constexpr int LPB = BROW_THREADS / T < 4096 / N ? BROW_THREADS / T : 4096 / N;
-  static constexpr int THREADS = LPB * T;
   static constexpr int PASSES = (4096 / N) / LPB;
   static constexpr int LDSB = row_lds_size<N, LPB, 1>() * (int)sizeof(xchg_t<AR>);
-  static_assert(THREADS == BROW_THREADS, "one block size for every length");
+  static_assert(LPB * T == BROW_THREADS, "one block size for every length");
 };
 
-// Column units of 8192/NY columns run as PASSES tiles of WT columns.
-template <int N, bool SMALL>
+template <int N, bool SMALL, int THREADS = BCOL_THREADS>
 struct BCol {
   using C = LineCfg<N>;
   static constexpr int P = SMALL ? C::PS : C::P;
   static constexpr int AR = SMALL ? C::ARS : F64;
   static constexpr int T = N / P;
   static constexpr int W = 8192 / N;
-  static constexpr int WT = BCOL_THREADS / T < W ? BCOL_THREADS / T : W;
+  static constexpr int WT = THREADS / T < W ? THREADS / T : W;
   static constexpr int PASSES = W / WT;
   static constexpr int LDSB = col_lds_size<N, WT, 1>() * (int)sizeof(xchg_t<AR>);
-  static_assert(WT * T == BCOL_THREADS, "one block size for every length");
+  static_assert(WT * T == THREADS, "whole blocks");
 };
+#ifndef NLSE_BCOL_T
+#define NLSE_BCOL_T 256
+#endif
+constexpr int bcol_threads(int n) { return n >= 2048 ? 512 : NLSE_BCOL_T; }
 
 static bool batch_len_ok(int64_t n) { return n == 128 || n == 256 || n == 512 || n == 1024 || n == 2048; }
+
 // unit groups: line length, small-field plans or not
 static int len_index(int64_t n, bool small) {
   return 2 * (n == 128 ? 0 : n == 256 ? 1 : n == 512 ? 2 : n == 1024 ? 3 : 4) + (small ? 1 : 0);
 }
 constexpr int NLEN = 10;
 
-// One unit of a row or column sweep.  GEN: some member's loss varies from
-// point to point (see nl1_block_I).
+// Pass k of a unit of a row or column sweep.  GEN: some member's loss varies
+// from point to point (see nl1_block_I).
 template <int N, bool SMALL, bool GEN>
-__device__ __forceinline__ void row_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
+__device__ __forceinline__ void row_pass(const BatchInst& I, const BatchUnit& un, int k, const BatchFlags& f,
+                                         void* lds) {
   using B = BRow<N, SMALL>;
   RowArgs a = I.row;
   a.inverse_first = f.inverse_first;
@@ -97,34 +106,17 @@ __device__ __forceinline__ void row_unit(const BatchInst& I, const BatchUnit& un
   a.nlp_a = I.nl[f.slot_a];
   a.nlp_b = I.nl[f.slot_b];
   a.out_scale = f.timing ? I.inv_nx : 1.f;
-#pragma unroll 1
-  for (int k = 0; k < B::PASSES; ++k)
-    row_body<N, B::P, B::LPB, 1, GEN, B::AR>(a, un.first + k * B::LPB, reinterpret_cast<xchg_t<B::AR>*>(lds));
+  row_body<N, B::P, B::LPB, 1, GEN, B::AR>(a, un.first + k * B::LPB, reinterpret_cast<xchg_t<B::AR>*>(lds));
 }
 
-template <int N, bool SMALL>
-__device__ __forceinline__ void col_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
-  using B = BCol<N, SMALL>;
+template <int N, bool SMALL, int THREADS>
+__device__ __forceinline__ void col_pass(const BatchInst& I, const BatchUnit& un, int k, const BatchFlags& f,
+                                         void* lds) {
+  using B = BCol<N, SMALL, THREADS>;
   ColArgs c = I.col;
   if (f.timing) c.scale = I.inv_ny;
-#pragma unroll 1
-  for (int k = 0; k < B::PASSES; ++k)
-    col_body<N, B::P, B::WT, 1, 1, PROP_SEP64, B::AR>(c, un.first * B::PASSES + k,
-                                                      reinterpret_cast<xchg_t<B::AR>*>(lds));
-}
-
-// One persistent kernel per line length: a single length per kernel keeps
-// the register footprint of the plain sweeps (a kernel holding every
-// length spills).
-template <int N, bool SMALL, bool GEN>
-__global__ __launch_bounds__(BROW_THREADS) void k_batch_row(const BatchInst* __restrict__ inst,
-                                                            const BatchUnit* __restrict__ units, int64_t nunits,
-                                                            BatchFlags f) {
-  __shared__ double2 lds[BRow<N, SMALL>::LDSB / 16 + 1];
-  for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
-    const BatchUnit un = units[u];
-    row_unit<N, SMALL, GEN>(inst[un.inst], un, f, lds);
-  }
+  col_body<N, B::P, B::WT, 1, 1, PROP_SEP64, B::AR>(c, un.first * B::PASSES + k,
+                                                    reinterpret_cast<xchg_t<B::AR>*>(lds));
 }
 
 // XCD-aware order: consecutive list entries (neighbouring column tiles,
@@ -134,14 +126,30 @@ __device__ __forceinline__ int64_t xcd_block() {
   return (grid % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (grid / 8) + blockIdx.x / 8 : blockIdx.x;
 }
 
-template <int N, bool SMALL>
-__global__ __launch_bounds__(BCOL_THREADS) void k_batch_col(const BatchInst* __restrict__ inst,
+// One kernel per line length: a single length per kernel keeps the register
+// footprint of the plain sweeps (a kernel holding every length spills).  The
+// blocks stride over the passes of the units.
+template <int N, bool SMALL, bool GEN>
+__global__ __launch_bounds__(BROW_THREADS) void k_batch_row(const BatchInst* __restrict__ inst,
                                                             const BatchUnit* __restrict__ units, int64_t nunits,
                                                             BatchFlags f) {
-  __shared__ double2 lds[BCol<N, SMALL>::LDSB / 16 + 1];
-  for (int64_t u = xcd_block(); u < nunits; u += gridDim.x) {
-    const BatchUnit un = units[u];
-    col_unit<N, SMALL>(inst[un.inst], un, f, lds);
+  using B = BRow<N, SMALL>;
+  __shared__ double2 lds[B::LDSB / 16 + 1];
+  for (int64_t u = blockIdx.x; u < nunits * B::PASSES; u += gridDim.x) {
+    const BatchUnit un = units[u / B::PASSES];
+    row_pass<N, SMALL, GEN>(inst[un.inst], un, (int)(u % B::PASSES), f, lds);
+  }
+}
+
+template <int N, bool SMALL>
+__global__ __launch_bounds__(bcol_threads(N)) void k_batch_col(const BatchInst* __restrict__ inst,
+                                                               const BatchUnit* __restrict__ units, int64_t nunits,
+                                                               BatchFlags f) {
+  using B = BCol<N, SMALL, bcol_threads(N)>;
+  __shared__ double2 lds[B::LDSB / 16 + 1];
+  for (int64_t u = xcd_block(); u < nunits * B::PASSES; u += gridDim.x) {
+    const BatchUnit un = units[u / B::PASSES];
+    col_pass<N, SMALL, bcol_threads(N)>(inst[un.inst], un, (int)(u % B::PASSES), f, lds);
   }
 }
 
@@ -152,15 +160,19 @@ __global__ __launch_bounds__(BCOL_THREADS) void k_batch_col(const BatchInst* __r
 // (which spilled), and the LDS array is the largest length's.
 template <int N, bool SMALL, bool GEN>
 __device__ __noinline__ void batch_row_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
-  row_unit<N, SMALL, GEN>(I, un, f, lds);
+#pragma unroll 1
+  for (int k = 0; k < BRow<N, SMALL>::PASSES; ++k) row_pass<N, SMALL, GEN>(I, un, k, f, lds);
 }
 
 template <int N, bool SMALL>
 __device__ __noinline__ void batch_col_unit(const BatchInst& I, const BatchUnit& un, const BatchFlags& f, void* lds) {
-  col_unit<N, SMALL>(I, un, f, lds);
+#pragma unroll 1
+  for (int k = 0; k < BCol<N, SMALL>::PASSES; ++k) col_pass<N, SMALL, BCOL_THREADS>(I, un, k, f, lds);
 }
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
+template <int N, bool SMALL>
+using BColAll = BCol<N, SMALL, BCOL_THREADS>;
 template <template <int, bool> class B>
 constexpr int lds_all() {
   return cmax(cmax(cmax(B<128, false>::LDSB, B<128, true>::LDSB), cmax(B<256, false>::LDSB, B<256, true>::LDSB)),
@@ -193,7 +205,7 @@ __global__ __launch_bounds__(BROW_THREADS) void k_batch_row_all(const BatchInst*
 __global__ __launch_bounds__(BCOL_THREADS) void k_batch_col_all(const BatchInst* __restrict__ inst,
                                                                 const BatchUnit* __restrict__ units, int64_t nunits,
                                                                 BatchFlags f) {
-  __shared__ double2 lds[lds_all<BCol>() / 16 + 1];
+  __shared__ double2 lds[lds_all<BColAll>() / 16 + 1];
   for (int64_t u = xcd_block(); u < nunits; u += gridDim.x) {
     const BatchUnit un = units[u];
     const BatchInst& I = inst[un.inst];
@@ -269,11 +281,17 @@ static BatchFlags row_flags(int precision, int stage) {
   return f;
 }
 
+// Blocks of a per-length launch: one per pass when the grid covers the units
+// (the default), else the grid given per CU (nlse_batch_set_grid).
+static unsigned pass_grid(int64_t units, int passes, int grid) {
+  return (unsigned)(grid >= units ? units * passes : grid);
+}
+
 template <int N, bool SMALL>
 static void launch_row_n(nlse_batch* b, int li, const BatchFlags& f, hipStream_t s) {
-  const dim3 grid((unsigned)b->row_grid[li]), block(BROW_THREADS);
   const BatchUnit* units = b->d_row + b->row_off[li];
   const int64_t n = b->row_off[li + 1] - b->row_off[li];
+  const dim3 grid(pass_grid(n, BRow<N, SMALL>::PASSES, b->row_grid[li])), block(BROW_THREADS);
   if (b->general)
     hipLaunchKernelGGL((k_batch_row<N, SMALL, true>), grid, block, 0, s, b->d_inst, units, n, f);
   else
@@ -282,8 +300,10 @@ static void launch_row_n(nlse_batch* b, int li, const BatchFlags& f, hipStream_t
 
 template <int N, bool SMALL>
 static void launch_col_n(nlse_batch* b, int li, const BatchFlags& f, hipStream_t s) {
-  hipLaunchKernelGGL((k_batch_col<N, SMALL>), dim3((unsigned)b->col_grid[li]), dim3(BCOL_THREADS), 0, s, b->d_inst,
-                     b->d_col + b->col_off[li], b->col_off[li + 1] - b->col_off[li], f);
+  constexpr int TH = bcol_threads(N);
+  const int64_t n = b->col_off[li + 1] - b->col_off[li];
+  hipLaunchKernelGGL((k_batch_col<N, SMALL>), dim3(pass_grid(n, BCol<N, SMALL, TH>::PASSES, b->col_grid[li])),
+                     dim3(TH), 0, s, b->d_inst, b->d_col + b->col_off[li], n, f);
 }
 
 // One persistent launch per line length present in the batch, or one for
@@ -446,9 +466,9 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
     b->col_off[li] = (int64_t)cols.size();
     rows.insert(rows.end(), rows_n[li].begin(), rows_n[li].end());
     cols.insert(cols.end(), cols_n[li].begin(), cols_n[li].end());
-    // persistent grids: 8 row blocks and 2 column blocks per CU
-    b->row_grid[li] = (int)std::min<int64_t>((int64_t)rows_n[li].size(), (int64_t)ncu * 8);
-    b->col_grid[li] = (int)std::min<int64_t>((int64_t)cols_n[li].size(), (int64_t)ncu * 2);
+    // a block per pass
+    b->row_grid[li] = (int)rows_n[li].size();
+    b->col_grid[li] = (int)cols_n[li].size();
   }
   b->row_off[NLEN] = (int64_t)rows.size();
   b->col_off[NLEN] = (int64_t)cols.size();
