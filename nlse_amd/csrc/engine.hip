@@ -938,7 +938,7 @@ int nlse_plan_create(const nlse_plan_desc* d, nlse_plan** out) {
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
         cus = 256;
       const int64_t t = d->ny / (p->small ? p->cops->p_col_small : p->cops->p_col);
-      want = 8;
+      want = p->cops->colw(d->nx, 0, p->small);
       for (; want > 1; want >>= 1) {
         const int64_t blocks = d->items * d->ncomp * (d->nx / want);
         if (blocks >= cus || (2 * blocks >= cus && want * t <= 256)) break;

@@ -354,9 +354,32 @@ struct LdsLine {
 template <int PADSH>
 __host__ __device__ __forceinline__ constexpr int lds_pad(int i) { return i + (i >> PADSH); }
 
+// Ratio twiddles {cos, tan} of the factored butterflies (dft_fma): R/2 entries
+// per stage of radix R and index jm, the stages of P = 16, 8 and 4 one after the
+// other, behind the other two tables.
+__host__ __device__ constexpr int rt_offset(int n, int p, int stage) {
+  const int logn = ilog2c(n), logp = ilog2c(p), rem = logn % logp;
+  int off = 0, ns = rem ? (1 << rem) : p;
+  for (int i = 1; i < stage; ++i) {
+    off += p / 2 * ns;
+    ns *= p;
+  }
+  return off;
+}
+__host__ __device__ constexpr int rt_size_np(int n, int p) {
+  if (p > n) return 0;
+  const int logn = ilog2c(n), logp = ilog2c(p);
+  return rt_offset(n, p, logn / logp + (logn % logp ? 1 : 0));
+}
+__host__ __device__ constexpr int rt_base(int n, int p) {
+  return (p < 16 ? rt_size_np(n, 16) : 0) + (p < 8 ? rt_size_np(n, 8) : 0);
+}
+__host__ __device__ constexpr int rt_size(int n) { return rt_size_np(n, 16) + rt_size_np(n, 8) + rt_size_np(n, 4); }
+
 // Twiddle table of a line length: the FP64 records {c, s} of every stage
 // table (tw_union_size(n) entries), followed by the same records as
-// compensated FP32 {c_hi, s_hi, c_lo, s_lo} for the FP32 transforms.
+// compensated FP32 {c_hi, s_hi, c_lo, s_lo} for the FP32 transforms, followed
+// by the ratio twiddles.
 __host__ __device__ constexpr int tw_f32_offset(int n) { return tw_union_size(n) > 0 ? tw_union_size(n) : 1; }
 
 // Arithmetic of a transform.  F64: butterflies and twiddles in FP64, one
@@ -397,98 +420,84 @@ __device__ __forceinline__ C from_f64(double2 a) {
   else return a;
 }
 
-// The FP64 twiddles of a thread's stages: two powers of w = exp(-2 pi i jm /
-// (Ns R)) per twiddled stage, w and w^2 (radix 4) or w and w^4 (radix 8, 16);
-// the others are products of these (3 for radix 16's factored form, 5 for
-// radix 8, 1 for radix 4).  They are loaded once, beside the field, and serve
-// every transform of the kernel: 15 table loads per radix-16 stage kept the
-// vector L1 as busy as the VALU (11.6 us each of a 28 us 2048^2 column
-// sweep), and loads issued at each stage exposed their latency.
-template <int N, int P>
-struct Twid {
-  static constexpr int NT = Plan<N, P>::NSTAGES > 1 ? Plan<N, P>::NSTAGES - 1 : 1;
-  double2 w[NT][2];
-};
-
-// Forward radix-R butterfly in FP64: inputs ld(k) times w^k (TW; w1, wq: the
-// powers Twid holds), outputs st(k, x).  Radix 16 runs as 4 x 4, w^(4 n1 + n2)
-// applied as w^(4 n1) before the first layer and w^n2 after it, which keeps
-// the live set near the 16 FP64 points.
-template <int R, bool TW, class Load, class Store>
-__device__ __forceinline__ void dft_io(Load ld, double2 w1, double2 wq, Store st) {
-  if constexpr (R == 16) {
-    double2 y[16];
-    double2 w2, w3, w8, w12;
-    if constexpr (TW) {
-      w8 = cmul_tw(wq, wq);
-      w12 = cmul_tw(w8, wq);
-      w2 = cmul_tw(w1, w1);
-      w3 = cmul_tw(w2, w1);
-    }
-#pragma unroll
-    for (int n2 = 0; n2 < 4; ++n2) {
-      double2 a = ld(n2), b = ld(4 + n2), c = ld(8 + n2), d = ld(12 + n2);
-      if constexpr (TW) {
-        b = cmul_tw(b, wq);
-        c = cmul_tw(c, w8);
-        d = cmul_tw(d, w12);
-      }
-      dft4(a, b, c, d);
-      if constexpr (TW) {
-        if (n2 > 0) {
-          const double2 w = n2 == 1 ? w1 : n2 == 2 ? w2 : w3;
-          a = cmul_tw(a, w);
-          b = cmul_tw(b, w);
-          c = cmul_tw(c, w);
-          d = cmul_tw(d, w);
-        }
-      }
-      // W16^(n2 k1)
-      if (n2 == 1) { b = rot(b, K_C8, K_S8); c = mul_w8_1(c); d = rot(d, K_S8, K_C8); }
-      if (n2 == 2) { b = mul_w8_1(b); c = mul_mi(c); d = mul_w8_3(d); }
-      if (n2 == 3) { b = rot(b, K_S8, K_C8); c = mul_w8_3(c); d = rot(d, -K_C8, -K_S8); }
-      y[n2 * 4 + 0] = a; y[n2 * 4 + 1] = b; y[n2 * 4 + 2] = c; y[n2 * 4 + 3] = d;
-    }
-#pragma unroll
-    for (int k1 = 0; k1 < 4; ++k1) {
-      dft4(y[k1], y[4 + k1], y[8 + k1], y[12 + k1]);
-      st(k1, y[k1]);
-      st(k1 + 4, y[4 + k1]);
-      st(k1 + 8, y[8 + k1]);
-      st(k1 + 12, y[12 + k1]);
-    }
+// Radix-R butterfly in FP64 as log2 R layers of radix-2 ones: X[k] = E[k] +
+// w W_R^k O[k], X[k + R/2] = E[k] - w W_R^k O[k] with E, O the transforms of
+// the even and odd points for w^2.  A twiddle c + i s is applied as c (1 + i
+// s/c), the c inside the additions: a butterfly is 6 FMAs where a complex
+// product and two additions are 8, twiddles included: 12 operations per point
+// of a twiddled radix-16 stage against 17 of the factored 4 x 4 form (VALU
+// issue is what bounds the sweeps of large fields).  The R/2 pairs {c, s/c} of
+// a stage: w W_R^k for k < R/4 (the others are -i times these), then the same
+// for w^2 and R/2, and so on.  Where c is nearly zero s/c is as large and the
+// product keeps its relative precision; c is never exactly zero (the table
+// holds cos(pi/2) as the FP64 cosine, 6e-17).
+__device__ __forceinline__ void bf2(double2 e, double2 o, double2 ct, bool mi, double2& x0, double2& x1) {
+  const double vr = fma(-ct.y, o.y, o.x), vi = fma(ct.y, o.x, o.y);
+  if (!mi) {
+    x0 = make_double2(fma(ct.x, vr, e.x), fma(ct.x, vi, e.y));
+    x1 = make_double2(fma(-ct.x, vr, e.x), fma(-ct.x, vi, e.y));
   } else {
-    double2 x[R], w[8];
-    if constexpr (TW) {
-      w[1] = w1;
-      if constexpr (R == 4) {
-        w[2] = wq;
-        w[3] = cmul_tw(w1, wq);
-      } else if constexpr (R == 8) {
-        w[4] = wq;
-        w[2] = cmul_tw(w1, w1);
-        w[3] = cmul_tw(w[2], w1);
-        w[5] = cmul_tw(wq, w1);
-        w[6] = cmul_tw(wq, w[2]);
-        w[7] = cmul_tw(wq, w[3]);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      x[k] = ld(k);
-      if (TW && k > 0) x[k] = cmul_tw(x[k], w[k]);
-    }
-    dft<R>(x);
-#pragma unroll
-    for (int k = 0; k < R; ++k) st(k, x[k]);
+    x0 = make_double2(fma(ct.x, vi, e.x), fma(-ct.x, vr, e.y));
+    x1 = make_double2(fma(-ct.x, vi, e.x), fma(ct.x, vr, e.y));
+  }
+}
+__device__ __forceinline__ void bf2(double2 e, double2 o, bool mi, double2& x0, double2& x1) {
+  if (mi) o = mul_mi(o);
+  x0 = cadd(e, o);
+  x1 = csub(e, o);
+}
+
+// {cos, tan} of -2 pi k / R, k < R/4
+template <int R, int K>
+constexpr double2 const_ct() {
+  static_assert(K > 0 && K < R / 4 && R <= 16, "W8, W16, W16^3");
+  constexpr double c = R == 8 || K == 2 ? K_R2 : (K == 1 ? K_C8 : K_S8);
+  constexpr double s = R == 8 || K == 2 ? -K_R2 : (K == 1 ? -K_S8 : -K_C8);
+  return double2{c, s / c};
+}
+
+template <int R, bool TW, int K = 0>
+__device__ __forceinline__ void dft_top(const double2* E, const double2* O, const double2* ct, double2* X) {
+  if constexpr (K < R / 2) {
+    constexpr int Q = R / 4;
+    constexpr bool MI = R >= 4 && K >= Q;
+    constexpr int KK = MI ? K - Q : K;
+    if constexpr (TW) bf2(E[K], O[K], ct[KK], MI, X[K], X[K + R / 2]);
+    else if constexpr (KK == 0) bf2(E[K], O[K], MI, X[K], X[K + R / 2]);
+    else bf2(E[K], O[K], const_ct<R, KK>(), MI, X[K], X[K + R / 2]);
+    dft_top<R, TW, K + 1>(E, O, ct, X);
   }
 }
 
-// Byte offset of stage S in the twiddle table (FP64 and FP32 records have the
-// same size).
+// points z(n) = ld(START + n * STEP), n < R
+template <int R, bool TW, int START, int STEP, class Load>
+__device__ __forceinline__ void dft_fma(Load ld, const double2* ct, double2* X) {
+  if constexpr (R == 1) {
+    X[0] = ld(START);
+  } else {
+    double2 E[R / 2], O[R / 2];
+    constexpr int Q = R >= 4 ? R / 4 : 1;
+    dft_fma<R / 2, TW, START, 2 * STEP>(ld, ct + Q, E);
+    dft_fma<R / 2, TW, START + STEP, 2 * STEP>(ld, ct + Q, O);
+    dft_top<R, TW>(E, O, ct, X);
+  }
+}
+
+// The twiddles of a thread's stages, loaded once beside the field where P < 16
+// (loads at each stage would expose their latency in the small fields these
+// sets serve); at P = 16 they would take the registers of a wave, and each
+// stage loads its own.
+template <int N, int P>
+struct Twid {
+  static constexpr int NT = P < 16 && Plan<N, P>::NSTAGES > 1 ? Plan<N, P>::NSTAGES - 1 : 1;
+  double2 ct[NT][P / 2 > 0 ? P / 2 : 1];
+};
+
+// Byte offset of stage S's twiddles: ratio pairs, or compensated FP32 records.
 template <int N, int P, int S, int AR>
 constexpr uint32_t stage_twiddles() {
-  return 16u * (uint32_t)((AR != F32C ? 0 : tw_f32_offset(N)) + tw_base(N, P) + Plan<N, P>::tw_offset(S));
+  return AR == F32C ? 16u * (uint32_t)(tw_f32_offset(N) + tw_base(N, P) + Plan<N, P>::tw_offset(S))
+                    : 16u * (uint32_t)(2 * tw_f32_offset(N) + rt_base(N, P) + rt_offset(N, P, S));
 }
 
 // A value the compiler cannot see through: what is computed from it is
@@ -499,16 +508,19 @@ __device__ __forceinline__ uint32_t opaque(uint32_t x) {
   return x;
 }
 
+template <int N, int P, int S>
+__device__ __forceinline__ void load_stage_twiddles(double2 (&ct)[P / 2 > 0 ? P / 2 : 1], const Buf& tw, uint32_t jm) {
+  constexpr int NS = Plan<N, P>::ns(S);
+#pragma unroll
+  for (int i = 0; i < P / 2; ++i) ct[i] = tw.load<double2>(16u * jm, stage_twiddles<N, P, S, F64>() + 16u * i * NS);
+}
+
 template <int N, int P, int S = 1>
 __device__ __forceinline__ void load_twiddles_from(Twid<N, P>& W, const Buf& tw, int t) {
   using PL = Plan<N, P>;
   if constexpr (S < PL::NSTAGES) {
-    constexpr int NS = PL::ns(S);
     static_assert(PL::radix(S) == P, "only the first stage has another radix, and no twiddles");
-    constexpr uint32_t TW0 = stage_twiddles<N, P, S, F64>();
-    const uint32_t o = 16u * (uint32_t)(t & (NS - 1));
-    W.w[S - 1][0] = tw.load<double2>(o, TW0);
-    W.w[S - 1][1] = tw.load<double2>(o, TW0 + 16u * (uint32_t)(((P == 4 ? 2 : 4) - 1) * NS));
+    load_stage_twiddles<N, P, S>(W.ct[S - 1], tw, (uint32_t)(t & (PL::ns(S) - 1)));
     load_twiddles_from<N, P, S + 1>(W, tw, t);
   }
 }
@@ -560,16 +572,18 @@ __device__ __forceinline__ void fft_stage(CI (&v)[G][P], CO (&w)[G][P], int t, c
             if constexpr (LAST) w[g][b + k * NB] = from_f64<CO>(x);
             else out[lds_pad<PADSH>(k * NS)] = from_f64<xchg_t<AR>>(x);
           };
-          double2 w1{}, wq{};
-          if constexpr (NS > 1 && P == 16) {
-            const uint32_t o = 16u * opaque((uint32_t)jm);
-            w1 = tw.load<double2>(o, TW0);
-            wq = tw.load<double2>(o, TW0 + 16u * 3u * NS);
-          } else if constexpr (NS > 1) {
-            w1 = W.w[S - 1][0];
-            wq = W.w[S - 1][1];
+          double2 X[R];
+          if constexpr (NS == 1) {
+            dft_fma<R, false, 0, 1>(ld, (const double2*)nullptr, X);
+          } else if constexpr (P == 16) {
+            double2 ct[P / 2];
+            load_stage_twiddles<N, P, S>(ct, tw, opaque((uint32_t)jm));
+            dft_fma<R, true, 0, 1>(ld, ct, X);
+          } else {
+            dft_fma<R, true, 0, 1>(ld, W.ct[S - 1], X);
           }
-          dft_io<R, (NS > 1)>(ld, w1, wq, st);
+#pragma unroll
+          for (int k = 0; k < R; ++k) st(k, X[k]);
         } else {
           float2 y[R];
 #pragma unroll

@@ -246,12 +246,16 @@ __device__ __forceinline__ void col_prop(const ColArgs& a, prop_t<KIND> (&w)[G][
     const Buf pyb(a.py + comp * N);
     double2 px[G];
 #pragma unroll
-    for (int g = 0; g < G; ++g) px[g] = a.px[comp * a.NX + c0 + g * CS];
+    for (int g = 0; g < G; ++g) {
+      px[g] = a.px[comp * a.NX + c0 + g * CS];
+      px[g].x *= (double)a.scale;
+      px[g].y *= (double)a.scale;
+    }
 #pragma unroll
     for (int m = 0; m < P; ++m) {
       const double2 py = pyb.load<double2>(16u * t, 16u * m * T);
 #pragma unroll
-      for (int g = 0; g < G; ++g) w[g][m] = prop_sep_c64(w[g][m], px[g], py, a.scale);
+      for (int g = 0; g < G; ++g) w[g][m] = prop_sep_c64(w[g][m], px[g], py);
     }
   } else if constexpr (KIND == PROP_SEP3D) {
     // column c = x*NT + t of an (NY, NX, NT) field: complex64(px*py)

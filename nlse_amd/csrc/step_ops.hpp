@@ -374,16 +374,15 @@ __device__ __forceinline__ void rabi(float2& A1, float2& A2, const RabiParams& r
 
 // A_c64 * P where P is the complex64 rounding of the FP64 product px*py
 // (the reference builds exp(-i(kx^2+ky^2) dz/2k) in FP64 and casts it to
-// complex64, nlse.py:194-197).  `scale` is an exact power of two (1/N).  The
-// product is a complex64 one, as the reference's: its FP32 roundings are not
-// free of bias (-2.8e-9 of the power per step in the speckle workload), and
-// an FP64 product, nearer to the exact result, would leave the complex64
+// complex64, nlse.py:194-197); px carries the factor 1/N, an exact power of
+// two.  The product is a complex64 one, as the reference's: its FP32 roundings
+// are not free of bias (-2.8e-9 of the power per step in the speckle workload),
+// and an FP64 product, nearer to the exact result, would leave the complex64
 // reference by 5e-6 of the power over 2001 steps.
-__device__ __forceinline__ float2 prop_sep_c64(float2 A, double2 px, double2 py, float scale) {
-  const double pr = fma(px.x, py.x, -px.y * py.y);
-  const double pi = fma(px.x, py.y, px.y * py.x);
-  const float2 P = make_float2((float)pr * scale, (float)pi * scale);
-  return make_float2(fmaf(A.x, P.x, -A.y * P.y), fmaf(A.x, P.y, A.y * P.x));
+__device__ __forceinline__ float2 prop_sep_c64(float2 A, double2 px, double2 py) {
+  const float pr = (float)fma(px.x, py.x, -px.y * py.y);
+  const float pi = (float)fma(px.x, py.y, px.y * py.x);
+  return make_float2(fmaf(A.x, pr, -A.y * pi), fmaf(A.x, pi, A.y * pr));
 }
 
 __device__ __forceinline__ float2 prop_c64(float2 A, float2 P, float scale) {
