@@ -1540,6 +1540,7 @@ static NlcArgs plan_nlc_args(const nlse_plan* p, void* A) {
   a.direct = n.direct ? 1 : 0;
   a.full = n.full ? 1 : 0;
   a.general = nl_general(p);
+  a.through = p->through;
   return a;
 }
 
@@ -1593,6 +1594,7 @@ static ColArgs nlc_col_args(const nlse_plan* p) {
   c.do_fwd = c.do_prop = c.do_inv = 1;
   c.pkind = PROP_KREAL;
   c.kq = p->nlc.kq;
+  c.through = p->through;
   return c;
 }
 

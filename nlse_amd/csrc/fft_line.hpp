@@ -44,109 +44,6 @@ __device__ __forceinline__ float2 conjf2(float2 a) { return make_float2(a.x, -a.
 // a * (-i)
 __device__ __forceinline__ float2 mul_mi(float2 a) { return make_float2(a.y, -a.x); }
 
-// ---------------------------------------------- compensated FP32 arithmetic
-// (transforms of intensities: see fft_line)
-// Split constants: value = HI + LO to ~2^-48 relative.
-#define NLSE_SPLIT(name, val)                                  \
-  constexpr float name##_HI = (float)(val);                    \
-  constexpr float name##_LO = (float)((val) - (double)(float)(val));
-NLSE_SPLIT(R2, 0.70710678118654752440084436210484904)   // 1/sqrt(2)
-NLSE_SPLIT(C8, 0.92387953251128675612818318939678829)   // cos(pi/8)
-NLSE_SPLIT(S8, 0.38268343236508977172845998403039887)   // sin(pi/8)
-#undef NLSE_SPLIT
-
-// x * c for a split constant, one rounding of a data-dependent value.
-#define NLSE_CMUL_S(x, name) fmaf((x), name##_HI, (x) * name##_LO)
-
-// a * (c - i s) with split c, s: (a.x c + a.y s) + i (a.y c - a.x s)
-#define NLSE_ROT(a, C, S)                                                          \
-  make_float2(fmaf((a).x, C##_HI, fmaf((a).y, S##_HI, fmaf((a).x, C##_LO, (a).y * S##_LO))), \
-              fmaf((a).y, C##_HI, fmaf(-(a).x, S##_HI, fmaf((a).y, C##_LO, -(a).x * S##_LO))))
-
-// a * w for a stage twiddle w = (c_hi + c_lo) + i (s_hi + s_lo),
-// tw = {c_hi, s_hi, c_lo, s_lo}.  The lo terms enter the FMA chain before
-// the final rounding: a correction applied after rounding (e.g. a
-// magnitude factor 1 + 1e-8) would be lost below half an ulp.
-__device__ __forceinline__ float2 cmul_tw(float2 a, float4 w) {
-  return make_float2(fmaf(a.x, w.x, fmaf(-a.y, w.y, fmaf(a.x, w.z, -a.y * w.w))),
-                     fmaf(a.x, w.y, fmaf(a.y, w.x, fmaf(a.x, w.w, a.y * w.z))));
-}
-
-// a * W8^1 = a * (1 - i)/sqrt2
-__device__ __forceinline__ float2 mul_w8_1(float2 a) {
-  return make_float2(NLSE_CMUL_S(a.x + a.y, R2), NLSE_CMUL_S(a.y - a.x, R2));
-}
-// a * W8^3 = a * (-1 - i)/sqrt2
-__device__ __forceinline__ float2 mul_w8_3(float2 a) {
-  return make_float2(NLSE_CMUL_S(a.y - a.x, R2), NLSE_CMUL_S(-(a.x + a.y), R2));
-}
-
-// ---------------------------------------------------------- butterflies
-// Forward DFTs (kernel exp(-2 pi i n k / R)), in place on x[0..R-1].
-__device__ __forceinline__ void dft2(float2* x) {
-  float2 a = x[0], b = x[1];
-  x[0] = cadd(a, b);
-  x[1] = csub(a, b);
-}
-
-__device__ __forceinline__ void dft4(float2& a, float2& b, float2& c, float2& d) {
-  float2 t0 = cadd(a, c), t1 = csub(a, c), t2 = cadd(b, d), t3 = mul_mi(csub(b, d));
-  a = cadd(t0, t2);  // X0
-  c = csub(t0, t2);  // X2
-  b = cadd(t1, t3);  // X1
-  d = csub(t1, t3);  // X3
-}
-
-__device__ __forceinline__ void dft4(float2* x) { dft4(x[0], x[1], x[2], x[3]); }
-
-__device__ __forceinline__ void dft8(float2* x) {
-  // n = 2 n1 + n2, k = k1 + 4 k2
-  float2 e0 = x[0], e1 = x[2], e2 = x[4], e3 = x[6];
-  float2 o0 = x[1], o1 = x[3], o2 = x[5], o3 = x[7];
-  dft4(e0, e1, e2, e3);
-  dft4(o0, o1, o2, o3);
-  o1 = mul_w8_1(o1);
-  o2 = mul_mi(o2);
-  o3 = mul_w8_3(o3);
-  x[0] = cadd(e0, o0); x[4] = csub(e0, o0);
-  x[1] = cadd(e1, o1); x[5] = csub(e1, o1);
-  x[2] = cadd(e2, o2); x[6] = csub(e2, o2);
-  x[3] = cadd(e3, o3); x[7] = csub(e3, o3);
-}
-
-__device__ __forceinline__ void dft16(float2* x) {
-  // n = 4 n1 + n2, k = k1 + 4 k2: radix-4 over n1, twiddle W16^(n2 k1),
-  // radix-4 over n2.
-  float2 y[16];
-#pragma unroll
-  for (int n2 = 0; n2 < 4; ++n2) {
-    float2 a = x[n2], b = x[4 + n2], c = x[8 + n2], d = x[12 + n2];
-    dft4(a, b, c, d);
-    y[n2 * 4 + 0] = a; y[n2 * 4 + 1] = b; y[n2 * 4 + 2] = c; y[n2 * 4 + 3] = d;
-  }
-  // W16^1 = c8 - i s8, W16^2 = W8^1, W16^3 = s8 - i c8,
-  // W16^4 = -i, W16^6 = W8^3, W16^9 = -c8 + i s8 = -(W16^1)
-  y[1 * 4 + 1] = NLSE_ROT(y[5], C8, S8);
-  y[1 * 4 + 2] = mul_w8_1(y[6]);
-  y[1 * 4 + 3] = NLSE_ROT(y[7], S8, C8);
-  y[2 * 4 + 1] = mul_w8_1(y[9]);
-  y[2 * 4 + 2] = mul_mi(y[10]);
-  y[2 * 4 + 3] = mul_w8_3(y[11]);
-  y[3 * 4 + 1] = NLSE_ROT(y[13], S8, C8);
-  y[3 * 4 + 2] = mul_w8_3(y[14]);
-  {
-    float2 r = NLSE_ROT(y[15], C8, S8);
-    y[15] = make_float2(-r.x, -r.y);
-  }
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) {
-    float2 a = y[0 * 4 + k1], b = y[1 * 4 + k1], c = y[2 * 4 + k1], d = y[3 * 4 + k1];
-    dft4(a, b, c, d);
-    x[k1] = a; x[k1 + 4] = b; x[k1 + 8] = c; x[k1 + 12] = d;
-  }
-}
-
-
 // FP64 butterfly arithmetic
 __device__ __forceinline__ double2 to_f64(float2 a) { return make_double2((double)a.x, (double)a.y); }
 __device__ __forceinline__ float2 to_f32(double2 a) { return make_float2((float)a.x, (float)a.y); }
@@ -356,7 +253,7 @@ __host__ __device__ __forceinline__ constexpr int lds_pad(int i) { return i + (i
 
 // Ratio twiddles {cos, tan} of the factored butterflies (dft_fma): R/2 entries
 // per stage of radix R and index jm, the stages of P = 16, 8 and 4 one after the
-// other, behind the other two tables.
+// other, behind the other table.
 __host__ __device__ constexpr int rt_offset(int n, int p, int stage) {
   const int logn = ilog2c(n), logp = ilog2c(p), rem = logn % logp;
   int off = 0, ns = rem ? (1 << rem) : p;
@@ -377,22 +274,14 @@ __host__ __device__ constexpr int rt_base(int n, int p) {
 __host__ __device__ constexpr int rt_size(int n) { return rt_size_np(n, 16) + rt_size_np(n, 8) + rt_size_np(n, 4); }
 
 // Twiddle table of a line length: the FP64 records {c, s} of every stage
-// table (tw_union_size(n) entries), followed by the same records as
-// compensated FP32 {c_hi, s_hi, c_lo, s_lo} for the FP32 transforms, followed
+// table (tw_union_size(n) entries; the complex128 kernels' twiddles), followed
 // by the ratio twiddles.
-__host__ __device__ constexpr int tw_f32_offset(int n) { return tw_union_size(n) > 0 ? tw_union_size(n) : 1; }
+__host__ __device__ constexpr int rt_begin(int n) { return tw_union_size(n) > 0 ? tw_union_size(n) : 1; }
 
-// Arithmetic of a transform.  F64: butterflies and twiddles in FP64, one
-// complex64 rounding per stage (the field's transforms, whose rounding noise
-// a long run accumulates).  F32C: compensated FP32 (hi+lo constants and
-// twiddles, one rounding per butterfly level): the transforms of the
-// nonlocal response's intensities, whose noise enters only the nonlinear
-// phase through the convolved intensity, while a gain bias would not (it
-// multiplies the whole nonlinear phase of the run) -- compensation keeps
-// the gain unbiased at about half the FP64 cost.
-// F64X: FP64 as F64, and the exchanges carry FP64 too: one rounding per
-// transform and no conversions between stages, for twice the LDS traffic.
-enum FftArith : int { F64 = 0, F32C = 1, F64X = 2 };
+// Precision of a transform's exchanges: F64 rounds to complex64 once per stage,
+// F64X carries FP64: one rounding per transform and no conversions between
+// stages, for twice the LDS traffic.  Butterflies are FP64 in both.
+enum FftArith : int { F64 = 0, F64X = 1 };
 
 template <int AR>
 using xchg_t = typename std::conditional<AR == F64X, double2, float2>::type;
@@ -483,21 +372,23 @@ __device__ __forceinline__ void dft_fma(Load ld, const double2* ct, double2* X) 
   }
 }
 
-// The twiddles of a thread's stages, loaded once beside the field where P < 16
-// (loads at each stage would expose their latency in the small fields these
-// sets serve); at P = 16 they would take the registers of a wave, and each
-// stage loads its own.
-template <int N, int P>
+// The twiddles of a thread's stages, loaded once beside the field for lines of
+// up to 512 points with less than 16 per thread (loads at each stage would
+// expose their latency in the small fields these sets serve); else they would
+// take the registers of a wave (16 per stage at P = 8), and each stage loads
+// its own.
+constexpr bool twid_kept(int n, int p) { return p < 16 && n <= 512; }
+
+template <int N, int P, bool KEEP = twid_kept(N, P)>
 struct Twid {
-  static constexpr int NT = P < 16 && Plan<N, P>::NSTAGES > 1 ? Plan<N, P>::NSTAGES - 1 : 1;
+  static constexpr int NT = KEEP && Plan<N, P>::NSTAGES > 1 ? Plan<N, P>::NSTAGES - 1 : 1;
   double2 ct[NT][P / 2 > 0 ? P / 2 : 1];
 };
 
-// Byte offset of stage S's twiddles: ratio pairs, or compensated FP32 records.
-template <int N, int P, int S, int AR>
+// Byte offset of stage S's ratio pairs.
+template <int N, int P, int S>
 constexpr uint32_t stage_twiddles() {
-  return AR == F32C ? 16u * (uint32_t)(tw_f32_offset(N) + tw_base(N, P) + Plan<N, P>::tw_offset(S))
-                    : 16u * (uint32_t)(2 * tw_f32_offset(N) + rt_base(N, P) + rt_offset(N, P, S));
+  return 16u * (uint32_t)(rt_begin(N) + rt_base(N, P) + rt_offset(N, P, S));
 }
 
 // A value the compiler cannot see through: what is computed from it is
@@ -512,23 +403,23 @@ template <int N, int P, int S>
 __device__ __forceinline__ void load_stage_twiddles(double2 (&ct)[P / 2 > 0 ? P / 2 : 1], const Buf& tw, uint32_t jm) {
   constexpr int NS = Plan<N, P>::ns(S);
 #pragma unroll
-  for (int i = 0; i < P / 2; ++i) ct[i] = tw.load<double2>(16u * jm, stage_twiddles<N, P, S, F64>() + 16u * i * NS);
+  for (int i = 0; i < P / 2; ++i) ct[i] = tw.load<double2>(16u * jm, stage_twiddles<N, P, S>() + 16u * i * NS);
 }
 
-template <int N, int P, int S = 1>
-__device__ __forceinline__ void load_twiddles_from(Twid<N, P>& W, const Buf& tw, int t) {
+template <int N, int P, bool KEEP, int S = 1>
+__device__ __forceinline__ void load_twiddles_from(Twid<N, P, KEEP>& W, const Buf& tw, int t) {
   using PL = Plan<N, P>;
   if constexpr (S < PL::NSTAGES) {
     static_assert(PL::radix(S) == P, "only the first stage has another radix, and no twiddles");
     load_stage_twiddles<N, P, S>(W.ct[S - 1], tw, (uint32_t)(t & (PL::ns(S) - 1)));
-    load_twiddles_from<N, P, S + 1>(W, tw, t);
+    load_twiddles_from<N, P, KEEP, S + 1>(W, tw, t);
   }
 }
 
-template <int N, int P>
-__device__ __forceinline__ Twid<N, P> load_twiddles(const Buf& tw, int t) {
-  Twid<N, P> W;
-  if constexpr (Plan<N, P>::NSTAGES > 1 && P >= 4 && P < 16) load_twiddles_from<N, P>(W, tw, t);
+template <int N, int P, bool KEEP = twid_kept(N, P)>
+__device__ __forceinline__ Twid<N, P, KEEP> load_twiddles(const Buf& tw, int t) {
+  Twid<N, P, KEEP> W;
+  if constexpr (Plan<N, P>::NSTAGES > 1 && P >= 4 && KEEP) load_twiddles_from<N, P, KEEP>(W, tw, t);
   return W;
 }
 
@@ -537,8 +428,8 @@ __device__ __forceinline__ Twid<N, P> load_twiddles(const Buf& tw, int t) {
 // through LDS in rounds of GR lines (the LDS region holds GR lines per thread
 // column: line g of round r lives at slot g - r*GR); the last stage (Ns = N/R)
 // lands on the natural set.
-template <int N, int P, int S, int G, int GR, int PADSH, int AR, int SYNC, typename CI, typename CO>
-__device__ __forceinline__ void fft_stage(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+template <int N, int P, int S, int G, int GR, int PADSH, int AR, int SYNC, bool KEEP, typename CI, typename CO>
+__device__ __forceinline__ void fft_stage(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P, KEEP>& W, const Buf& tw,
                                           xchg_t<AR>* lds, int lds_stride) {
   using PL = Plan<N, P>;
   constexpr int R = PL::radix(S);
@@ -549,7 +440,6 @@ __device__ __forceinline__ void fft_stage(CI (&v)[G][P], CO (&w)[G][P], int t, c
   static_assert(G % GR == 0, "lines per round must divide the lines per thread");
   // T a multiple of the padding period: no carry in lds_pad(t + m T)
   constexpr bool LDS_STEP = T % (1 << PADSH) == 0;
-  constexpr uint32_t TW0 = stage_twiddles<N, P, S, AR>();
 #pragma unroll
   for (int r = 0; r < G / GR; ++r) {
     if constexpr (!LAST) line_sync<SYNC>();  // the exchange before this one has been read
@@ -566,39 +456,23 @@ __device__ __forceinline__ void fft_stage(CI (&v)[G][P], CO (&w)[G][P], int t, c
         // or base mod NS R = jm < NS, or R divides 2^PADSH), so one address
         // serves all outputs through instruction offsets
         xchg_t<AR>* out = lds + gg * lds_stride + lds_pad<PADSH>((j / NS) * NS * R + jm);
-        if constexpr (AR != F32C) {
-          auto ld = [&](int k) { return to_f64(v[g][b + k * NB]); };
-          auto st = [&](int k, double2 x) {
-            if constexpr (LAST) w[g][b + k * NB] = from_f64<CO>(x);
-            else out[lds_pad<PADSH>(k * NS)] = from_f64<xchg_t<AR>>(x);
-          };
-          double2 X[R];
-          if constexpr (NS == 1) {
-            dft_fma<R, false, 0, 1>(ld, (const double2*)nullptr, X);
-          } else if constexpr (P == 16) {
-            double2 ct[P / 2];
-            load_stage_twiddles<N, P, S>(ct, tw, opaque((uint32_t)jm));
-            dft_fma<R, true, 0, 1>(ld, ct, X);
-          } else {
-            dft_fma<R, true, 0, 1>(ld, W.ct[S - 1], X);
-          }
-#pragma unroll
-          for (int k = 0; k < R; ++k) st(k, X[k]);
+        auto ld = [&](int k) { return to_f64(v[g][b + k * NB]); };
+        auto st = [&](int k, double2 x) {
+          if constexpr (LAST) w[g][b + k * NB] = from_f64<CO>(x);
+          else out[lds_pad<PADSH>(k * NS)] = from_f64<xchg_t<AR>>(x);
+        };
+        double2 X[R];
+        if constexpr (NS == 1) {
+          dft_fma<R, false, 0, 1>(ld, (const double2*)nullptr, X);
+        } else if constexpr (!KEEP) {
+          double2 ct[P / 2];
+          load_stage_twiddles<N, P, S>(ct, tw, opaque((uint32_t)jm));
+          dft_fma<R, true, 0, 1>(ld, ct, X);
         } else {
-          float2 y[R];
-#pragma unroll
-          for (int k = 0; k < R; ++k) {
-            y[k] = v[g][b + k * NB];
-            if (NS > 1 && k > 0)
-              y[k] = cmul_tw(y[k], tw.load<float4>(16u * (uint32_t)jm, TW0 + 16u * (uint32_t)((k - 1) * NS)));
-          }
-          dft<R>(y);
-#pragma unroll
-          for (int k = 0; k < R; ++k) {
-            if constexpr (LAST) w[g][b + k * NB] = y[k];
-            else out[lds_pad<PADSH>(k * NS)] = y[k];
-          }
+          dft_fma<R, true, 0, 1>(ld, W.ct[S - 1], X);
         }
+#pragma unroll
+        for (int k = 0; k < R; ++k) st(k, X[k]);
       }
     }
     if constexpr (!LAST) {
@@ -613,8 +487,8 @@ __device__ __forceinline__ void fft_stage(CI (&v)[G][P], CO (&w)[G][P], int t, c
   }
 }
 
-template <int N, int P, int S, int G, int GR, int PADSH, int AR, int SYNC, typename CI, typename CO>
-__device__ __forceinline__ void fft_stages_from(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+template <int N, int P, int S, int G, int GR, int PADSH, int AR, int SYNC, bool KEEP, typename CI, typename CO>
+__device__ __forceinline__ void fft_stages_from(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P, KEEP>& W, const Buf& tw,
                                                 xchg_t<AR>* lds, int lds_stride) {
   if constexpr (S == Plan<N, P>::NSTAGES - 1) {
     fft_stage<N, P, S, G, GR, PADSH, AR, SYNC>(v, w, t, W, tw, lds, lds_stride);
@@ -641,16 +515,17 @@ __device__ __forceinline__ void swap_parts(C (&v)[G][P]) {
 // natural set v in, natural set w out.  The inverse is swap(F(swap(x))) with
 // swap(a + ib) = b + ia (= conj(F(conj x))), a register renaming.  An FP64
 // input or output set is taken or left without rounding.
-template <int N, int P, int G, bool INV, int GR, int PADSH, int AR, int SYNC, typename CI, typename CO>
-__device__ __forceinline__ void fft_line_io(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+template <int N, int P, int G, bool INV, int GR, int PADSH, int AR, int SYNC, bool KEEP, typename CI, typename CO>
+__device__ __forceinline__ void fft_line_io(CI (&v)[G][P], CO (&w)[G][P], int t, const Twid<N, P, KEEP>& W, const Buf& tw,
                                             xchg_t<AR>* lds, int lds_stride) {
   if constexpr (INV) swap_parts<G, P>(v);
   fft_stages_from<N, P, 0, G, GR, PADSH, AR, SYNC>(v, w, t, W, tw, lds, lds_stride);
   if constexpr (INV) swap_parts<G, P>(w);
 }
 
-template <int N, int P, int G, bool INV, int GR = G, int PADSH = NLSE_ROW_PADSH, int AR = F64, int SYNC = SYNC_BLOCK>
-__device__ __forceinline__ void fft_line(float2 (&v)[G][P], int t, const Twid<N, P>& W, const Buf& tw,
+template <int N, int P, int G, bool INV, int GR = G, int PADSH = NLSE_ROW_PADSH, int AR = F64, int SYNC = SYNC_BLOCK,
+          bool KEEP>
+__device__ __forceinline__ void fft_line(float2 (&v)[G][P], int t, const Twid<N, P, KEEP>& W, const Buf& tw,
                                          xchg_t<AR>* lds, int lds_stride) {
   fft_line_io<N, P, G, INV, GR, PADSH, AR, SYNC>(v, v, t, W, tw, lds, lds_stride);
 }

@@ -82,26 +82,16 @@ void build_ratio_twiddles(double2* rt) {
   }
 }
 
-// The FP64 table, then the same records as compensated FP32
-// {c_hi, s_hi, c_lo, s_lo} (c = c_hi + c_lo to ~2^-48) at tw_f32_offset(N)
-// double2 slots (a float4 has the size of a double2).
+// The FP64 table, then the ratio twiddles (rt_begin).
 template <int N>
 std::vector<double2> build_twiddles() {
-  const int n64 = tw_f32_offset(N);
-  std::vector<double2> tw(2 * n64 + rt_size(N), make_double2(0.0, 0.0));
-  build_ratio_twiddles<N, 16>(tw.data() + 2 * n64);
-  build_ratio_twiddles<N, 8>(tw.data() + 2 * n64);
-  build_ratio_twiddles<N, 4>(tw.data() + 2 * n64);
+  std::vector<double2> tw(rt_begin(N) + rt_size(N), make_double2(0.0, 0.0));
   build_stage_twiddles<N, 16>(tw);
   build_stage_twiddles<N, 8>(tw);
   build_stage_twiddles<N, 4>(tw);
-  static_assert(sizeof(float4) == sizeof(double2), "table layout");
-  for (int i = 0; i < n64; ++i) {
-    const double c = tw[i].x, sn = tw[i].y;
-    const float ch = (float)c, sh = (float)sn;
-    float4 r = make_float4(ch, sh, (float)(c - (double)ch), (float)(sn - (double)sh));
-    std::memcpy(&tw[n64 + i], &r, sizeof r);
-  }
+  build_ratio_twiddles<N, 16>(tw.data() + rt_begin(N));
+  build_ratio_twiddles<N, 8>(tw.data() + rt_begin(N));
+  build_ratio_twiddles<N, 4>(tw.data() + rt_begin(N));
   return tw;
 }
 
@@ -185,10 +175,18 @@ struct LineCfg {
   static constexpr int LPBZ = lines_per_block(128, N / PZ);
   static constexpr int PN = pick_p(N, NLSE_P8_FROM_NLNL, NLSE_P8_UPTO_NLNL);
   static constexpr int LPBN = lines_per_block(128, N / PN);
-  // whole 1-D runs
+  // whole 1-D runs; up to LINES1S lines (or line pairs), which leave a CU one
+  // or two lines, take the small plan: few points per lane, FP64 exchanges
+  // up to 1024 points, twiddles kept.  Per step, default against small plan:
+  // 250 lines of 1024 4.2 -> 3.0 us (pairs 11.3 -> 5.9), 200 of 256 3.1 ->
+  // 1.25, of 512 3.9 -> 2.0, of 2048 4.9 -> 3.7 us; 2000 lines of 1024 9.8 ->
+  // 12.8, 400 of 2048 5.2 -> 7.1 us
   static constexpr int P1 = N >= 16 ? 16 : N;
   static constexpr int LPB1D1 = lines_per_block(256, N / P1);
   static constexpr int LPB1D2 = lines_per_block(128, N / P1);
+  static constexpr int P1S = (N <= 256 || N == 1024) ? 4 : ((N == 512 || N == 2048) ? 8 : P1);
+  static constexpr int AR1S = N <= 1024 ? F64X : F64;
+  static constexpr int64_t LINES1S = P1S == P1 ? 0 : (N <= 1024 ? 1 << 17 : 1 << 16) / (N / P1S);
   // default column tile: 8 columns (64-byte row segments; narrower tiles
   // read 32-byte segments: 12.9 us against 8.5 us for an in-place copy of
   // a 2048^2 field); 2-D plans narrow it for small fields (nlse_plan_create)
@@ -248,23 +246,29 @@ static int row_launch(int p, int G, const RowArgs& a, hipStream_t s) {
   return fail(NLSE_ERR_ARG, "no row kernel of %d points per thread for length %d", p, N);
 }
 
+template <int N, int P, int L1, int L2, int AR, bool KEEP>
+static int line1d_launch_p(int G, const Line1DArgs& a, hipStream_t s) {
+  constexpr int T = N / P;
+  const int64_t blocks = G == 1 ? (a.ngroups + L1 - 1) / L1 : (a.ngroups + L2 - 1) / L2;
+  if (G == 2)
+    hipLaunchKernelGGL((k_line1d<N, P, L2, 2, true, AR, KEEP>), dim3((unsigned)blocks), dim3(L2 * T), 0, s, a);
+  else if (a.general)
+    hipLaunchKernelGGL((k_line1d<N, P, L1, 1, true, AR, KEEP>), dim3((unsigned)blocks), dim3(L1 * T), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_line1d<N, P, L1, 1, false, AR, KEEP>), dim3((unsigned)blocks), dim3(L1 * T), 0, s, a);
+  return launch_status("k_line1d");
+}
+
 template <int N>
 static int line1d_launch(int G, const Line1DArgs& a, hipStream_t s) {
   using C = LineCfg<N>;
-  constexpr int T = N / C::P1;
-  if (G == 1) {
-    constexpr int L = C::LPB1D1;
-    const int64_t blocks = (a.ngroups + L - 1) / L;
-    if (a.general)
-      hipLaunchKernelGGL((k_line1d<N, C::P1, L, 1, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-    else
-      hipLaunchKernelGGL((k_line1d<N, C::P1, L, 1, false>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-  } else {
-    constexpr int L = C::LPB1D2;
-    const int64_t blocks = (a.ngroups + L - 1) / L;
-    hipLaunchKernelGGL((k_line1d<N, C::P1, L, 2, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+  if constexpr (C::P1S != C::P1) {
+    if (a.ngroups <= C::LINES1S) {
+      constexpr int L = lines_per_block(64, N / C::P1S);
+      return line1d_launch_p<N, C::P1S, L, L, C::AR1S, true>(G, a, s);
+    }
   }
-  return launch_status("k_line1d");
+  return line1d_launch_p<N, C::P1, C::LPB1D1, C::LPB1D2, F64, false>(G, a, s);
 }
 
 // Nonlocal line kernels: stage 1 (k_nlc_z) or stage 2 (k_nlc_nl), one

@@ -54,6 +54,7 @@ struct NlcArgs {
   float drv_dz;
   float out_scale;
   int general;            // the loss varies from point to point (see nl1_block_I)
+  int through;            // write the results through to memory (ST_THROUGH)
   // band values of the convolved intensity
   const int* rowmap;      // [NY] band row index, or -1
   const float* rowband;   // [slabs][nb][NX]
@@ -104,6 +105,18 @@ __device__ __forceinline__ NlcLines nlc_lines(const NlcArgs& a, uint32_t g0, uin
   return L;
 }
 
+// Store a natural set at lane offset d, uniform offset u (bytes).
+template <int P, int T>
+__device__ __forceinline__ void put_line(const Buf& B, const float2 (&v)[P], uint32_t d, uint32_t u, bool through) {
+  if (through) {
+#pragma unroll
+    for (int m = 0; m < P; ++m) B.store<ST_THROUGH>(v[m], d, u + 8u * m * T);
+  } else {
+#pragma unroll
+    for (int m = 0; m < P; ++m) B.store(v[m], d, u + 8u * m * T);
+  }
+}
+
 // Stage 1: [I_x] of the two field lines (stored back in real space), then
 // Z = |A_a|^2 + i |A_b|^2 and its forward transform along x.
 template <int N, int P, int LPB, int FULL = 0>
@@ -140,9 +153,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_z(NlcArgs a) {
     }
     if (active) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int m = 0; m < P; ++m) A0.store(v[g][m], d, g * cs + 8u * m * T);
+      for (int g = 0; g < 2; ++g) put_line<P, T>(A0, v[g], d, g * cs, a.through);
     }
   }
   if constexpr (FULL) {
@@ -151,7 +162,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_z(NlcArgs a) {
     for (int g = 0; g < 2; ++g)
 #pragma unroll
       for (int m = 0; m < P; ++m) v[g][m] = make_float2(sqmag(v[g][m]), 0.f);
-    fft_line<N, P, 2, false, 1, NLSE_ROW_PADSH, F32C, SYNC>(v, t, W, tw, lline, LINE);
+    fft_line<N, P, 2, false, 1, NLSE_ROW_PADSH, F64, SYNC>(v, t, W, tw, lline, LINE);
     if (active) {
 #pragma unroll
       for (int g = 0; g < 2; ++g)
@@ -162,11 +173,8 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_z(NlcArgs a) {
     float2 z[1][P];
 #pragma unroll
     for (int m = 0; m < P; ++m) z[0][m] = make_float2(sqmag(v[0][m]), sqmag(v[1][m]));
-    fft_line<N, P, 1, false, 1, NLSE_ROW_PADSH, F32C, SYNC>(z, t, W, tw, lline, LINE);
-    if (active) {
-#pragma unroll
-      for (int m = 0; m < P; ++m) Z0.store(z[0][m], zd, 8u * m * T);
-    }
+    fft_line<N, P, 1, false, 1, NLSE_ROW_PADSH, F64, SYNC>(z, t, W, tw, lline, LINE);
+    if (active) put_line<P, T>(Z0, z[0], zd, 0, a.through);
   }
 }
 
@@ -212,7 +220,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
 #pragma unroll
     for (int m = 0; m < P; ++m) v[g][m] = A0.load<float2>(d, g * cs + 8u * m * T);
   const Twid<N, P> W = load_twiddles<N, P>(tw, t);
-  if (!a.direct) fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F32C, SYNC>(z, t, W, tw, lline, LINE);
+  if (!a.direct) fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F64, SYNC>(z, t, W, tw, lline, LINE);
   // z.x: convolved intensity of line 0, z.y: of line 1; band points take
   // their band values: a band row from the row band, else the r points at
   // either end from the column band (uniform tests skip the other points)
@@ -241,10 +249,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
 #pragma unroll
       for (int m = 0; m < P; ++m) w[0][m] = make_float2(w[0][m].x * a.out_scale, w[0][m].y * a.out_scale);
     }
-    if (active) {
-#pragma unroll
-      for (int m = 0; m < P; ++m) A0.store(w[0][m], d, c1 + 8u * m * T);
-    }
+    if (active) put_line<P, T>(A0, w[0], d, c1, a.through);
   };
 
   if constexpr (NC == 1) {
@@ -257,7 +262,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
 #pragma unroll
       for (int m = 0; m < P; ++m)
         z2[0][m] = a.Z[((int64_t)L.item * a.ny + L.y[1]) * N + t + m * T];
-      fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F32C, SYNC>(z2, t, W, tw, lline, LINE);
+      fft_line<N, P, 1, true, 1, NLSE_ROW_PADSH, F64, SYNC>(z2, t, W, tw, lline, LINE);
 #pragma unroll
       for (int m = 0; m < P; ++m) z[0][m].y = z2[0][m].x;
     }
@@ -284,9 +289,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
     }
     if (active) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int m = 0; m < P; ++m) A0.store(u[g][m], d, g * cs + 8u * m * T);
+      for (int g = 0; g < 2; ++g) put_line<P, T>(A0, u[g], d, g * cs, a.through);
     }
   } else {
     const NLParams2* pp = reinterpret_cast<const NLParams2*>(a.nlp) + 2 * L.item;

@@ -339,8 +339,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
       for (int g = 0; g < G; ++g) v[g][m] = AB.load<float2>(d, m * rs + 8u * g * WT);
     }
   }
-  Twid<N, P> W;
-  if constexpr (PK != PROP_KREAL) W = load_twiddles<N, P>(tw, t);
+  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
 
   constexpr int PADSH = 3;
   if constexpr (PK >= 0 && PK != PK_NONE && PK != PROP_KREAL) {
@@ -352,11 +351,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
     col_prop<N, P, G, CS, PK>(a, w, comp, t, c0);
     fft_line_io<N, P, G, true, GR, PADSH, FA, SYNC_BLOCK>(w, v, t, W, tw, lline, LINE);
   } else {
-    // the real spectrum multiplies an intensity (nonlocal response): its
-    // transforms are FP32 (see FftArith); field transforms are FP64
-    constexpr int AR = PK == PROP_KREAL ? F32C : FA;
-    static_assert(PK != PROP_KREAL || FA != F64X, "FP32 exchange");
-    if (a.do_fwd) fft_line<N, P, G, false, GR, PADSH, AR>(v, t, W, tw, lline, LINE);
+    if (a.do_fwd) fft_line<N, P, G, false, GR, PADSH, FA>(v, t, W, tw, lline, LINE);
     if (PK != PK_NONE && a.do_prop) {
       const int comp = (int)(slab % (uint32_t)a.ncomp);
       if (PK == PROP_KREAL || a.pkind == PROP_KREAL) {
@@ -399,7 +394,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
         }
       }
     }
-    if (a.do_inv) fft_line<N, P, G, true, GR, PADSH, AR>(v, t, W, tw, lline, LINE);
+    if (a.do_inv) fft_line<N, P, G, true, GR, PADSH, FA>(v, t, W, tw, lline, LINE);
   }
 
   if (a.out_scale != 1.f) {
@@ -474,7 +469,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
   float2* Z = a.A + slab * (int64_t)(N / 2) * a.NX;
   float2* lline = lds + cw * LINE;
   const Buf tw(a.tw);
-  const Twid<N, P> W{};  // (FP64 twiddles: none here)
+  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
 
   float2 v[1][P];
 #pragma unroll
@@ -484,7 +479,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
     v[0][m] = make_float2(0.5f * (za.x + zb.x), 0.5f * (za.y - zb.y));
     v[0][m + H] = make_float2(0.5f * (za.y + zb.y), 0.5f * (zb.x - za.x));
   }
-  fft_line<N, P, 1, false, 1, 3, F32C>(v, t, W, tw, lline, LINE);
+  fft_line<N, P, 1, false, 1, 3, F64>(v, t, W, tw, lline, LINE);
   const int hx = a.NX / 2 + 1;
 #pragma unroll
   for (int m = 0; m < P; ++m) {
@@ -493,7 +488,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
     const float f = a.kq[kyq * hx + j] * a.scale;
     v[0][m] = make_float2(v[0][m].x * f, v[0][m].y * f);
   }
-  fft_line<N, P, 1, true, 1, 3, F32C>(v, t, W, tw, lline, LINE);
+  fft_line<N, P, 1, true, 1, 3, F64>(v, t, W, tw, lline, LINE);
   if (act) {
 #pragma unroll
     for (int m = 0; m < H; ++m) {
@@ -567,13 +562,14 @@ struct Line1DArgs {
   int general;            // the loss varies from point to point (see nl1_block_I)
 };
 
-template <int N, int P, int LPB, int G, bool GEN = false>
+// KEEP: the twiddles too stay in registers for the whole run.
+template <int N, int P, int LPB, int G, bool GEN = false, int AR = F64, bool KEEP = false>
 __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
   constexpr int LINE = LdsLine<N, NLSE_ROW_PADSH, 0>::SIZE;
   constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
-  __shared__ float2 lds[LPB * G * LINE];
+  __shared__ xchg_t<AR> lds[LPB * G * LINE];
   const int li = threadIdx.x / T;
   const int t = threadIdx.x % T;
   const int64_t gi = (int64_t)blockIdx.x * LPB + li;
@@ -582,7 +578,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
   int64_t off[G];
   off[0] = item * G * N;
   if constexpr (G == 2) off[1] = off[0] + N;
-  float2* lline = lds + li * G * LINE;
+  xchg_t<AR>* lline = lds + li * G * LINE;
 
   float2 v[G][P];
 #pragma unroll
@@ -591,57 +587,56 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
     for (int m = 0; m < P; ++m) v[g][m] = active ? a.A[off[g] + t + m * T] : make_float2(0.f, 0.f);
   float vr[P], vi[P];
   load_v_set<P, T, GEN>(a.V, a.vkind, 0, (uint32_t)t, vr, vi);
+  // the propagator and the parameters stay in registers for the whole run
   const Buf tw(a.tw);
-  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
+  const Twid<N, P, KEEP> W = load_twiddles<N, P, KEEP>(tw, t);
   double2 pr[G][P];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int m = 0; m < P; ++m) pr[g][m] = a.prop[g * N + t + m * T];
+    for (int m = 0; m < P; ++m) {
+      pr[g][m] = a.prop[g * N + t + m * T];
+      pr[g][m].x *= a.scale;
+      pr[g][m].y *= a.scale;
+    }
+  using NL = typename std::conditional<G == 1, NLParams1, NLParams2>::type;
+  NL pre[G], post[G];  // (pre: "double" only)
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    post[g] = reinterpret_cast<const NL*>(a.precision == 1 ? a.nl_post : a.nl_full)[G * item + g];
+    pre[g] = a.precision == 1 ? reinterpret_cast<const NL*>(a.nl_pre)[G * item + g] : post[g];
+  }
+  const bool has_rabi = G == 2 && a.rabi != nullptr && a.precision == 0;
+  RabiParams rb{};
+  if (has_rabi) rb = a.rabi[item];
 
-  auto apply_nl = [&](const void* prm) {
+  auto apply_nl = [&](const NL (&p)[G]) {
     if (a.nlk != nullptr) {
       // nonlocal response: convolved intensities (nlse_1d.py:65-66 kernel)
       float I[G][P];
       conv1d_intensity<N, P, G>(v, I, reinterpret_cast<float*>(lline), t, a.nlk, a.nlr);
-      if constexpr (G == 1) {
-        const NLParams1 p = reinterpret_cast<const NLParams1*>(prm)[item];
-        nl1_block_I<P, GEN>(v[0], I[0], p, a.loss_sat, a.vkind == V_CPLX, vr, vi);
-      } else {
-        const NLParams2* pp = reinterpret_cast<const NLParams2*>(prm) + 2 * item;
-        const NLParams2 p1 = pp[0], p2 = pp[1];
-        nl2_block_I<P>(v[0], v[1], I[0], I[1], p1, p2, vr, vi);
-      }
+      if constexpr (G == 1) nl1_block_I<P, GEN>(v[0], I[0], p[0], a.loss_sat, a.vkind == V_CPLX, vr, vi);
+      else nl2_block_I<P>(v[0], v[1], I[0], I[1], p[0], p[1], vr, vi);
     } else if constexpr (G == 1) {
-      const NLParams1 p = reinterpret_cast<const NLParams1*>(prm)[item];
-      nl1_block<P, GEN>(v[0], p, a.loss_sat, a.vkind == V_CPLX, vr, vi);
+      nl1_block<P, GEN>(v[0], p[0], a.loss_sat, a.vkind == V_CPLX, vr, vi);
     } else {
-      const NLParams2* pp = reinterpret_cast<const NLParams2*>(prm) + 2 * item;
-      const NLParams2 p1 = pp[0], p2 = pp[1];
-      nl2_block<P>(v[0], v[1], p1, p2, vr, vi);
+      nl2_block<P>(v[0], v[1], p[0], p[1], vr, vi);
     }
   };
 
   for (int64_t s = 0; s < a.nsteps; ++s) {
-    if (a.precision == 1) apply_nl(a.nl_pre);
+    if (a.precision == 1) apply_nl(pre);
     double2 w[G][P];
-    fft_line_io<N, P, G, false, G, NLSE_ROW_PADSH, F64, SYNC>(v, w, t, W, tw, lline, LINE);
+    fft_line_io<N, P, G, false, G, NLSE_ROW_PADSH, AR, SYNC>(v, w, t, W, tw, lline, LINE);
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
-      for (int m = 0; m < P; ++m) w[g][m] = prop_c128(w[g][m], pr[g][m], a.scale);
-    fft_line_io<N, P, G, true, G, NLSE_ROW_PADSH, F64, SYNC>(w, v, t, W, tw, lline, LINE);
-    if (a.precision == 1) {
-      apply_nl(a.nl_post);
-    } else {
-      apply_nl(a.nl_full);
-      if constexpr (G == 2) {
-        if (a.rabi != nullptr) {
-          const RabiParams rb = a.rabi[item];
+      for (int m = 0; m < P; ++m) w[g][m] = prop_c128(w[g][m], pr[g][m], 1.0);
+    fft_line_io<N, P, G, true, G, NLSE_ROW_PADSH, AR, SYNC>(w, v, t, W, tw, lline, LINE);
+    apply_nl(post);
+    if (has_rabi) {
 #pragma unroll
-          for (int m = 0; m < P; ++m) rabi(v[0][m], v[1][m], rb);
-        }
-      }
+      for (int m = 0; m < P; ++m) rabi(v[0][m], v[G - 1][m], rb);
     }
   }
   if (active) {

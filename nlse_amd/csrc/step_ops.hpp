@@ -93,35 +93,40 @@ __device__ __forceinline__ bool wave_all(bool c) {
 }
 __device__ __forceinline__ bool wave_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 
-// A *= exp(-a + i th) for n points in memory with the library functions, for
-// arguments outside the series' ranges (a strided by `as`: 0 for one loss).
-// Out of line and on a copy of the points: rarely taken, and a call amid the
-// points would tie up the registers of the common path.
-__device__ __noinline__ void phase_loss_lib(float2* A, const float* a, int as, const float* th, int n) {
+// A *= exp(-a + i th) for n points {Re A, Im A, a, th} in private memory with
+// the library functions, for arguments outside the series' ranges.  Out of
+// line and on a copy of the points: rarely taken, and a call amid the points
+// would tie up the registers of the common path.
+typedef __attribute__((address_space(5))) float private_float;
+__device__ __noinline__ void phase_loss_lib(private_float* p, int n) {
   for (int m = 0; m < n; ++m) {
+    private_float* q = p + 4 * m;
+    const float ax = q[0], ay = q[1];
     float s2, c2;
-    const float em = expm1f(-a[m * as]);
-    sincosf(0.5f * th[m], &s2, &c2);
+    const float em = expm1f(-q[2]);
+    sincosf(0.5f * q[3], &s2, &c2);
     const float cm1 = -2.0f * s2 * s2;
     const float dr = fmaf(em, 1.0f + cm1, cm1);
     const float di = (1.0f + em) * (2.0f * s2 * c2);
-    A[m] = make_float2(A[m].x + fmaf(A[m].x, dr, -A[m].y * di), A[m].y + fmaf(A[m].y, dr, A[m].x * di));
+    q[0] = ax + fmaf(ax, dr, -ay * di);
+    q[1] = ay + fmaf(ay, dr, ax * di);
   }
 }
 
+// (a strided by `as`: 0 for one loss)
 template <int P>
 __device__ __forceinline__ void phase_loss_slow(float2* A, const float* a, int as, const float* th) {
-  float2 tA[P];
-  float ta[P], tt[P];
+  float pts[4 * P];
 #pragma unroll
   for (int m = 0; m < P; ++m) {
-    tA[m] = A[m];
-    ta[m] = a[m * as];
-    tt[m] = th[m];
+    pts[4 * m] = A[m].x;
+    pts[4 * m + 1] = A[m].y;
+    pts[4 * m + 2] = a[m * as];
+    pts[4 * m + 3] = th[m];
   }
-  phase_loss_lib(tA, ta, 1, tt, P);
+  phase_loss_lib((private_float*)pts, P);
 #pragma unroll
-  for (int m = 0; m < P; ++m) A[m] = tA[m];
+  for (int m = 0; m < P; ++m) A[m] = make_float2(pts[4 * m], pts[4 * m + 1]);
 }
 
 // Apply exp(-a + i theta) to P points with one wave-uniform choice of the
