@@ -914,7 +914,7 @@ int nlse_plan_create(const nlse_plan_desc* d, nlse_plan** out) {
   }
   const int64_t points = d->items * d->ncomp * (d->ndim >= 2 ? d->ny : 1) * d->nx * (d->ndim == 3 ? d->nt : 1);
   p->small = d->ndim == 2 && points <= SMALL_FIELD;
-  p->through = points * 8 <= WRITE_THROUGH;
+  p->through = points * (p->wide ? 16 : 8) <= WRITE_THROUGH;
   if (d->row_points != 0) {
     const int pr = p->rops->p_row, pa = p->rops->p_row_alt, ps = p->rops->p_row_small;
     const bool ok = d->row_points == pr || (d->ndim != 1 && (d->row_points == pa || (p->small && d->row_points == ps)));
@@ -1748,6 +1748,7 @@ static WRowArgs wrow_args(const nlse_plan* p, void* A) {
   r.drv_r1 = p->fr1;
   r.drv_dz = p->drv_dz;
   r.out_scale = 1.0;
+  r.through = p->through;
   return r;
 }
 
@@ -1766,6 +1767,7 @@ static WColArgs wcol_args(const nlse_plan* p, void* A) {
   c.ptab = p->ptab;
   c.scale = 1.0 / ((double)p->d.nx * (double)p->d.ny);
   c.out_scale = 1.0;
+  c.through = p->through;
   return c;
 }
 
@@ -1838,6 +1840,7 @@ static WColArgs wcolx3d_args(const nlse_plan* p, void* A) {
   c.tw = p->wtwx;
   c.scale = 1.0;
   c.out_scale = 1.0;
+  c.through = p->through;
   return c;
 }
 

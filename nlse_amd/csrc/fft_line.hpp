@@ -50,95 +50,9 @@ __device__ __forceinline__ float2 to_f32(double2 a) { return make_float2((float)
 __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ double2 mul_mi(double2 a) { return make_double2(a.y, -a.x); }
-// a * w for a stage twiddle w = c + i s
-__device__ __forceinline__ double2 cmul_tw(double2 a, double2 w) {
-  return make_double2(fma(a.x, w.x, -a.y * w.y), fma(a.x, w.y, a.y * w.x));
-}
 constexpr double K_R2 = 0.70710678118654752440084436210484904;  // 1/sqrt(2)
 constexpr double K_C8 = 0.92387953251128675612818318939678829;  // cos(pi/8)
 constexpr double K_S8 = 0.38268343236508977172845998403039887;  // sin(pi/8)
-// a * (c - i s)
-__device__ __forceinline__ double2 rot(double2 a, double c, double s) {
-  return make_double2(fma(a.x, c, a.y * s), fma(a.y, c, -a.x * s));
-}
-// a * W8^1 = a * (1 - i)/sqrt2
-__device__ __forceinline__ double2 mul_w8_1(double2 a) { return make_double2((a.x + a.y) * K_R2, (a.y - a.x) * K_R2); }
-// a * W8^3 = a * (-1 - i)/sqrt2
-__device__ __forceinline__ double2 mul_w8_3(double2 a) { return make_double2((a.y - a.x) * K_R2, -(a.x + a.y) * K_R2); }
-
-// ---------------------------------------------------------- butterflies
-// Forward DFTs (kernel exp(-2 pi i n k / R)), in place on x[0..R-1].
-__device__ __forceinline__ void dft2(double2* x) {
-  double2 a = x[0], b = x[1];
-  x[0] = cadd(a, b);
-  x[1] = csub(a, b);
-}
-
-__device__ __forceinline__ void dft4(double2& a, double2& b, double2& c, double2& d) {
-  double2 t0 = cadd(a, c), t1 = csub(a, c), t2 = cadd(b, d), t3 = mul_mi(csub(b, d));
-  a = cadd(t0, t2);  // X0
-  c = csub(t0, t2);  // X2
-  b = cadd(t1, t3);  // X1
-  d = csub(t1, t3);  // X3
-}
-
-__device__ __forceinline__ void dft4(double2* x) { dft4(x[0], x[1], x[2], x[3]); }
-
-__device__ __forceinline__ void dft8(double2* x) {
-  // n = 2 n1 + n2, k = k1 + 4 k2
-  double2 e0 = x[0], e1 = x[2], e2 = x[4], e3 = x[6];
-  double2 o0 = x[1], o1 = x[3], o2 = x[5], o3 = x[7];
-  dft4(e0, e1, e2, e3);
-  dft4(o0, o1, o2, o3);
-  o1 = mul_w8_1(o1);
-  o2 = mul_mi(o2);
-  o3 = mul_w8_3(o3);
-  x[0] = cadd(e0, o0); x[4] = csub(e0, o0);
-  x[1] = cadd(e1, o1); x[5] = csub(e1, o1);
-  x[2] = cadd(e2, o2); x[6] = csub(e2, o2);
-  x[3] = cadd(e3, o3); x[7] = csub(e3, o3);
-}
-
-__device__ __forceinline__ void dft16(double2* x) {
-  // n = 4 n1 + n2, k = k1 + 4 k2: radix-4 over n1, twiddle W16^(n2 k1),
-  // radix-4 over n2.
-  double2 y[16];
-#pragma unroll
-  for (int n2 = 0; n2 < 4; ++n2) {
-    double2 a = x[n2], b = x[4 + n2], c = x[8 + n2], d = x[12 + n2];
-    dft4(a, b, c, d);
-    y[n2 * 4 + 0] = a; y[n2 * 4 + 1] = b; y[n2 * 4 + 2] = c; y[n2 * 4 + 3] = d;
-  }
-  // W16^1 = c8 - i s8, W16^2 = W8^1, W16^3 = s8 - i c8,
-  // W16^4 = -i, W16^6 = W8^3, W16^9 = -c8 + i s8 = -(W16^1)
-  y[1 * 4 + 1] = rot(y[5], K_C8, K_S8);
-  y[1 * 4 + 2] = mul_w8_1(y[6]);
-  y[1 * 4 + 3] = rot(y[7], K_S8, K_C8);
-  y[2 * 4 + 1] = mul_w8_1(y[9]);
-  y[2 * 4 + 2] = mul_mi(y[10]);
-  y[2 * 4 + 3] = mul_w8_3(y[11]);
-  y[3 * 4 + 1] = rot(y[13], K_S8, K_C8);
-  y[3 * 4 + 2] = mul_w8_3(y[14]);
-  {
-    double2 r = rot(y[15], K_C8, K_S8);
-    y[15] = make_double2(-r.x, -r.y);
-  }
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) {
-    double2 a = y[0 * 4 + k1], b = y[1 * 4 + k1], c = y[2 * 4 + k1], d = y[3 * 4 + k1];
-    dft4(a, b, c, d);
-    x[k1] = a; x[k1 + 4] = b; x[k1 + 8] = c; x[k1 + 12] = d;
-  }
-}
-
-template <int R, typename C>
-__device__ __forceinline__ void dft(C* x) {
-  if constexpr (R == 2) dft2(x);
-  else if constexpr (R == 4) dft4(x);
-  else if constexpr (R == 8) dft8(x);
-  else if constexpr (R == 16) dft16(x);
-  else static_assert(R == 2, "unsupported radix");
-}
 
 // ------------------------------------------------------------ radix plan
 // Stages for N = 2^n with at most P points per thread: the remainder radix
@@ -164,37 +78,7 @@ struct Plan {
     for (int i = 0; i < s; ++i) p *= radix(i);
     return p;
   }
-  // Twiddle table offset of stage s (stages with Ns > 1), layout [k-1][jm].
-  __host__ __device__ static constexpr int tw_offset(int s) {
-    int off = 0;
-    for (int i = 1; i < s; ++i) off += (radix(i) - 1) * ns(i);
-    return off;
-  }
-  static constexpr int TW_SIZE = tw_offset(NSTAGES);
 };
-
-// Twiddle records of the stages of Plan<n, p> (0 when p > n).
-__host__ __device__ constexpr int tw_size_np(int n, int p) {
-  if (p > n) return 0;
-  const int logn = ilog2c(n), logp = ilog2c(p);
-  const int rem = logn % logp, nst = logn / logp + (rem ? 1 : 0);
-  int off = 0, ns = rem ? (1 << rem) : p;
-  for (int i = 1; i < nst; ++i) {
-    off += (p - 1) * ns;
-    ns *= p;
-  }
-  return off;
-}
-
-// One twiddle table per line length serves every per-thread set size: the
-// stage tables of P = 16, 8 and 4 are stored one after the other, so
-// kernels of one length with different P share a table.
-__host__ __device__ constexpr int tw_base(int n, int p) {
-  return (p < 16 ? tw_size_np(n, 16) : 0) + (p < 8 ? tw_size_np(n, 8) : 0);
-}
-__host__ __device__ constexpr int tw_union_size(int n) {
-  return tw_size_np(n, 16) + tw_size_np(n, 8) + tw_size_np(n, 4);
-}
 
 // Stores kept in the L2 until the kernel's end, or written through to memory
 // (sc1) while the kernel runs.
@@ -232,6 +116,10 @@ struct Buf {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, lane, uni, ST);
   }
+  template <int ST = ST_BACK>
+  __device__ __forceinline__ void store(double2 x, uint32_t lane, uint32_t uni) const {
+    store<ST>(__builtin_bit_cast(float4, x), lane, uni);
+  }
 };
 
 // Padding of the row kernels' LDS lines (one float2 every 2^NLSE_ROW_PADSH
@@ -253,7 +141,7 @@ __host__ __device__ __forceinline__ constexpr int lds_pad(int i) { return i + (i
 
 // Ratio twiddles {cos, tan} of the factored butterflies (dft_fma): R/2 entries
 // per stage of radix R and index jm, the stages of P = 16, 8 and 4 one after the
-// other, behind the other table.
+// other: one table per line length serves every number of points per thread.
 __host__ __device__ constexpr int rt_offset(int n, int p, int stage) {
   const int logn = ilog2c(n), logp = ilog2c(p), rem = logn % logp;
   int off = 0, ns = rem ? (1 << rem) : p;
@@ -272,11 +160,6 @@ __host__ __device__ constexpr int rt_base(int n, int p) {
   return (p < 16 ? rt_size_np(n, 16) : 0) + (p < 8 ? rt_size_np(n, 8) : 0);
 }
 __host__ __device__ constexpr int rt_size(int n) { return rt_size_np(n, 16) + rt_size_np(n, 8) + rt_size_np(n, 4); }
-
-// Twiddle table of a line length: the FP64 records {c, s} of every stage
-// table (tw_union_size(n) entries; the complex128 kernels' twiddles), followed
-// by the ratio twiddles.
-__host__ __device__ constexpr int rt_begin(int n) { return tw_union_size(n) > 0 ? tw_union_size(n) : 1; }
 
 // Precision of a transform's exchanges: F64 rounds to complex64 once per stage,
 // F64X carries FP64: one rounding per transform and no conversions between
@@ -388,7 +271,7 @@ struct Twid {
 // Byte offset of stage S's ratio pairs.
 template <int N, int P, int S>
 constexpr uint32_t stage_twiddles() {
-  return 16u * (uint32_t)(rt_begin(N) + rt_base(N, P) + rt_offset(N, P, S));
+  return 16u * (uint32_t)(rt_base(N, P) + rt_offset(N, P, S));
 }
 
 // A value the compiler cannot see through: what is computed from it is

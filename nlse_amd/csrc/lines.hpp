@@ -37,27 +37,8 @@ struct LineOps {
 };
 
 // ------------------------------------------------------ twiddle tables
-// One table per (device, line length): the stage tables of Plan<N, P> for
-// P = 16, 8, 4 in that order (tw_base), each in the layout of
-// Plan<N,P>::tw_offset: stage s (s >= 1), entry [(k-1)*Ns + jm] =
-// exp(-2 pi i jm k / (Ns R)), evaluated and stored in FP64 as {c, s}.
-template <int N, int P>
-void build_stage_twiddles(std::vector<double2>& tw) {
-  if constexpr (P <= N) {
-    using PL = Plan<N, P>;
-    const int base = tw_base(N, P);
-    for (int s = 1; s < PL::NSTAGES; ++s) {
-      const int R = PL::radix(s), NS = PL::ns(s), off = base + PL::tw_offset(s);
-      for (int k = 1; k < R; ++k)
-        for (int jm = 0; jm < NS; ++jm) {
-          // angle = -2 pi * jm*k/(NS*R); reduce the rational first
-          const long num = (long)jm * k, den = (long)NS * R;
-          const double ang = -2.0 * M_PI * (double)num / (double)den;
-          tw[off + (k - 1) * NS + jm] = make_double2(std::cos(ang), std::sin(ang));
-        }
-    }
-  }
-}
+// One table per (device, line length): the ratio pairs of the stages of Plan<N,
+// P> for P = 16, 8, 4 in that order (rt_base), evaluated and stored in FP64.
 
 // Ratio pairs {c, s/c} of the stages of Plan<N, P> (rt_offset): for the levels r
 // = R, R/2, .., 2 of a stage of radix R, w^(R/r) W_r^k with k < max(1, r/4) and
@@ -82,16 +63,12 @@ void build_ratio_twiddles(double2* rt) {
   }
 }
 
-// The FP64 table, then the ratio twiddles (rt_begin).
 template <int N>
 std::vector<double2> build_twiddles() {
-  std::vector<double2> tw(rt_begin(N) + rt_size(N), make_double2(0.0, 0.0));
-  build_stage_twiddles<N, 16>(tw);
-  build_stage_twiddles<N, 8>(tw);
-  build_stage_twiddles<N, 4>(tw);
-  build_ratio_twiddles<N, 16>(tw.data() + rt_begin(N));
-  build_ratio_twiddles<N, 8>(tw.data() + rt_begin(N));
-  build_ratio_twiddles<N, 4>(tw.data() + rt_begin(N));
+  std::vector<double2> tw(rt_size(N) > 0 ? rt_size(N) : 1, make_double2(0.0, 0.0));
+  build_ratio_twiddles<N, 16>(tw.data());
+  build_ratio_twiddles<N, 8>(tw.data());
+  build_ratio_twiddles<N, 4>(tw.data());
   return tw;
 }
 

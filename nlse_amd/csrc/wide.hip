@@ -34,13 +34,13 @@ int lds_limit(const void* fn, size_t bytes) {
 // two-component thread is then 64 VGPRs).
 template <int N>
 constexpr int wp() {
-  return N >= 8 ? 8 : N;
+  return 8;
 }
 
 template <int N, int G>
 int wrow_launch_g(const WRowArgs& a, hipStream_t s) {
   constexpr int P = wp<N>(), T = N / P;
-  constexpr int L = T >= 256 / G ? 1 : (256 / G) / T;
+  constexpr int L = T >= 128 / G ? 1 : (128 / G) / T;
   const size_t bytes = (size_t)L * G * WLine<N>::SIZE * sizeof(double2);
   auto fn = k_wrow<N, P, L, G>;
   int rc = lds_limit((const void*)fn, bytes);

@@ -26,92 +26,15 @@ namespace nlse {
 constexpr int WPADSH = 3;
 template <int N>
 struct WLine {
-  static constexpr int SIZE = N + (N >> WPADSH) + 1;
+  static constexpr int SIZE = LdsLine<N, WPADSH, 0>::SIZE;
 };
-__device__ __forceinline__ int wpad(int i) { return i + (i >> WPADSH); }
 
-// One Stockham stage of G lines in FP64 (see fft_stage): outputs of a
-// middle stage go through LDS, the last stage lands on the natural set.
-template <int N, int P, int S, int G>
-__device__ __forceinline__ void wfft_stage(double2 (&v)[G][P], int t, const double2* __restrict__ tw,
-                                           double2* lds) {
-  using PL = Plan<N, P>;
-  constexpr int R = PL::radix(S);
-  constexpr int NS = PL::ns(S);
-  constexpr int NB = P / R;
-  constexpr int T = PL::T;
-  constexpr bool LAST = (S == PL::NSTAGES - 1);
-  constexpr int LINE = WLine<N>::SIZE;
-  double2 tws[NB][R > 1 ? R - 1 : 1];
-  if constexpr (NS > 1) {
-    const double2* twst = tw + tw_base(N, P) + PL::tw_offset(S);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int jm = (t + b * T) & (NS - 1);
-#pragma unroll
-      for (int k = 1; k < R; ++k) tws[b][k - 1] = twst[(k - 1) * NS + jm];
-    }
-  }
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * T;
-    const int jm = j & (NS - 1);
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      double2 x[R];
-#pragma unroll
-      for (int k = 0; k < R; ++k) x[k] = v[g][b + k * NB];
-      if constexpr (NS > 1) {
-#pragma unroll
-        for (int k = 1; k < R; ++k) x[k] = cmul_tw(x[k], tws[b][k - 1]);
-      }
-      dft<R>(x);
-      if constexpr (LAST) {
-#pragma unroll
-        for (int k = 0; k < R; ++k) v[g][b + k * NB] = x[k];
-      } else {
-        const int base = (j / NS) * NS * R + jm;
-#pragma unroll
-        for (int k = 0; k < R; ++k) lds[g * LINE + wpad(base + k * NS)] = x[k];
-      }
-    }
-  }
-  if constexpr (!LAST) {
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = lds[g * LINE + wpad(t + m * T)];
-    __syncthreads();
-  }
-}
-
-template <int N, int P, int S, int G>
-__device__ __forceinline__ void wfft_stages_from(double2 (&v)[G][P], int t, const double2* __restrict__ tw,
-                                                 double2* lds) {
-  if constexpr (S < Plan<N, P>::NSTAGES) {
-    wfft_stage<N, P, S, G>(v, t, tw, lds);
-    wfft_stages_from<N, P, S + 1, G>(v, t, tw, lds);
-  }
-}
-
-// Forward or unnormalised inverse DFT of G lines (inverse = swap re/im
-// around the forward transform).
-template <int N, int P, int G, bool INV>
-__device__ __forceinline__ void wfft_line(double2 (&v)[G][P], int t, const double2* __restrict__ tw, double2* lds) {
-  if constexpr (INV) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = make_double2(v[g][m].y, v[g][m].x);
-  }
-  wfft_stages_from<N, P, 0, G>(v, t, tw, lds);
-  if constexpr (INV) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) v[g][m] = make_double2(v[g][m].y, v[g][m].x);
-  }
+// Forward or unnormalised inverse DFT of G lines: the factored FP64 butterflies
+// of fft_line.hpp with FP64 exchanges.
+template <int N, int P, int G, bool INV, int SYNC, bool KEEP>
+__device__ __forceinline__ void wfft_line(double2 (&v)[G][P], int t, const Twid<N, P, KEEP>& W, const Buf& tw,
+                                          double2* lds) {
+  fft_line_io<N, P, G, INV, G, WPADSH, F64X, SYNC>(v, v, t, W, tw, lds, WLine<N>::SIZE);
 }
 
 // ------------------------------------------------------------ pointwise
@@ -147,10 +70,6 @@ enum : int { V_REAL64 = 3, V_CPLX128 = 4 };
 // numpy/cupy give k/2*V for a float32 array; complex64 V: the same per part,
 // which is exact complex64 scaling by a real), returned as FP64 (re, im).
 __device__ __forceinline__ double2 wvprime(const void* V, int vkind, int64_t idx, double vmul) {
-  if (vkind == V_REAL) {
-    const float x = reinterpret_cast<const float*>(V)[idx];
-    return make_double2(vmul != 0.0 ? (double)((float)vmul * x) : (double)x, 0.0);
-  }
   if (vkind == V_CPLX) {
     const float2 w = reinterpret_cast<const float2*>(V)[idx];
     if (vmul == 0.0) return make_double2((double)w.x, (double)w.y);
@@ -168,44 +87,165 @@ __device__ __forceinline__ double2 wvprime(const void* V, int vkind, int64_t idx
   return make_double2(0.0, 0.0);
 }
 
-// A *= exp(-a + i th) as A + A (f - 1) with
-// f - 1 = expm1(-a) cos(th) - 2 sin^2(th/2) + i e^{-a} sin(th).
-__device__ __forceinline__ double2 wapply(double2 A, double a, double th) {
-  double s2, c2;
-  sincos(0.5 * th, &s2, &c2);
-  const double em = expm1(-a);
-  const double cosm1 = -2.0 * s2 * s2;
-  const double dr = fma(em, 1.0 + cosm1, cosm1);
-  const double di = (1.0 + em) * (2.0 * s2 * c2);
-  return make_double2(A.x + fma(A.x, dr, -A.y * di), A.y + fma(A.y, dr, A.x * di));
+// V' of the P points idx + m * step, the kind tested once; a float32 potential
+// is given in vf (loaded beside the field).
+template <int P>
+__device__ __forceinline__ void wvprime_set(double (&vr)[P], double (&vi)[P], const float (&vf)[P], const void* V,
+                                            int vkind, int64_t idx, int step, double vmul) {
+#pragma unroll
+  for (int m = 0; m < P; ++m) {
+    vr[m] = vmul != 0.0 ? (double)((float)vmul * vf[m]) : (double)vf[m];
+    vi[m] = 0.0;
+  }
+  auto each = [&](int kind) {
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      const double2 w = wvprime(V, kind, idx + m * step, vmul);
+      vr[m] = w.x;
+      vi[m] = w.y;
+    }
+  };
+  if (vkind == V_CPLX) each(V_CPLX);
+  else if (vkind == V_REAL64) each(V_REAL64);
+  else if (vkind == V_CPLX128) each(V_CPLX128);
 }
 
-// nl_prop / nl_prop_without_V on one point of a complex128 field
-// (kernels_gpu.py:4-65 / kernels_cpu.py:5-63 in complex128): intensity I
-// (|A|^2, or the convolved intensity of a nonlocal response), V' of the point.
-__device__ __forceinline__ double2 wnl1(double2 A, double I, const WNL1& p, bool loss_sat, double2 vp) {
-  const double sat = 1.0 / fma(I, p.inv_isat, 1.0);
-  const double s = loss_sat ? sat : 1.0;
-  double a = fma(p.adz, s, fma(p.dzv, vp.y, 0.0));
-  double th = fma(p.gdz * I, sat, p.dzv * vp.x);
-  if (p.cplx) {
-    a = fma(p.gdz_i * I, sat, fma(p.dzv_i, vp.x, a));
-    th -= fma(p.dzv_i, vp.y, p.adz_i * s);
+// A *= exp(-a + i th) for n points {Re A, Im A, a, th} in private memory as
+// A + A (f - 1) with f - 1 = expm1(-a) cos(th) - 2 sin^2(th/2) + i e^{-a}
+// sin(th), by the library functions: arguments outside the series' ranges.
+typedef __attribute__((address_space(5))) double private_double;
+__device__ __noinline__ inline void wphase_lib(private_double* p, int n) {
+  for (int m = 0; m < n; ++m) {
+    private_double* q = p + 4 * m;
+    const double ax = q[0], ay = q[1];
+    double s2, c2;
+    sincos(0.5 * q[3], &s2, &c2);
+    const double em = expm1(-q[2]);
+    const double cosm1 = -2.0 * s2 * s2;
+    const double dr = fma(em, 1.0 + cosm1, cosm1);
+    const double di = (1.0 + em) * (2.0 * s2 * c2);
+    q[0] = ax + fma(ax, dr, -ay * di);
+    q[1] = ay + fma(ay, dr, ax * di);
   }
-  return wapply(A, a, th);
+}
+
+// e^x - 1 for |x| <= 1/8: Taylor series to x^12 (next term 3e-21 relative).
+__device__ __forceinline__ double wexpm1_small(double x) {
+  double p = 1.0 / 479001600.0;
+  p = fma(x, p, 1.0 / 39916800.0);
+  p = fma(x, p, 1.0 / 3628800.0);
+  p = fma(x, p, 1.0 / 362880.0);
+  p = fma(x, p, 1.0 / 40320.0);
+  p = fma(x, p, 1.0 / 5040.0);
+  p = fma(x, p, 1.0 / 720.0);
+  p = fma(x, p, 1.0 / 120.0);
+  p = fma(x, p, 1.0 / 24.0);
+  p = fma(x, p, 1.0 / 6.0);
+  p = fma(x, p, 0.5);
+  return fma(x * x, p, x);
+}
+
+// sin and cos for |x| <= pi/4: Taylor series to x^17 and x^18 (next terms 1e-19
+// and 3e-21 relative).
+__device__ __forceinline__ void wsincos_small(double x, double& s, double& c) {
+  const double z = x * x;
+  double p = 1.0 / 355687428096000.0;
+  p = fma(z, p, -1.0 / 1307674368000.0);
+  p = fma(z, p, 1.0 / 6227020800.0);
+  p = fma(z, p, -1.0 / 39916800.0);
+  p = fma(z, p, 1.0 / 362880.0);
+  p = fma(z, p, -1.0 / 5040.0);
+  p = fma(z, p, 1.0 / 120.0);
+  p = fma(z, p, -1.0 / 6.0);
+  s = fma(x * z, p, x);
+  double q = -1.0 / 6402373705728000.0;
+  q = fma(z, q, 1.0 / 20922789888000.0);
+  q = fma(z, q, -1.0 / 87178291200.0);
+  q = fma(z, q, 1.0 / 479001600.0);
+  q = fma(z, q, -1.0 / 3628800.0);
+  q = fma(z, q, 1.0 / 40320.0);
+  q = fma(z, q, -1.0 / 720.0);
+  q = fma(z, q, 1.0 / 24.0);
+  q = fma(z, q, -0.5);
+  c = fma(z, q, 1.0);
+}
+
+// The same on P points with one choice of the evaluation for the wave: the
+// series for half phases up to pi/4 and losses up to 1/8 (about 45 operations
+// a point, 35 where one loss serves all points, against some 250 of the library
+// functions).
+template <int P>
+__device__ __forceinline__ void wapply(double2 (&A)[P], const double (&a)[P], bool one_loss, const double (&th)[P]) {
+  bool small = true;
+#pragma unroll
+  for (int m = 0; m < P; ++m) small = small && fabs(th[m]) <= 1.5707963267948966 && fabs(a[m]) <= 0.125;
+  if (wave_all(small)) {
+    double em = wexpm1_small(-a[0]);
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      if (m > 0 && !one_loss) em = wexpm1_small(-a[m]);
+      double s2, c2;
+      wsincos_small(0.5 * th[m], s2, c2);
+      const double cosm1 = -2.0 * s2 * s2;
+      const double dr = fma(em, 1.0 + cosm1, cosm1);
+      const double di = (1.0 + em) * (2.0 * s2 * c2);
+      A[m] = make_double2(A[m].x + fma(A[m].x, dr, -A[m].y * di), A[m].y + fma(A[m].y, dr, A[m].x * di));
+    }
+  } else {
+    double pts[4 * P];
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      pts[4 * m] = A[m].x;
+      pts[4 * m + 1] = A[m].y;
+      pts[4 * m + 2] = a[m];
+      pts[4 * m + 3] = th[m];
+    }
+    wphase_lib((private_double*)pts, P);
+#pragma unroll
+    for (int m = 0; m < P; ++m) A[m] = make_double2(pts[4 * m], pts[4 * m + 1]);
+  }
+}
+
+// nl_prop / nl_prop_without_V on P points of a complex128 field
+// (kernels_gpu.py:4-65 / kernels_cpu.py:5-63 in complex128): intensity I
+// (|A|^2, or the convolved intensity of a nonlocal response), V' of the points.
+template <int P>
+__device__ __forceinline__ void wnl1(double2 (&A)[P], const double (&I)[P], const WNL1& p, bool loss_sat,
+                                     const double (&vr)[P], const double (&vi)[P], bool has_vi) {
+  double a[P], th[P];
+  const bool sats = wave_any(p.inv_isat != 0.0), cplx = wave_any(p.cplx != 0);
+#pragma unroll
+  for (int m = 0; m < P; ++m) {
+    const double sat = sats ? 1.0 / fma(I[m], p.inv_isat, 1.0) : 1.0;
+    const double s = loss_sat ? sat : 1.0;
+    a[m] = fma(p.adz, s, fma(p.dzv, vi[m], 0.0));
+    th[m] = fma(p.gdz * I[m], sat, p.dzv * vr[m]);
+    if (cplx) {
+      a[m] = fma(p.gdz_i * I[m], sat, fma(p.dzv_i, vr[m], a[m]));
+      th[m] -= fma(p.dzv_i, vi[m], p.adz_i * s);
+    }
+  }
+  wapply<P>(A, a, !(cplx || has_vi || (loss_sat && sats)), th);
 }
 
 // nl_prop_c for one component (kernels_cpu.py:66-141) from the shared
 // intensity snapshot (Is: own component, Io: the other).
-__device__ __forceinline__ double2 wnl2(double2 A, double Is, double Io, const WNL2& p, double2 vp) {
-  const double sat = 1.0 / fma(Io, p.inv_is_o, fma(Is, p.inv_is_s, 1.0));
-  double a = fma(p.adz, sat, p.dzv * vp.y);
-  double th = fma(p.gs_dz * Is, sat, fma(p.gc_dz * Io, sat, p.dzv * vp.x));
-  if (p.cplx) {
-    a = fma(p.gs_dz_i * Is, sat, fma(p.gc_dz_i * Io, sat, fma(p.dzv_i, vp.x, a)));
-    th -= fma(p.dzv_i, vp.y, p.adz_i * sat);
+template <int P>
+__device__ __forceinline__ void wnl2(double2 (&A)[P], const double (&Is)[P], const double (&Io)[P], const WNL2& p,
+                                     const double (&vr)[P], const double (&vi)[P], bool has_vi) {
+  double a[P], th[P];
+  const bool sats = wave_any(p.inv_is_s != 0.0 || p.inv_is_o != 0.0), cplx = wave_any(p.cplx != 0);
+#pragma unroll
+  for (int m = 0; m < P; ++m) {
+    const double sat = sats ? 1.0 / fma(Io[m], p.inv_is_o, fma(Is[m], p.inv_is_s, 1.0)) : 1.0;
+    a[m] = fma(p.adz, sat, p.dzv * vi[m]);
+    th[m] = fma(p.gs_dz * Is[m], sat, fma(p.gc_dz * Io[m], sat, p.dzv * vr[m]));
+    if (cplx) {
+      a[m] = fma(p.gs_dz_i * Is[m], sat, fma(p.gc_dz_i * Io[m], sat, fma(p.dzv_i, vr[m], a[m])));
+      th[m] -= fma(p.dzv_i, vi[m], p.adz_i * sat);
+    }
   }
-  return wapply(A, a, th);
+  wapply<P>(A, a, !(cplx || has_vi || sats), th);
 }
 
 __device__ __forceinline__ void wrabi(double2& A1, double2& A2, const WRabi& r) {
@@ -250,6 +290,7 @@ struct WRowArgs {
   int has_b;
   int loss_sat;
   int write_I;            // store the field and |A|^2 (FP64) after I_x, nothing else
+  int through;            // stores written through (fields of WRITE_THROUGH bytes at most)
   const void* nlp_a;      // WNL1[items] or WNL2[items*2]
   const void* nlp_b;
   const WRabi* rabi;      // [items]
@@ -266,6 +307,12 @@ struct WRowArgs {
   double out_scale;
 };
 
+// Two waves per SIMD of 1024^2 points load, transform and store in step, so a
+// sweep is the sum of its memory time (5 us), VALU (5 us) and exchanges (3 us)
+// and launch, not their maximum: 18.8 us.  Series instead of library functions,
+// the factored butterflies and stores written through took a 2-D step from
+// 43.3 to 37.6 us (2048^2: 118.7 to 87.5, 256^2: 16.3 to 12.0); 4 points per
+// lane (121 us at 2048^2) and kept twiddles at 1024 points did not help.
 // Rows of length N (x rows of 2-D fields, t rows of 3-D fields): LPB line
 // groups per block, G components per group.  Dynamic LDS: LPB*G lines.
 template <int N, int P, int LPB, int G>
@@ -288,54 +335,80 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wrow(WRowArgs a) {
     off[1] = off[0] + a.rows_per_item * N;
   }
   double2* lline = wsm + li * G * LINE;
+  constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
+  constexpr bool KEEP = G == 1 && twid_kept(N, P);  // two lines leave no registers for them
 
   double2 v[G][P];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int m = 0; m < P; ++m) v[g][m] = active ? a.A[off[g] + t + m * T] : make_double2(0.0, 0.0);
+  const Buf tw(a.tw);
+  const Twid<N, P, KEEP> W = load_twiddles<N, P, KEEP>(tw, t);
+  // a float32 potential is loaded beside the field
+  const int64_t vbase = item * a.v_item_stride + y * N + t;
+  const bool v_early = a.vkind == V_REAL && (a.has_a || a.has_b);
+  float vf[P];
+#pragma unroll
+  for (int m = 0; m < P; ++m) vf[m] = v_early ? reinterpret_cast<const float*>(a.V)[vbase + m * T] : 0.f;
 
-  if (a.inverse_first) wfft_line<N, P, G, true>(v, t, a.tw, lline);
+  // a written-through field is addressed by 32 bits
+  const Buf buf(a.A);
+  auto put = [&]() {
+    if (!active) return;
+    if (a.through) {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int m = 0; m < P; ++m)
+          buf.store<ST_THROUGH>(v[g][m], 16u * (uint32_t)(off[g] + t), 16u * (uint32_t)(m * T));
+    } else {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int m = 0; m < P; ++m) a.A[off[g] + t + m * T] = v[g][m];
+    }
+  };
+
+  if (a.inverse_first) wfft_line<N, P, G, true, SYNC>(v, t, W, tw, lline);
 
   if (a.write_I) {
+    put();
     if (active) {
 #pragma unroll
       for (int g = 0; g < G; ++g)
 #pragma unroll
-        for (int m = 0; m < P; ++m) {
-          a.A[off[g] + t + m * T] = v[g][m];
-          a.I[off[g] + t + m * T] = v[g][m].x * v[g][m].x + v[g][m].y * v[g][m].y;
-        }
+        for (int m = 0; m < P; ++m) a.I[off[g] + t + m * T] = v[g][m].x * v[g][m].x + v[g][m].y * v[g][m].y;
     }
     return;
   }
 
   // nonlinear application with the records `nlp`: intensities from the
   // convolved buffer (nonlocal response) or |A|^2, V' rounded per record
-  const int64_t vbase = item * a.v_item_stride + y * N + t;
+  const bool has_vi = a.vkind == V_CPLX || a.vkind == V_CPLX128;
   auto nl_pass = [&](const void* nlp, bool use_ic) {
+    double I[G][P], vr[P], vi[P];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int m = 0; m < P; ++m) I[g][m] = v[g][m].x * v[g][m].x + v[g][m].y * v[g][m].y;
+    if (use_ic) {
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int m = 0; m < P; ++m) I[g][m] = a.Ic[off[g] + t + m * T];
+    }
     if constexpr (G == 1) {
       const WNL1 p = reinterpret_cast<const WNL1*>(nlp)[item];
-#pragma unroll
-      for (int m = 0; m < P; ++m) {
-        const double I = use_ic ? a.Ic[off[0] + t + m * T] : v[0][m].x * v[0][m].x + v[0][m].y * v[0][m].y;
-        v[0][m] = wnl1(v[0][m], I, p, a.loss_sat != 0, wvprime(a.V, a.vkind, vbase + m * T, p.vmul));
-      }
+      wvprime_set<P>(vr, vi, vf, a.V, a.vkind, vbase, T, p.vmul);
+      wnl1<P>(v[0], I[0], p, a.loss_sat != 0, vr, vi, has_vi);
     } else {
       const WNL2* pp = reinterpret_cast<const WNL2*>(nlp) + 2 * item;
-      const WNL2 p1 = pp[0], p2 = pp[1];
 #pragma unroll
-      for (int m = 0; m < P; ++m) {
-        double I1, I2;
-        if (use_ic) {
-          I1 = a.Ic[off[0] + t + m * T];
-          I2 = a.Ic[off[G - 1] + t + m * T];
-        } else {
-          I1 = v[0][m].x * v[0][m].x + v[0][m].y * v[0][m].y;
-          I2 = v[G - 1][m].x * v[G - 1][m].x + v[G - 1][m].y * v[G - 1][m].y;
-        }
-        v[0][m] = wnl2(v[0][m], I1, I2, p1, wvprime(a.V, a.vkind, vbase + m * T, p1.vmul));
-        v[G - 1][m] = wnl2(v[G - 1][m], I2, I1, p2, wvprime(a.V, a.vkind, vbase + m * T, p2.vmul));
+      for (int g = 0; g < 2; ++g) {
+        const WNL2 p = pp[g];
+        wvprime_set<P>(vr, vi, vf, a.V, a.vkind, vbase, T, p.vmul);
+        wnl2<P>(v[g], I[g], I[1 - g], p, vr, vi, has_vi);
       }
     }
   };
@@ -362,7 +435,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wrow(WRowArgs a) {
   // the second application (start of the next Strang step) always sees |A|^2
   if (a.has_b) nl_pass(a.nlp_b, false);
 
-  if (a.forward_last) wfft_line<N, P, G, false>(v, t, a.tw, lline);
+  if (a.forward_last) wfft_line<N, P, G, false, SYNC>(v, t, W, tw, lline);
 
   if (a.out_scale != 1.0) {
 #pragma unroll
@@ -370,12 +443,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wrow(WRowArgs a) {
 #pragma unroll
       for (int m = 0; m < P; ++m) v[g][m] = make_double2(v[g][m].x * a.out_scale, v[g][m].y * a.out_scale);
   }
-  if (active) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int m = 0; m < P; ++m) a.A[off[g] + t + m * T] = v[g][m];
-  }
+  put();
 }
 
 // ---------------------------------------------------------- column sweep
@@ -395,6 +463,7 @@ struct WColArgs {
   int nt;
   double scale;
   double out_scale;
+  int through;         // as in WRowArgs
 };
 
 // Columns of length N: WT adjacent columns per block, one per thread column.
@@ -420,7 +489,10 @@ __global__ __launch_bounds__(WT*(N / P)) void k_wcol(WColArgs a) {
 #pragma unroll
   for (int m = 0; m < P; ++m) v[0][m] = a.A[base + (int64_t)(t + m * T) * a.NX];
 
-  if (a.do_fwd) wfft_line<N, P, 1, false>(v, t, a.tw, lline);
+  const Buf tw(a.tw);
+  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
+
+  if (a.do_fwd) wfft_line<N, P, 1, false, SYNC_BLOCK>(v, t, W, tw, lline);
   if (a.do_prop) {
     const int comp = (int)(slab % a.ncomp);
     if (a.pkind == PROP_SEP64) {
@@ -460,13 +532,20 @@ __global__ __launch_bounds__(WT*(N / P)) void k_wcol(WColArgs a) {
       }
     }
   }
-  if (a.do_inv) wfft_line<N, P, 1, true>(v, t, a.tw, lline);
+  if (a.do_inv) wfft_line<N, P, 1, true, SYNC_BLOCK>(v, t, W, tw, lline);
   if (a.out_scale != 1.0) {
 #pragma unroll
     for (int m = 0; m < P; ++m) v[0][m] = make_double2(v[0][m].x * a.out_scale, v[0][m].y * a.out_scale);
   }
+  if (a.through) {
+    const Buf buf(a.A);
 #pragma unroll
-  for (int m = 0; m < P; ++m) a.A[base + (int64_t)(t + m * T) * a.NX] = v[0][m];
+    for (int m = 0; m < P; ++m)
+      buf.store<ST_THROUGH>(v[0][m], 16u * (uint32_t)(base + t * a.NX), 16u * (uint32_t)(m * T * a.NX));
+  } else {
+#pragma unroll
+    for (int m = 0; m < P; ++m) a.A[base + (int64_t)(t + m * T) * a.NX] = v[0][m];
+  }
 }
 
 // ------------------------------------------------- nonlocal response (2-D)
@@ -541,6 +620,15 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wline1d(WLine1DArgs a) {
 #pragma unroll
     for (int m = 0; m < P; ++m) pr[g][m] = a.prop[g * N + t + m * T];
 
+  constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
+  constexpr bool KEEP = G == 1 && twid_kept(N, P);  // two lines leave no registers for them
+  const Buf tw(a.tw);
+  const Twid<N, P, KEEP> W = load_twiddles<N, P, KEEP>(tw, t);
+  const bool has_vi = a.vkind == V_CPLX || a.vkind == V_CPLX128;
+  float vf[P];
+#pragma unroll
+  for (int m = 0; m < P; ++m) vf[m] = a.vkind == V_REAL ? reinterpret_cast<const float*>(a.V)[t + m * T] : 0.f;
+
   auto apply_nl = [&](const void* prm) {
     double I[G][P];
     if (a.nlk != nullptr) {
@@ -570,31 +658,31 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wline1d(WLine1DArgs a) {
 #pragma unroll
         for (int m = 0; m < P; ++m) I[g][m] = v[g][m].x * v[g][m].x + v[g][m].y * v[g][m].y;
     }
+    double vr[P], vi[P];
     if constexpr (G == 1) {
       const WNL1 p = reinterpret_cast<const WNL1*>(prm)[item];
-#pragma unroll
-      for (int m = 0; m < P; ++m)
-        v[0][m] = wnl1(v[0][m], I[0][m], p, a.loss_sat != 0, wvprime(a.V, a.vkind, t + m * T, p.vmul));
+      wvprime_set<P>(vr, vi, vf, a.V, a.vkind, t, T, p.vmul);
+      wnl1<P>(v[0], I[0], p, a.loss_sat != 0, vr, vi, has_vi);
     } else {
       const WNL2* pp = reinterpret_cast<const WNL2*>(prm) + 2 * item;
-      const WNL2 p1 = pp[0], p2 = pp[1];
 #pragma unroll
-      for (int m = 0; m < P; ++m) {
-        v[0][m] = wnl2(v[0][m], I[0][m], I[1][m], p1, wvprime(a.V, a.vkind, t + m * T, p1.vmul));
-        v[1][m] = wnl2(v[1][m], I[1][m], I[0][m], p2, wvprime(a.V, a.vkind, t + m * T, p2.vmul));
+      for (int g = 0; g < 2; ++g) {
+        const WNL2 p = pp[g];
+        wvprime_set<P>(vr, vi, vf, a.V, a.vkind, t, T, p.vmul);
+        wnl2<P>(v[g], I[g], I[1 - g], p, vr, vi, has_vi);
       }
     }
   };
 
   for (int64_t s = 0; s < a.nsteps; ++s) {
     if (a.precision == 1) apply_nl(a.nl_pre);
-    wfft_line<N, P, G, false>(v, t, a.tw, lline);
+    wfft_line<N, P, G, false, SYNC>(v, t, W, tw, lline);
 #pragma unroll
     for (int g = 0; g < G; ++g)
 #pragma unroll
       for (int m = 0; m < P; ++m)
         v[g][m] = wcmul(v[g][m], make_double2(pr[g][m].x * a.scale, pr[g][m].y * a.scale));
-    wfft_line<N, P, G, true>(v, t, a.tw, lline);
+    wfft_line<N, P, G, true, SYNC>(v, t, W, tw, lline);
     if (a.precision == 1) {
       apply_nl(a.nl_post);
     } else {
