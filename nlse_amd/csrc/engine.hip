@@ -755,6 +755,7 @@ struct nlse_plan {
   const double2* twt = nullptr;
   int row_points = 0;             // row kernels' set size (radix plan) if given, else chosen (row_p)
   bool small = false;             // small-field plans (SMALL_FIELD)
+  bool large = false;             // a stack of LARGE_STACK points
   bool through = false;           // sweeps write through (WRITE_THROUGH)
   bool cplx = false;              // any nonlinear record of a complex dz
   bool cplx_slot[3] = {false, false, false};
@@ -914,6 +915,7 @@ int nlse_plan_create(const nlse_plan_desc* d, nlse_plan** out) {
   }
   const int64_t points = d->items * d->ncomp * (d->ndim >= 2 ? d->ny : 1) * d->nx * (d->ndim == 3 ? d->nt : 1);
   p->small = d->ndim == 2 && points <= SMALL_FIELD;
+  p->large = d->ndim == 2 && d->ncomp == 1 && d->items > 1 && points >= LARGE_STACK;
   p->through = points * (p->wide ? 16 : 8) <= WRITE_THROUGH;
   if (d->row_points != 0) {
     const int pr = p->rops->p_row, pa = p->rops->p_row_alt, ps = p->rops->p_row_small;
@@ -930,7 +932,12 @@ int nlse_plan_create(const nlse_plan_desc* d, nlse_plan** out) {
     // block, or every second CU one of at most 256 threads (wider tiles read
     // longer row segments, see LineCfg::WDEF).  Local step at W = 8 / 4 / 2:
     // 1024^2 24.9 / 21.3 / - us, 512^2 - / 10.6 / 11.4 us, 256^2 10.6 / 8.3 /
-    // 7.8 us
+    // 7.8 us.  Columns of 1024 points and more in fields that are not written
+    // through take at most 4: the L2 joins the segments of neighbouring tiles
+    // (same XCD) before they leave it, and smaller blocks overlap better.
+    // Column sweep at W = 8 / 4: 8 x 1024^2 47.9 / 40.2 us, 28 x 1024^2 139 /
+    // 123, 2 x 2048^2 54.0 / 48.3, 6 x 2048^2 139 / 131 us; written through
+    // 4 x 1024^2 26.8 / 29.2, 2048^2 28.5 / 32.3 us
     int want = d->col_width;
     if (want == 0) {
       int dev = 0, cus = 256;
@@ -939,6 +946,7 @@ int nlse_plan_create(const nlse_plan_desc* d, nlse_plan** out) {
         cus = 256;
       const int64_t t = d->ny / (p->small ? p->cops->p_col_small : p->cops->p_col);
       want = p->cops->colw(d->nx, 0, p->small);
+      if (!p->through && d->ny >= 1024) want = std::min(want, 4);
       for (; want > 1; want >>= 1) {
         const int64_t blocks = d->items * d->ncomp * (d->nx / want);
         if (blocks >= cus || (2 * blocks >= cus && want * t <= 256)) break;
@@ -974,7 +982,8 @@ int nlse_plan_destroy(nlse_plan* p) {
 static int row_p(const nlse_plan* p) {
   if (p->wide) return 8;
   if (p->row_points) return p->row_points;
-  return p->small && !p->nlc.on ? p->rops->p_row_small : p->rops->p_row;
+  if (p->nlc.on) return p->rops->p_row;
+  return p->small ? p->rops->p_row_small : (p->large ? p->rops->p_row_large : p->rops->p_row);
 }
 
 int nlse_plan_config(const nlse_plan* p, int* row_points, int* col_width) {

@@ -20,9 +20,10 @@ namespace nlse {
 struct LineOps {
   int (*twiddles)(const double2**);
   // x rows (G = 1, or component pairs G = 2) with p points per thread: p_row
-  // by default, p_row_alt on request, p_row_small for small fields
+  // by default, p_row_alt on request, p_row_small for small fields, p_row_large
+  // for stacks of LARGE_STACK points
   int (*row)(int, int, const RowArgs&, hipStream_t);
-  int p_row, p_row_alt, p_row_small;
+  int p_row, p_row_alt, p_row_small, p_row_large;
   int (*line1d)(int, const Line1DArgs&, hipStream_t);
   int (*nlc)(int, const NlcArgs&, hipStream_t);
   // columns: tile width, small-field plan or not
@@ -134,6 +135,15 @@ constexpr int64_t SMALL_FIELD = 1 << 18;
 // 59.7 -> 56.4 us; 28 x 1024^2 (235 MB) 280 -> 298 us.
 constexpr int64_t WRITE_THROUGH = 48 << 20;
 
+// Stacks of one-component fields of at least this many points take p_row_large
+// in their row sweeps: 16 points per lane on 1024-point rows exchange once less
+// through LDS (24 instead of 32 bytes written per point and sweep), which pays
+// where enough waves hide one lane's longer chain.  Row sweep with 8 / 16
+// points: one 1024^2 field 8.9 / 10.8 us, 2 fields 13.8 / 12.6, 4 fields 21.6 /
+// 19.8, 28 fields 127 / 119 us (512-point rows: no difference).  A single field
+// keeps its plan whatever its size: an uneven batch computes it in that plan.
+constexpr int64_t LARGE_STACK = 1 << 21;
+
 template <int N>
 struct LineCfg {
   // column sweeps
@@ -147,6 +157,7 @@ struct LineCfg {
   // x rows
   static constexpr int PR = (N == 512 || N == 1024) ? 8 : P;
   static constexpr int PRS = N <= 256 ? 4 : PR;
+  static constexpr int PRL = N == 1024 ? 16 : PR;
   // nonlocal row kernels (one line pair per N/P threads, 128 per block)
   static constexpr int PZ = pick_p(N, NLSE_P8_FROM_NLZ, NLSE_P8_UPTO_NLZ);
   static constexpr int LPBZ = lines_per_block(128, N / PZ);
@@ -448,7 +459,7 @@ static int colu_launch(const ColArgs& a, hipStream_t s) {
 template <int N>
 LineOps make_ops() {
   using C = LineCfg<N>;
-  return LineOps{&get_twiddles<N>,  &row_launch<N>, C::PR,          row_p_alt<N>(), C::PRS,
+  return LineOps{&get_twiddles<N>,  &row_launch<N>, C::PR,          row_p_alt<N>(), C::PRS, C::PRL,
                  &line1d_launch<N>, &nlc_launch<N>, &col_launch<N>, &col_width_for<N>,
                  C::P,              C::PS,          &colz_band_launch<N>, &colu_launch<N>};
 }
