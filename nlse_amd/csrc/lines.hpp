@@ -97,28 +97,14 @@ static int get_twiddles(const double2** out) {
 }
 
 // -------------------------------------------------- kernel dispatchers
-// Points per thread (P) of each kernel kind and line length.  A smaller P puts
-// more lanes on a line (a shorter chain of instructions per lane, what a field
-// of few lines waits for), a larger P has fewer stages, i.e. fewer exchanges
-// and conversions.  Nonlocal row kernels (measured on MI355X): k_nlc_nl keeps
-// P = 8 at 2048 (26.7 vs 29.6 us); k_nlc_z P = 8 at 512 and 1024 only; at 512
-// both take P = 8.
-#ifndef NLSE_P8_FROM_NLZ
-#define NLSE_P8_FROM_NLZ 512
-#endif
-#ifndef NLSE_P8_UPTO_NLZ
-#define NLSE_P8_UPTO_NLZ 2048
-#endif
-#ifndef NLSE_P8_FROM_NLNL
-#define NLSE_P8_FROM_NLNL 512
-#endif
-#ifndef NLSE_P8_UPTO_NLNL
-#define NLSE_P8_UPTO_NLNL (1 << 30)
-#endif
-
-constexpr int pick_p(int n, int p8_from, int p8_upto) {
-  return n >= p8_from && n < p8_upto && n >= 8 ? 8 : (n >= 16 ? 16 : n);
-}
+// Points per thread (P) of the nonlocal row kernels.  A smaller P puts more
+// lanes on a line (a shorter chain of instructions per lane, what a field of
+// few lines waits for), a larger P has fewer stages, i.e. fewer exchanges and
+// conversions.  Nonlocal step with P = 4 / 8 / 16 in both kernels: 256^2 23.0 /
+// 25.8 / 31.5 us, 128^2 22.0 / 24.4 / 30.9, 256 fields of 256^2 309 / 307 / 313;
+// k_nlc_nl at 2048 points keeps 8 (26.7 against 29.6 us), k_nlc_z takes 16 there
+// (90.7 against 91.9 us a step).
+constexpr int pick_p(int n, int p8_upto) { return n <= 256 ? (n >= 32 ? 4 : 8) : (n < p8_upto ? 8 : 16); }
 constexpr int lines_per_block(int threads, int t) { return threads / t >= 1 ? threads / t : 1; }
 
 // Fields of at most this many points (all items and components) take the
@@ -158,11 +144,13 @@ struct LineCfg {
   static constexpr int PR = (N == 512 || N == 1024) ? 8 : P;
   static constexpr int PRS = N <= 256 ? 4 : PR;
   static constexpr int PRL = N == 1024 ? 16 : PR;
-  // nonlocal row kernels (one line pair per N/P threads, 128 per block)
-  static constexpr int PZ = pick_p(N, NLSE_P8_FROM_NLZ, NLSE_P8_UPTO_NLZ);
-  static constexpr int LPBZ = lines_per_block(128, N / PZ);
-  static constexpr int PN = pick_p(N, NLSE_P8_FROM_NLNL, NLSE_P8_UPTO_NLNL);
-  static constexpr int LPBN = lines_per_block(128, N / PN);
+  // nonlocal row kernels (a thread group per line pair); up to NLC_FEW points
+  // in the first lines of all pairs, lines of 512 and 1024 points take 4 per
+  // thread: nonlocal step with 8 / 4, 1024^2 42.8 / 40.3 us, 512^2 27.9 / 26.8,
+  // 4 fields of 512^2 39.8 / 39.1, 8 fields 53.4 / 55.8, 4 of 1024^2 92.9 / 96.7
+  static constexpr int PZ = pick_p(N, 2048);
+  static constexpr int PN = pick_p(N, 1 << 30);
+  static constexpr int64_t NLC_FEW = N == 512 || N == 1024 ? 1 << 19 : 0;
   // whole 1-D runs; up to LINES1S lines (or line pairs), which leave a CU one
   // or two lines, take the small plan: few points per lane, FP64 exchanges
   // up to 1024 points, twiddles kept.  Per step, default against small plan:
@@ -261,29 +249,41 @@ static int line1d_launch(int G, const Line1DArgs& a, hipStream_t s) {
 
 // Nonlocal line kernels: stage 1 (k_nlc_z) or stage 2 (k_nlc_nl), one
 // line pair per N/P threads.
+// (PZ, PN points per thread of k_nlc_z and k_nlc_nl, 128 threads per block)
+template <int N, int PZ, int PN>
+static void nlc_launch_p(int stage, const NlcArgs& a, hipStream_t s) {
+  const bool full = a.full && a.ncomp == 1;
+  if (stage == 1) {
+    constexpr int T = N / PZ, L = lines_per_block(128, T);
+    const int64_t blocks = (a.ngroups + L - 1) / L;
+    if (full)
+      hipLaunchKernelGGL((k_nlc_z<N, PZ, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_nlc_z<N, PZ, L>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+  } else {
+    constexpr int T = N / PN, L = lines_per_block(128, T);
+    const int64_t blocks = (a.ngroups + L - 1) / L;
+    if (full)
+      hipLaunchKernelGGL((k_nlc_nl<N, PN, L, 1, 1, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    else if (a.ncomp != 1)
+      hipLaunchKernelGGL((k_nlc_nl<N, PN, L, 2, 0, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    else if (a.general)
+      hipLaunchKernelGGL((k_nlc_nl<N, PN, L, 1, 0, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_nlc_nl<N, PN, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+  }
+}
+
 template <int N>
 static int nlc_launch(int stage, const NlcArgs& a, hipStream_t s) {
   using C = LineCfg<N>;
-  const bool full = a.full && a.ncomp == 1;
-  if (stage == 1) {
-    constexpr int L = C::LPBZ, T = N / C::PZ;
-    const int64_t blocks = (a.ngroups + L - 1) / L;
-    if (full)
-      hipLaunchKernelGGL((k_nlc_z<N, C::PZ, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-    else
-      hipLaunchKernelGGL((k_nlc_z<N, C::PZ, L>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-  } else {
-    constexpr int L = C::LPBN, T = N / C::PN;
-    const int64_t blocks = (a.ngroups + L - 1) / L;
-    if (full)
-      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1, 1, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-    else if (a.ncomp != 1)
-      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 2, 0, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-    else if (a.general)
-      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1, 0, true>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
-    else
-      hipLaunchKernelGGL((k_nlc_nl<N, C::PN, L, 1>), dim3((unsigned)blocks), dim3(L * T), 0, s, a);
+  if constexpr (C::NLC_FEW > 0) {
+    if ((int64_t)a.ngroups * N <= C::NLC_FEW) {
+      nlc_launch_p<N, 4, 4>(stage, a, s);
+      return launch_status(stage == 1 ? "k_nlc_z" : "k_nlc_nl");
+    }
   }
+  nlc_launch_p<N, C::PZ, C::PN>(stage, a, s);
   return launch_status(stage == 1 ? "k_nlc_z" : "k_nlc_nl");
 }
 
