@@ -247,8 +247,8 @@ typedef struct nlse_plan_desc {
   int64_t items;     /* leading (broadcast) items */
   int ncomp;         /* 1, or 2 for CNLSE / DDGPE layouts (..., 2, NY, NX) */
   int loss_saturates;
-  int row_points;    /* points per thread of the x-row kernels (radix plan): 0 = default,
-                        else the default or the alternative (8 <-> 16) set size */
+  int row_points;    /* points per thread of the x-row kernels (radix plan): 0 = default for
+                        the field's size, else 8 or 16 (or the small fields' own size) */
   int col_width;     /* 0 = default; columns per block of the column pass */
   int field_c128;    /* 1: the field is complex128 and is propagated in FP64 (a complex128
                         E_in keeps its precision, nlse.py:531-534); 0: complex64 */

@@ -76,13 +76,10 @@ struct BCol {
   static constexpr int W = 8192 / N;
   static constexpr int WT = THREADS / T < W ? THREADS / T : W;
   static constexpr int PASSES = W / WT;
-  static constexpr int LDSB = col_lds_size<N, WT, 1>() * (int)sizeof(xchg_t<AR>);
+  static constexpr int LDSB = col_lds_size<N, WT, 1, xchg_t<AR>>() * (int)sizeof(xchg_t<AR>);
   static_assert(WT * T == THREADS, "whole blocks");
 };
-#ifndef NLSE_BCOL_T
-#define NLSE_BCOL_T 256
-#endif
-constexpr int bcol_threads(int n) { return n >= 2048 ? 512 : NLSE_BCOL_T; }
+constexpr int bcol_threads(int n) { return n >= 2048 ? 512 : 256; }
 
 static bool batch_len_ok(int64_t n) { return n == 128 || n == 256 || n == 512 || n == 1024 || n == 2048; }
 

@@ -13,18 +13,18 @@
 // through LDS with one float2 of padding every 16 entries, which keeps the
 // b64 accesses of each 16-lane group on distinct banks.
 //
-// Arithmetic: each stage converts its R inputs to FP64, applies the stage
-// twiddles (FP64 records) and the radix-R butterfly in FP64, and rounds the
-// R outputs once to complex64 when it stores them (to LDS, or to the
-// natural set after the last stage).  On gfx950 an FP64 add, multiply or
-// FMA issues at the same rate as an FP32 one without packed math, so this
-// costs about what compensated FP32 butterflies cost (hi+lo constants and
-// twiddles), and it leaves one rounding per stage instead of one per
-// butterfly level.  The long split-step runs accumulate this rounding noise
-// as sqrt(steps), so fewer roundings per transform is what keeps a 2001-step
-// run close to an exactly rounded transform.  FP64 twiddles also remove the
-// systematic gain bias a table rounded to complex64 would add (a mean
-// |w|^2 - 1 of about -1e-8 per stage, -5e-8 per forward/inverse pair).
+// Arithmetic: each stage converts its R inputs to FP64, applies the radix-R
+// butterfly with its twiddles in FP64 (dft_fma), and rounds the R outputs once
+// to complex64 when it stores them (to LDS, or to the natural set after the last
+// stage); F64X transforms exchange FP64 and round once.  On gfx950 an FP64 add,
+// multiply or FMA issues at the same rate as an FP32 one without packed math, so
+// this costs no more than compensated FP32 butterflies, and it leaves one
+// rounding per stage instead of one per butterfly level.  The long split-step
+// runs accumulate this rounding noise as sqrt(steps), so fewer roundings per
+// transform is what keeps a 2001-step run close to an exactly rounded transform.
+// FP64 twiddles also remove the systematic gain bias a table rounded to
+// complex64 would add (a mean |w|^2 - 1 of about -1e-8 per stage, -5e-8 per
+// forward/inverse pair).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -134,6 +134,19 @@ struct Buf {
 template <int N, int PADSH, int EXTRA>
 struct LdsLine {
   static constexpr int SIZE = N + (N >> PADSH) + EXTRA + 1;
+};
+
+// Lines of a tile of WT columns (entries of type X, padded every 8): lanes go
+// over the columns first, and LDS serves the entries of 128 bytes at a time, so
+// the lines of a tile start 128 bytes / WT apart modulo 128.  32 bytes apart
+// whatever the tile, a 2048-point sweep of 8 columns counted 8192 clocks of
+// bank conflicts per CU, of which other waves hid most: 2048^2 nonlocal step
+// 92.6 -> 91.2 us, complex128 1024^2 37.2 -> 36.5, 2048^2 84.1 -> 82.6 us.
+template <int N, int WT, typename X>
+struct ColLine {
+  static constexpr int ENTRIES = 128 / (int)sizeof(X);
+  static constexpr int EXTRA = WT == 1 ? 0 : (WT < ENTRIES ? ENTRIES / WT - 1 : 0);
+  static constexpr int SIZE = LdsLine<N, 3, EXTRA>::SIZE;
 };
 
 template <int PADSH>

@@ -135,7 +135,6 @@ struct LineCfg {
   // column sweeps
   static constexpr int P = N >= 16 ? 16 : N;
   static constexpr int T = N / P;
-  static constexpr int LINE = LdsLine<N, 3, 3>::SIZE;  // column-pass lines
   // small fields: up to 256 points 4 per thread, FP64 exchanges (one rounding
   // per transform, so the extra stages round nothing); 512 points 8
   static constexpr int PS = N <= 256 ? 4 : (N == 512 ? 8 : P);
@@ -176,10 +175,12 @@ struct LineCfg {
 template <int N, int W, int PC, int AR>
 struct ColCfg {
   static constexpr int T = N / PC;
-  static constexpr int LINEB = LineCfg<N>::LINE * (int)sizeof(xchg_t<AR>);  // bytes of a line
-  static constexpr bool ONE = W * T <= 1024 && W * LINEB <= 150 * 1024;
+  template <int WTX>
+  static constexpr int lineb() { return ColLine<N, WTX, xchg_t<AR>>::SIZE * (int)sizeof(xchg_t<AR>); }
+  static constexpr bool ONE = W * T <= 1024 && W * lineb<W>() <= 150 * 1024;
   static constexpr int WTMAX = lines_per_block(512, T);
   static constexpr int WT = ONE || W < WTMAX ? W : WTMAX;
+  static constexpr int LINEB = lineb<WT>();  // bytes of a line
   static constexpr int G = W / WT;
   static constexpr int GRMAX = (150 * 1024) / (WT * LINEB);
   static constexpr int gr(int g) { return (g <= GRMAX || g == 1) ? g : gr(g / 2); }
@@ -382,7 +383,7 @@ static int colz_band_launch_wp(const ColArgs& c, const BandArgs& b, size_t band_
   constexpr int TPB = THREADS / (64 * BAND_WAVES);
   const int64_t ncol = c.nslabs * (c.NX / W);
   const int64_t nbb = (nband + TPB - 1) / TPB;
-  const size_t col_bytes = sizeof(float2) * (size_t)col_lds_size<N, WT, 1>();
+  const size_t col_bytes = sizeof(float2) * (size_t)col_lds_size<N, WT, 1, float2>();
   const size_t band_bytes = TPB * band_lds;
   const size_t bytes = col_bytes > band_bytes ? col_bytes : band_bytes;
   if (bytes > 160 * 1024) return 1;

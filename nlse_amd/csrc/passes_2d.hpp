@@ -31,7 +31,7 @@ struct RowArgs {
   float2* A;
   int64_t ngroups;        // rows (G=1) or row pairs (G=2)
   int64_t rows_per_item;  // NY: rows per item and component
-  const double2* tw;      // twiddles of the row length (FP64 records)
+  const double2* tw;      // twiddles of the row length (FP64 ratio pairs)
   int inverse_first;      // apply I_x (unnormalised) first
   int forward_last;       // apply F_x last
   int has_a;              // first nonlinear application (end of step k)
@@ -203,7 +203,7 @@ struct ColArgs {
   int64_t nslabs;      // items * components
   int NX;              // columns per slab
   int ncomp;           // propagator component = slab % ncomp
-  const double2* tw;   // twiddles of the column length (FP64 records)
+  const double2* tw;   // twiddles of the column length (FP64 ratio pairs)
   int do_fwd;          // F_y
   int do_prop;         // multiply by the propagator (with `scale`)
   int do_inv;          // I_y
@@ -225,12 +225,10 @@ struct ColArgs {
 // thread owning G columns (c0 + g*WT + cw) so that twiddles and the y
 // factor of the propagator are shared; LDS exchanges run in rounds of GR
 // columns per thread column.
-// LDS float2s of one column block: one float2 of padding every 8 entries
-// and 4 more per line, so the lines of the WT thread columns start 8
-// banks apart.
-template <int N, int WT, int GR>
+// LDS entries of one column block.
+template <int N, int WT, int GR, typename X>
 constexpr int col_lds_size() {
-  return WT * GR * LdsLine<N, 3, 3>::SIZE;
+  return WT * GR * ColLine<N, WT, X>::SIZE;
 }
 
 // The propagator on the natural sets w of G columns c0 + g*CS: complex64
@@ -300,7 +298,7 @@ template <int N, int P, int WT, int G, int GR, int PK = -1, int FA = F64>
 __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>* lds) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
-  constexpr int LINE = LdsLine<N, 3, 3>::SIZE;
+  constexpr int LINE = ColLine<N, WT, xchg_t<FA>>::SIZE;
   constexpr int TILE = WT * G;
 
   const int cw = threadIdx.x % WT;
@@ -425,7 +423,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
 // PK: the propagator kind compiled in (-1: any kind, chosen at run time).
 template <int N, int P, int WT, int G, int GR, int PK = -1, int FA = F64>
 __global__ __launch_bounds__(WT*(N / P)) void k_col(ColArgs a) {
-  __shared__ xchg_t<FA> lds[col_lds_size<N, WT, GR>()];
+  __shared__ xchg_t<FA> lds[col_lds_size<N, WT, GR, xchg_t<FA>>()];
   // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs,
   // so block b runs on XCD b % 8; give each XCD a contiguous range of
   // tiles so that the two 64-byte halves of a 128-byte line are fetched
@@ -451,10 +449,10 @@ template <int N, int P, int WT>
 __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
-  constexpr int LINE = LdsLine<N, 3, 3>::SIZE;
+  constexpr int LINE = ColLine<N, WT, float2>::SIZE;
   constexpr int H = P / 2;
   static_assert(H * T == N / 2, "the first half of a natural set covers rows [0, N/2)");
-  __shared__ float2 lds[col_lds_size<N, WT, 1>()];
+  __shared__ float2 lds[col_lds_size<N, WT, 1, float2>()];
   const int units = a.NX / 2 + 1;
   const int tiles = (units + WT - 1) / WT;
   const int64_t nblk = (int64_t)gridDim.x;

@@ -58,7 +58,7 @@ int wrow_launch(int G, const WRowArgs& a, hipStream_t s) {
 template <int N, int WT>
 int wcol_launch_w(const WColArgs& a, hipStream_t s) {
   constexpr int P = wp<N>(), T = N / P;
-  const size_t bytes = (size_t)WT * WLine<N>::SIZE * sizeof(double2);
+  const size_t bytes = (size_t)WT * ColLine<N, WT, double2>::SIZE * sizeof(double2);
   auto fn = k_wcol<N, P, WT>;
   int rc = lds_limit((const void*)fn, bytes);
   if (rc) return rc;

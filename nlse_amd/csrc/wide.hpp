@@ -471,7 +471,7 @@ template <int N, int P, int WT>
 __global__ __launch_bounds__(WT*(N / P)) void k_wcol(WColArgs a) {
   extern __shared__ double2 wsm[];
   constexpr int T = N / P;
-  constexpr int LINE = WLine<N>::SIZE;
+  constexpr int LINE = ColLine<N, WT, double2>::SIZE;
   const int cw = threadIdx.x % WT;
   const int t = threadIdx.x / WT;
   const int64_t tiles = a.NX / WT;
