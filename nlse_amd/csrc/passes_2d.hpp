@@ -458,42 +458,69 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
   const int64_t nblk = (int64_t)gridDim.x;
   const int64_t bb = (nblk % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8 : blockIdx.x;
   const int64_t slab = bb / tiles;
+  const int jt = (int)(bb % tiles) * WT;
+  const uint32_t nx = (uint32_t)a.NX;
   const int cw = threadIdx.x % WT;
   const int t = threadIdx.x / WT;
-  const int j0 = (int)(bb % tiles) * WT + cw;
-  const bool act = j0 < units;
-  const int j = act ? j0 : 0;
-  const int ca = j, cb = j == 0 ? 0 : a.NX - j;
-  float2* Z = a.A + slab * (int64_t)(N / 2) * a.NX;
+  // this thread's unit and the byte offsets of its two columns; found again
+  // after the transforms, which need every register of 1024-thread blocks
+  struct Unit {
+    int j;
+    bool act, two;
+    uint32_t da, db;
+  };
+  auto unit = [&]() {
+    const uint32_t id = opaque(threadIdx.x);
+    Unit u;
+    const int j0 = jt + (int)(id % WT);
+    u.act = j0 < units;
+    u.j = u.act ? j0 : 0;
+    const uint32_t cb = u.j == 0 ? 0u : nx - (uint32_t)u.j;
+    u.two = cb != (uint32_t)u.j;
+    u.da = 8u * (id / WT * nx + (uint32_t)u.j);
+    u.db = 8u * (id / WT * nx + cb);
+    return u;
+  };
   float2* lline = lds + cw * LINE;
-  const Buf tw(a.tw);
+  // (a slab of Z and the spectrum quadrant are far below 4 GiB)
+  const Buf Z(a.A + slab * (int64_t)(N / 2) * a.NX), kq(a.kq), tw(a.tw);
+  const uint32_t rs = 8u * (uint32_t)T * (uint32_t)a.NX;
   const Twid<N, P> W = load_twiddles<N, P>(tw, t);
 
   float2 v[1][P];
+  const Unit in = unit();
 #pragma unroll
   for (int m = 0; m < H; ++m) {
-    const int64_t row = (int64_t)(t + m * T) * a.NX;
-    const float2 za = Z[row + ca], zb = Z[row + cb];
+    const float2 za = Z.load<float2>(in.da, m * rs), zb = Z.load<float2>(in.db, m * rs);
     v[0][m] = make_float2(0.5f * (za.x + zb.x), 0.5f * (za.y - zb.y));
     v[0][m + H] = make_float2(0.5f * (za.y + zb.y), 0.5f * (zb.x - za.x));
   }
   fft_line<N, P, 1, false, 1, 3, F64>(v, t, W, tw, lline, LINE);
-  const int hx = a.NX / 2 + 1;
+  const int hx = a.NX / 2 + 1, jq = unit().j, tq = (int)(opaque(threadIdx.x) / WT);
 #pragma unroll
   for (int m = 0; m < P; ++m) {
-    const int ky = t + m * T;
+    const int ky = tq + m * T;
     const int kyq = ky <= N / 2 ? ky : N - ky;
-    const float f = a.kq[kyq * hx + j] * a.scale;
+    const float f = kq.load<float>(4u * (uint32_t)(kyq * hx + jq), 0) * a.scale;
     v[0][m] = make_float2(v[0][m].x * f, v[0][m].y * f);
   }
   fft_line<N, P, 1, true, 1, 3, F64>(v, t, W, tw, lline, LINE);
-  if (act) {
+  // the results are rounded before the branches (else the last stage's FP64
+  // values are kept through them, and spill)
 #pragma unroll
-    for (int m = 0; m < H; ++m) {
-      const int64_t row = (int64_t)(t + m * T) * a.NX;
-      const float2 yt = v[0][m], yb = v[0][m + H];
-      Z[row + ca] = make_float2(yt.x - yb.y, yt.y + yb.x);
-      if (cb != ca) Z[row + cb] = make_float2(yt.x + yb.y, yb.x - yt.y);
+  for (int m = 0; m < P; ++m) {
+    v[0][m].x = __builtin_bit_cast(float, opaque(__builtin_bit_cast(uint32_t, v[0][m].x)));
+    v[0][m].y = __builtin_bit_cast(float, opaque(__builtin_bit_cast(uint32_t, v[0][m].y)));
+  }
+  const Unit out = unit();
+  if (out.act) {
+#pragma unroll
+    for (int m = 0; m < H; ++m)
+      Z.store(make_float2(v[0][m].x - v[0][m + H].y, v[0][m].y + v[0][m + H].x), out.da, m * rs);
+    if (out.two) {
+#pragma unroll
+      for (int m = 0; m < H; ++m)
+        Z.store(make_float2(v[0][m].x + v[0][m + H].y, v[0][m + H].x - v[0][m].y), out.db, m * rs);
     }
   }
 }

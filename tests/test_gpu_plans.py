@@ -161,7 +161,7 @@ def test_line_pair_counts(gpu, nx, lead):
 
 # nonlocal row kernels: 4 points per lane up to 256-point lines, and up to 2^19
 # points of pairs at 512 and 1024
-@pytest.mark.parametrize("lead,ny,nx", [((), 16, 32), ((), 64, 128), ((3,), 128, 256), ((4,), 512, 512),
+@pytest.mark.parametrize("lead,ny,nx", [((), 64, 16), ((), 16, 32), ((), 64, 128), ((3,), 128, 256), ((4,), 512, 512),
                                         ((5,), 512, 512), ((), 1024, 1024), ((2,), 1024, 1024), ((), 64, 2048)])
 def test_nonlocal_row_plans(gpu, lead, ny, nx):
     g, o = _pair("NLSE", _material(nx, ny, nl_length=1.6 * window / nx),
