@@ -171,24 +171,37 @@ __device__ __forceinline__ void wsincos_small(double x, double& s, double& c) {
 }
 
 // The same on P points with one choice of the evaluation for the wave: the
-// series for half phases up to pi/4 and losses up to 1/8 (about 45 operations
-// a point, 35 where one loss serves all points, against some 250 of the library
-// functions).
+// series for phases up to 2^16 (reduced by multiples of pi where one of the wave
+// passes pi/2) and losses up to 1/8: about 45 operations a point, 35 where one
+// loss serves all points, against some 250 of the library functions.
 template <int P>
 __device__ __forceinline__ void wapply(double2 (&A)[P], const double (&a)[P], bool one_loss, const double (&th)[P]) {
-  bool small = true;
+  bool small = true, series = true;
 #pragma unroll
-  for (int m = 0; m < P; ++m) small = small && fabs(th[m]) <= 1.5707963267948966 && fabs(a[m]) <= 0.125;
-  if (wave_all(small)) {
+  for (int m = 0; m < P; ++m) {
+    small = small && fabs(th[m]) <= 1.5707963267948966;
+    series = series && fabs(th[m]) <= 65536.0 && fabs(a[m]) <= 0.125;
+  }
+  if (wave_all(series)) {
+    const bool reduce = !wave_all(small);
     double em = wexpm1_small(-a[0]);
 #pragma unroll
     for (int m = 0; m < P; ++m) {
       if (m > 0 && !one_loss) em = wexpm1_small(-a[m]);
-      double s2, c2;
-      wsincos_small(0.5 * th[m], s2, c2);
-      const double cosm1 = -2.0 * s2 * s2;
+      // half phase h = n pi/2 + r: sin^2 h and sin h cos h are sin^2 r and
+      // sin r cos r for even n, cos^2 r and -sin r cos r for odd n
+      double h = 0.5 * th[m], s2, c2;
+      bool odd = false;
+      if (reduce) {
+        const double n = rint(h * 0.63661977236758138);
+        h = fma(-n, 6.123233995736766e-17, fma(-n, 1.5707963267948966, h));
+        odd = ((int)n & 1) != 0;
+      }
+      wsincos_small(h, s2, c2);
+      const double q = odd ? c2 : s2, r = odd ? -s2 : c2;
+      const double cosm1 = -2.0 * q * q;
       const double dr = fma(em, 1.0 + cosm1, cosm1);
-      const double di = (1.0 + em) * (2.0 * s2 * c2);
+      const double di = (1.0 + em) * (2.0 * q * r);
       A[m] = make_double2(A[m].x + fma(A[m].x, dr, -A[m].y * di), A[m].y + fma(A[m].y, dr, A[m].x * di));
     }
   } else {
@@ -336,7 +349,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wrow(WRowArgs a) {
   }
   double2* lline = wsm + li * G * LINE;
   constexpr int SYNC = T <= 64 ? SYNC_WAVE : SYNC_BLOCK;
-  constexpr bool KEEP = G == 1 && twid_kept(N, P);  // two lines leave no registers for them
+  constexpr bool KEEP = false;  // kept, they take 40 more VGPRs for 2 % at 256^2 and nothing beyond
 
   double2 v[G][P];
 #pragma unroll
@@ -490,7 +503,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_wcol(WColArgs a) {
   for (int m = 0; m < P; ++m) v[0][m] = a.A[base + (int64_t)(t + m * T) * a.NX];
 
   const Buf tw(a.tw);
-  const Twid<N, P> W = load_twiddles<N, P>(tw, t);
+  const Twid<N, P, false> W = load_twiddles<N, P, false>(tw, t);
 
   if (a.do_fwd) wfft_line<N, P, 1, false, SYNC_BLOCK>(v, t, W, tw, lline);
   if (a.do_prop) {
