@@ -56,20 +56,34 @@ struct RabiParams {
   float cm1_i = 0.f, sn_i = 0.f;  // imaginary parts
 };
 
-// sin and cos of h, |h| <= pi/4: Taylor series (coefficients 1/n!)
-// truncated where the remainder is below 2^-28 relative (sin to x^11,
-// cos to x^12 would be the next terms: 0.785^11/11! = 1.8e-9).
+// sin and cos of h, |h| <= pi/4: polynomials of least largest error (6e-11 and
+// 6e-12; each coefficient rounded to FP32 before the next ones were fitted, so
+// that these make up for it).  With the Taylor coefficients the mean of |f|^2 - 1
+// is -1.5e-9 at phases near pi/2, with these -1e-10.
 __device__ __forceinline__ void sincos_small(float h, float& s, float& c) {
   const float x2 = h * h;
-  float ps = fmaf(x2, 2.75573192e-6f, -1.98412698e-4f);  // 1/9!, -1/7!
-  ps = fmaf(x2, ps, 8.33333333e-3f);                      // 1/5!
-  ps = fmaf(x2, ps, -1.66666667e-1f);                     // -1/3!
+  float ps = fmaf(x2, 2.80394079e-6f, -1.98502734e-4f);
+  ps = fmaf(x2, ps, 8.33337288e-3f);
+  ps = fmaf(x2, ps, -1.66666672e-1f);
   s = fmaf(h * x2, ps, h);
-  float pc = fmaf(x2, -2.75573192e-7f, 2.48015873e-5f);   // -1/10!, 1/8!
-  pc = fmaf(x2, pc, -1.38888889e-3f);                     // -1/6!
-  pc = fmaf(x2, pc, 4.16666667e-2f);                      // 1/4!
-  pc = fmaf(x2, pc, -0.5f);                               // -1/2!
+  float pc = fmaf(x2, -2.89776466e-7f, 2.48229862e-5f);
+  pc = fmaf(x2, pc, -1.38889824e-3f);
+  pc = fmaf(x2, pc, 4.16666679e-2f);
+  pc = fmaf(x2, pc, -0.5f);
   c = fmaf(x2, pc, 1.0f);
+}
+
+// q and r with sin^2 h = q^2 and sin h cos h = q r, |h| <= 2^15: h = n pi/2 + x
+// in two FMAs (the first is exact), q = sin x and r = cos x for even n, q = cos x
+// and r = -sin x for odd n.
+__device__ __forceinline__ void sincos_reduced(float h, float& q, float& r) {
+  const float n = rintf(h * 0.636619772f);
+  const float x = fmaf(-n, -4.37113901e-8f, fmaf(-n, 1.57079637f, h));
+  float s, c;
+  sincos_small(x, s, c);
+  const bool odd = ((int)n & 1) != 0;
+  q = odd ? c : s;
+  r = odd ? -s : c;
 }
 
 // expm1(x), |x| <= 1/8: Taylor series to x^7 (remainder 0.125^8/8! < 2e-12).
@@ -81,6 +95,26 @@ __device__ __forceinline__ float expm1_small(float x) {
   p = fmaf(x, p, 0.5f);                                // 1/2!
   return fmaf(x * x, p, x);
 }
+
+// expm1(x), |x| <= 80: x = n ln 2 + y in two FMAs (the first is exact), 2^n
+// (expm1(y) + 1) - 1 with the Taylor series of y to y^8 (remainder 0.35^9/9! =
+// 2e-10).
+__device__ __forceinline__ float expm1_reduced(float x) {
+  const float n = rintf(x * 1.44269504f);
+  const float y = fmaf(-n, -1.90465432e-9f, fmaf(-n, 0.693147182f, x));
+  float p = fmaf(y, 2.48015873e-5f, 1.98412698e-4f);  // 1/8!, 1/7!
+  p = fmaf(y, p, 1.38888889e-3f);
+  p = fmaf(y, p, 8.33333333e-3f);
+  p = fmaf(y, p, 4.16666667e-2f);
+  p = fmaf(y, p, 1.66666667e-1f);
+  p = fmaf(y, p, 0.5f);
+  p = fmaf(y * y, p, y);
+  const float e = ldexpf(1.0f, (int)n);
+  return fmaf(e, p, e - 1.0f);
+}
+
+// Ranges of the reduced forms; beyond them (and for NaN) the library functions.
+constexpr float PHASE_REDUCED = 65536.0f, LOSS_REDUCED = 80.0f;
 
 // 1/d to ~1 ulp: hardware reciprocal and one Newton step; exact for d = 1.
 __device__ __forceinline__ float recip(float d) {
@@ -94,9 +128,9 @@ __device__ __forceinline__ bool wave_all(bool c) {
 __device__ __forceinline__ bool wave_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 
 // A *= exp(-a + i th) for n points {Re A, Im A, a, th} in private memory with
-// the library functions, for arguments outside the series' ranges.  Out of
-// line and on a copy of the points: rarely taken, and a call amid the points
-// would tie up the registers of the common path.
+// the library functions, for arguments outside the ranges of the forms above.
+// Out of line and on a copy of the points: such phases of complex64 fields hold
+// no digits, and a call amid the points would tie up the registers of the others.
 typedef __attribute__((address_space(5))) float private_float;
 __device__ __noinline__ void phase_loss_lib(private_float* p, int n) {
   for (int m = 0; m < n; ++m) {
@@ -129,25 +163,40 @@ __device__ __forceinline__ void phase_loss_slow(float2* A, const float* a, int a
   for (int m = 0; m < P; ++m) A[m] = make_float2(pts[4 * m], pts[4 * m + 1]);
 }
 
+// A *= 1 + em + ..., the factor f = exp(-a + i theta) as A + A (f - 1), from em =
+// expm1(-a) and q, r of the half phase.
+__device__ __forceinline__ float2 apply_half_phase(float2 A, float em, float q, float r) {
+  const float cosm1 = -2.0f * q * q;
+  const float dr = fmaf(em, 1.0f + cosm1, cosm1);
+  const float di = (1.0f + em) * (2.0f * q * r);
+  const float cx = fmaf(A.x, dr, -A.y * di);
+  const float cy = fmaf(A.y, dr, A.x * di);
+  return make_float2(A.x + cx, A.y + cy);
+}
+
 // Apply exp(-a + i theta) to P points with one wave-uniform choice of the
 // evaluation path for all of them.
 template <int P>
 __device__ __forceinline__ void apply_phase_loss_block(float2* A, const float* a, const float* theta) {
-  bool small = true;
+  bool small = true, reduced = true;
 #pragma unroll
-  for (int m = 0; m < P; ++m) small = small && fabsf(0.5f * theta[m]) <= 0.78539816f && fabsf(a[m]) <= 0.125f;
+  for (int m = 0; m < P; ++m) {
+    small = small && fabsf(0.5f * theta[m]) <= 0.78539816f && fabsf(a[m]) <= 0.125f;
+    reduced = reduced && fabsf(theta[m]) <= PHASE_REDUCED && fabsf(a[m]) <= LOSS_REDUCED;
+  }
   if (wave_all(small)) {
 #pragma unroll
     for (int m = 0; m < P; ++m) {
       float s2, c2;
-      const float em = expm1_small(-a[m]);
       sincos_small(0.5f * theta[m], s2, c2);
-      const float cosm1 = -2.0f * s2 * s2;
-      const float dr = fmaf(em, 1.0f + cosm1, cosm1);
-      const float di = (1.0f + em) * (2.0f * s2 * c2);
-      const float cx = fmaf(A[m].x, dr, -A[m].y * di);
-      const float cy = fmaf(A[m].y, dr, A[m].x * di);
-      A[m] = make_float2(A[m].x + cx, A[m].y + cy);
+      A[m] = apply_half_phase(A[m], expm1_small(-a[m]), s2, c2);
+    }
+  } else if (wave_all(reduced)) {
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      float q, r;
+      sincos_reduced(0.5f * theta[m], q, r);
+      A[m] = apply_half_phase(A[m], expm1_reduced(-a[m]), q, r);
     }
   } else {
     phase_loss_slow<P>(A, a, 1, theta);
@@ -179,14 +228,19 @@ __device__ __forceinline__ void sincosm1_quarter(float x, float& s, float& cm1) 
 // A *= exp(-a + i th[m]) on P points with one loss `a` for all of them:
 // e^{-a} - 1 is evaluated once, and steps of small phase (the wave's largest
 // |th| <= 1/4) take the short series: about 18 operations per point against
-// 38 of apply_phase_loss_block.
+// 38 of apply_phase_loss_block.  Phases past pi/2 and losses past 1/8 are reduced
+// in registers.  By the library on a copy of the wave's points in private memory,
+// 20 steps of 28 fields of 1024^2 with phases of 1.7 took 9.1 ms, and with the
+// library inlined 7.8; now 5.4 (5.3 with small phases).  The power changed by up to
+// 6e-8 a step, now 5e-11.
 template <int P>
 __device__ __forceinline__ void apply_phase_block(float2* A, float a, const float* th) {
-  bool quarter = fabsf(a) <= 0.125f, half = quarter;
+  bool quarter = fabsf(a) <= 0.125f, half = quarter, reduced = fabsf(a) <= LOSS_REDUCED;
 #pragma unroll
   for (int m = 0; m < P; ++m) {
     quarter = quarter && fabsf(th[m]) <= 0.25f;
     half = half && fabsf(th[m]) <= 1.5707963f;
+    reduced = reduced && fabsf(th[m]) <= PHASE_REDUCED;
   }
   const float em = expm1_small(-a), e1 = 1.0f + em;
   if (wave_all(quarter)) {
@@ -205,6 +259,14 @@ __device__ __forceinline__ void apply_phase_block(float2* A, float a, const floa
       const float cm1 = -2.0f * s2 * s2;
       const float dr = fmaf(e1, cm1, em), di = e1 * (2.0f * s2 * c2);
       A[m] = make_float2(A[m].x + fmaf(A[m].x, dr, -A[m].y * di), A[m].y + fmaf(A[m].y, dr, A[m].x * di));
+    }
+  } else if (wave_all(reduced)) {
+    const float emr = expm1_reduced(-a);
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      float q, r;
+      sincos_reduced(0.5f * th[m], q, r);
+      A[m] = apply_half_phase(A[m], emr, q, r);
     }
   } else {
     phase_loss_slow<P>(A, &a, 0, th);
