@@ -456,7 +456,11 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
     for (int64_t y = 0; y < it.ny; y += lpb) rows_n[len_index(it.nx, I.small)].push_back(BatchUnit{(int)i, 0, y});
     for (int64_t t = 0; t < it.nx / w; ++t) cols_n[len_index(it.ny, I.small)].push_back(BatchUnit{(int)i, 0, t});
   }
-  for (BatchInst& I : b->h_inst) I.row.through = I.col.through = total * 8 <= WRITE_THROUGH;
+  // both sweeps, tiles of 4 columns among them, go through up to WRITE_THROUGH.
+  // Both through / both back / rows through and columns back, a step: 60 fields of
+  // 256^2 (31 MB) 45 / 47 / 52 us, 3 of 2048 x 512 43 / 44 / 46, 20 of 512^2 54 / 52
+  // / 53, 2048^2 55 / 52 / 53
+  for (BatchInst& I : b->h_inst) I.row.through = I.col.through = total * 8 <= WRITE_THROUGH ? 2 : 0;
   std::vector<BatchUnit> rows, cols;
   for (int li = 0; li < NLEN; ++li) {
     b->row_off[li] = (int64_t)rows.size();

@@ -756,7 +756,7 @@ struct nlse_plan {
   int row_points = 0;             // row kernels' set size (radix plan) if given, else chosen (row_p)
   bool small = false;             // small-field plans (SMALL_FIELD)
   bool large = false;             // a stack of LARGE_STACK points
-  bool through = false;           // sweeps write through (WRITE_THROUGH)
+  int through = 0;                // level of the field's stores (through_level)
   bool cplx = false;              // any nonlinear record of a complex dz
   bool cplx_slot[3] = {false, false, false};
   int colw = 1;                   // y-column tile
@@ -916,7 +916,7 @@ int nlse_plan_create(const nlse_plan_desc* d, nlse_plan** out) {
   const int64_t points = d->items * d->ncomp * (d->ndim >= 2 ? d->ny : 1) * d->nx * (d->ndim == 3 ? d->nt : 1);
   p->small = d->ndim == 2 && points <= SMALL_FIELD;
   p->large = d->ndim == 2 && d->ncomp == 1 && d->items > 1 && points >= LARGE_STACK;
-  p->through = points * (p->wide ? 16 : 8) <= WRITE_THROUGH;
+  p->through = through_level(points * 8);
   if (d->row_points != 0) {
     const int pr = p->rops->p_row, pa = p->rops->p_row_alt, ps = p->rops->p_row_small;
     const bool ok = d->row_points == pr || (d->ndim != 1 && (d->row_points == pa || (p->small && d->row_points == ps)));

@@ -81,8 +81,10 @@ struct Plan {
 };
 
 // Stores kept in the L2 until the kernel's end, or written through to memory
-// (sc1) while the kernel runs.
+// (sc1) while the kernel runs: if the field's level (through_level) reaches what
+// lanes that store `bytes` contiguous bytes need.
 enum : int { ST_BACK = 0, ST_THROUGH = 16 };
+constexpr int through_need(int bytes) { return bytes >= 64 ? 1 : (bytes >= 16 ? 2 : 3); }
 
 // Memory seen from a uniform address: a buffer descriptor in scalar registers.
 // An access is one instruction at a per-lane 32-bit byte offset plus a uniform

@@ -119,7 +119,19 @@ constexpr int64_t SMALL_FIELD = 1 << 18;
 // whose reads come from other XCDs, may start.  Step of a local field, stores
 // back / through: 1024^2 25.2 -> 21.0 us, 2 x 1024^2 46.2 -> 31.8 us, 2048^2
 // 59.7 -> 56.4 us; 28 x 1024^2 (235 MB) 280 -> 298 us.
-constexpr int64_t WRITE_THROUGH = 48 << 20;
+// Stores of fewer contiguous bytes than a line leave in as many pieces: 64 bytes
+// (rows of 8 lanes, tiles of 8 columns) go through up to WRITE_THROUGH, 16 and 32
+// up to WRITE_THROUGH_NARROW, single points never.  Whole calls with all stores
+// back / through / by this rule: 8-byte rows, 3-D 512 x 512 x 16 2.74 / 3.43 / 2.65
+// ms, 200 fields of 256 x 16 2.38 / 2.60 / 2.13; 8-byte columns, 4096 x 64 2.02 /
+// 2.73 / 2.01, 4096 x 256 3.20 / 3.58 / 2.86; 16-byte rows, 512 x 256 x 32 (32 MiB)
+// 2.29 / 2.62 / 2.25; 32-byte columns, 16 of 4096 x 64 (32 MiB) 4.63 / 5.74 / 4.63,
+// 1024^2 (8 MiB) 25.2 / 21.0 / 21.0 us a step; 16-byte columns, cnlse 4096 x 256 (16
+// MiB) 3.16 / 3.05 / 3.05.
+constexpr int64_t WRITE_THROUGH = 48 << 20, WRITE_THROUGH_NARROW = 16 << 20;
+constexpr int through_level(int64_t bytes) {
+  return bytes <= WRITE_THROUGH_NARROW ? 2 : (bytes <= WRITE_THROUGH ? 1 : 0);
+}
 
 // Stacks of one-component fields of at least this many points take p_row_large
 // in their row sweeps: 16 points per lane on 1024-point rows exchange once less

@@ -54,7 +54,7 @@ struct NlcArgs {
   float drv_dz;
   float out_scale;
   int general;            // the loss varies from point to point (see nl1_block_I)
-  int through;            // write the results through to memory (ST_THROUGH)
+  int through;            // level of the field's stores (through_level)
   // band values of the convolved intensity
   const int* rowmap;      // [NY] band row index, or -1
   const float* rowband;   // [slabs][nb][NX]
@@ -107,8 +107,8 @@ __device__ __forceinline__ NlcLines nlc_lines(const NlcArgs& a, uint32_t g0, uin
 
 // Store a natural set at lane offset d, uniform offset u (bytes).
 template <int P, int T>
-__device__ __forceinline__ void put_line(const Buf& B, const float2 (&v)[P], uint32_t d, uint32_t u, bool through) {
-  if (through) {
+__device__ __forceinline__ void put_line(const Buf& B, const float2 (&v)[P], uint32_t d, uint32_t u, int through) {
+  if (through >= through_need(8 * T)) {
 #pragma unroll
     for (int m = 0; m < P; ++m) B.store<ST_THROUGH>(v[m], d, u + 8u * m * T);
   } else {

@@ -53,7 +53,7 @@ struct RowArgs {
   float drv_dz;
   float out_scale;        // applied to the stored result (1 or 1/N)
   int general;            // the loss varies from point to point (see nl1_block_I)
-  int through;            // write the result through to memory (ST_THROUGH)
+  int through;            // level of the field's stores (through_level)
 };
 
 // LDS entries of one row block.
@@ -178,7 +178,7 @@ __device__ __forceinline__ void row_body(const RowArgs& a, int64_t g0, xchg_t<AR
       for (int m = 0; m < P; ++m) v[g][m] = make_float2(v[g][m].x * a.out_scale, v[g][m].y * a.out_scale);
   }
   if (active) {
-    if (a.through) {
+    if (a.through >= through_need(8 * T)) {
 #pragma unroll
       for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -217,7 +217,7 @@ struct ColArgs {
   int nt;              // columns = NX * NT for PROP_SEP3D
   float scale;         // 1/(NX NY) folded into the propagator
   float out_scale;     // applied to the stored result when no propagator
-  int through;         // write the result through to memory (ST_THROUGH)
+  int through;         // level of the field's stores (through_level)
 };
 
 // Column sweep.  A block covers W = WT*G adjacent columns of one slab:
@@ -416,7 +416,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
       }
     }
   };
-  if (!WIDE && a.through) put(std::integral_constant<int, ST_THROUGH>{});
+  if (!WIDE && a.through >= through_need(8 * TILE)) put(std::integral_constant<int, ST_THROUGH>{});
   else put(std::integral_constant<int, ST_BACK>{});
 }
 

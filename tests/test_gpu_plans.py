@@ -208,3 +208,25 @@ def test_complex128_plans(gpu, vdtype, lead, ny, nx):
     err = rel_l2(g.out_field(E, 2.5 * DZ, precision="double", verbose=False), o.out_field(E, 2.5 * DZ, "double"))
     print(vdtype, lead, ny, nx, f"{err:.2e}")
     assert err < C128
+
+
+# stores of 8, 16, 32 and 64 contiguous bytes a row (lines of 16 to 128 points,
+# tiles of 1 to 8 columns) in stacks on both sides of 16 and 48 MiB: what decides
+# between stores back and through changes no bit.  All stacks have more points
+# than the small-field plans, and the same row sets
+@pytest.mark.parametrize("comp", [1, 2])
+@pytest.mark.parametrize("ny,nx,counts", [(256, 16, (80, 640, 1540)), (256, 32, (40, 320, 770)), (128, 64, (40, 320, 770)),
+                                          (64, 128, (40, 320, 770)), (4096, 8, (10, 80, 193))])
+def test_stores_back_or_through(gpu, ny, nx, counts, comp):
+    name, kw = ("NLSE", _material(nx, ny)) if comp == 1 else ("CNLSE", _material(nx, ny, n12=-3e-10))
+    E = _beam((2,) if comp == 2 else (), ny, nx, ny)
+    scale = np.linspace(0.5, 1.0, counts[-1], dtype=np.float32).reshape((-1,) + (1,) * E.ndim)
+    ref = None
+    for k in counts:
+        g, o = _pair(name, kw)
+        out = g.out_field(E * scale[:k], 1.5 * DZ, normalize=False, verbose=False)
+        if ref is None:
+            ref = out[:3]
+            want = o.out_field(E * scale[:3], 1.5 * DZ, normalize=False)
+            assert rel_l2(ref, want) < C64
+        assert np.array_equal(out[:3], ref), k
