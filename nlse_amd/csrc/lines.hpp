@@ -300,11 +300,24 @@ static int nlc_launch(int stage, const NlcArgs& a, hipStream_t s) {
   return launch_status(stage == 1 ? "k_nlc_z" : "k_nlc_nl");
 }
 
-template <int N, int W, int PK, int PC, int AR>
+// The default tile: at most the widest of one column per thread (4096^2, tile of 8
+// columns, four per thread, against 4: column sweep 144 -> 131 us).
+template <int N>
+constexpr int col_width_default() {
+  int w = LineCfg<N>::WDEF;
+  while (w > 1 && w * LineCfg<N>::T > 1024) w /= 2;
+  return w;
+}
+
+// Slabs past the reach of 32-bit offsets have instances for the default tile alone.
+constexpr bool big_slab(int64_t n, int64_t ncols) { return n * ncols * 8 > (int64_t)0xffffffff; }
+
+template <int N, int W, int PK, int PC, int AR, bool BIG = false>
 static void col_launch_k(const ColArgs& a, hipStream_t s) {
   using K = ColCfg<N, W, PC, AR>;
   const int64_t blocks = a.nslabs * (a.NX / W);
-  hipLaunchKernelGGL((k_col<N, PC, K::WT, K::G, K::GR, PK, AR>), dim3((unsigned)blocks), dim3(K::WT * K::T), 0, s, a);
+  hipLaunchKernelGGL((k_col<N, PC, K::WT, K::G, K::GR, PK, AR, BIG>), dim3((unsigned)blocks), dim3(K::WT * K::T), 0, s,
+                     a);
 }
 
 template <int N, int W>
@@ -318,23 +331,33 @@ static bool col_launch_w(bool small, const ColArgs& a, hipStream_t s) {
     }
   }
   if constexpr (ColCfg<N, W, C::P, F64>::OK) {
-    // the separable 2-D and 3-D propagators, the real kernel spectrum of
-    // the nonlocal response and the propagator-free transforms get their
-    // own instances (fewer live registers than the run-time dispatch over
-    // every kind); slabs of 4 GiB and more take the PK = -1 instance
-    const bool prop = a.do_prop != 0;
-    const bool big = (int64_t)N * a.NX * 8 > (int64_t)0xffffffff;
-    if (big || (prop && a.pkind != PROP_SEP64 && a.pkind != PROP_KREAL && a.pkind != PROP_SEP3D))
-      col_launch_k<N, W, -1, C::P, F64>(a, s);
-    else if (!prop)
-      col_launch_k<N, W, PK_NONE, C::P, F64>(a, s);
-    else if (a.pkind == PROP_SEP64)
-      col_launch_k<N, W, PROP_SEP64, C::P, F64>(a, s);
-    else if (a.pkind == PROP_KREAL)
-      col_launch_k<N, W, PROP_KREAL, C::P, F64>(a, s);
-    else
-      col_launch_k<N, W, PROP_SEP3D, C::P, F64>(a, s);
-    return true;
+    // one instance per propagator kind (fewer live registers than a run-time
+    // dispatch).  Step with a dense complex64 table, by a dispatch over all kinds
+    // (228 VGPRs, or scratch in blocks of 1024 threads) / by its instance (104):
+    // 2048^2 58.4 / 50.6 us, 4096^2 231 / 203, two components of 1024^2 35.6 / 31.5,
+    // tiles of 16 columns at 2048^2 109 / 84 (107 before addresses by 64 bits)
+    constexpr int P = C::P;
+    const int kind = a.do_prop ? a.pkind : PK_NONE;
+    if constexpr (W == col_width_default<N>()) {
+      // of 3-D fields only
+      if (big_slab(N, a.NX)) {
+        switch (kind) {
+          case PK_NONE: col_launch_k<N, W, PK_NONE, P, F64, true>(a, s); return true;
+          case PROP_SEP3D: col_launch_k<N, W, PROP_SEP3D, P, F64, true>(a, s); return true;
+          case PROP_C128: col_launch_k<N, W, PROP_C128, P, F64, true>(a, s); return true;
+          default: return false;
+        }
+      }
+    }
+    switch (kind) {
+      case PK_NONE: col_launch_k<N, W, PK_NONE, P, F64>(a, s); return true;
+      case PROP_SEP64: col_launch_k<N, W, PROP_SEP64, P, F64>(a, s); return true;
+      case PROP_C64: col_launch_k<N, W, PROP_C64, P, F64>(a, s); return true;
+      case PROP_SEP3D: col_launch_k<N, W, PROP_SEP3D, P, F64>(a, s); return true;
+      case PROP_C128: col_launch_k<N, W, PROP_C128, P, F64>(a, s); return true;
+      case PROP_KREAL: col_launch_k<N, W, PROP_KREAL, P, F64>(a, s); return true;
+      default: return false;
+    }
   }
   return false;
 }
@@ -358,12 +381,8 @@ static bool col_ok(int w, bool small) {
 
 template <int N>
 static int col_width_for(int64_t ncols, int want, bool small) {
-  // by default at most the widest tile of one column per thread (4096^2, tile
-  // of 8 columns, four per thread, against 4: column sweep 144 -> 131 us)
-  int w = want > 0 ? want : LineCfg<N>::WDEF;
+  int w = want > 0 && !big_slab(N, ncols) ? want : col_width_default<N>();
   if (w > 64) w = 64;
-  if (want <= 0)
-    while (w > 1 && w * LineCfg<N>::T > 1024) w >>= 1;
   while (w > 1 && (w > ncols || (ncols % w) != 0 || !col_ok<N>(w, small))) w >>= 1;
   return w;
 }

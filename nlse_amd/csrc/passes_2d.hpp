@@ -274,27 +274,41 @@ __device__ __forceinline__ void col_prop(const ColArgs& a, prop_t<KIND> (&w)[G][
 #pragma unroll
       for (int g = 0; g < G; ++g) w[g][m] = prop_sep3d(w[g][m], px[g], py, pt[g]);
     }
-  } else if constexpr (KIND == PROP_C128) {
-    const double2* pt = a.ptab128 + c0;
-#pragma unroll
-    for (int m = 0; m < P; ++m)
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-        w[g][m] = prop_c128(w[g][m], pt[(int64_t)(t + m * T) * a.NX + g * CS], (double)a.scale);
   } else {
-    const float2* pt = a.ptab + (int64_t)comp * N * a.NX + c0;
+    static_assert(KIND == PROP_C128, "kinds addressed by column");
+    const double2* pt = a.ptab128 + (int64_t)opaque((uint32_t)t) * a.NX + c0;
 #pragma unroll
-    for (int m = 0; m < P; ++m)
+    for (int m = 0; m < P; ++m) {
 #pragma unroll
       for (int g = 0; g < G; ++g)
-        w[g][m] = prop_c64(w[g][m], pt[(int64_t)(t + m * T) * a.NX + g * CS], a.scale);
+        w[g][m] = prop_c128(w[g][m], pt[(int64_t)(m * T) * a.NX + g * CS], (double)a.scale);
+      // no more than four rows of the table in registers
+      if (m % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// A dense complex64 propagator read as the field is: from the tile's uniform
+// address pt, the lane's offset d and the row stride rs.
+template <int P, int G, int WT, bool PAIRED>
+__device__ __forceinline__ void col_prop_dense(const Buf& pt, float2 (&w)[G][P], uint32_t d, uint32_t rs, float scale) {
+#pragma unroll
+  for (int m = 0; m < P; ++m) {
+    if constexpr (PAIRED) {
+      const float4 q = pt.load<float4>(d, m * rs);
+      w[0][m] = prop_c64(w[0][m], make_float2(q.x, q.y), scale);
+      w[1][m] = prop_c64(w[1][m], make_float2(q.z, q.w), scale);
+    } else {
+#pragma unroll
+      for (int g = 0; g < G; ++g) w[g][m] = prop_c64(w[g][m], pt.load<float2>(d, m * rs + 8u * g * WT), scale);
+    }
   }
 }
 
 // Column sweep body for tile `b` (tile index over slabs x tiles per slab).
-// PK >= 0 compiles only that propagator kind (fewer live registers); -1
-// dispatches on a.pkind.
-template <int N, int P, int WT, int G, int GR, int PK = -1, int FA = F64>
+// PK: the propagator kind compiled in.  BIG: slabs of 4 GiB and more, addressed
+// by 64 bits.
+template <int N, int P, int WT, int G, int GR, int PK, int FA = F64, bool BIG = false>
 __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>* lds) {
   using PL = Plan<N, P>;
   constexpr int T = PL::T;
@@ -313,21 +327,23 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
   constexpr int CS = PAIRED ? 1 : WT;
   const int u0 = (int)((uint32_t)b - slab * tiles) * TILE;  // uniform: first column of the tile
   const int c0 = u0 + (PAIRED ? G * cw : cw);
-  // slabs below 4 GiB are addressed from a uniform descriptor; the PK = -1
-  // instance takes any size (the launcher chooses)
-  constexpr bool WIDE = PK == -1;
+  // slabs below 4 GiB are addressed from a uniform descriptor (the launcher
+  // chooses)
   float2* const A0 = a.A + (int64_t)slab * N * a.NX + u0;
+  // (BIG: the lane's 64-bit address, found again for the stores)
+  auto big_at = [&]() { return A0 + (int64_t)opaque((uint32_t)t) * a.NX + (c0 - u0); };
   const Buf AB(A0), tw(a.tw);
   const uint32_t rs = 8u * (uint32_t)T * (uint32_t)a.NX;
   const uint32_t d = 8u * ((uint32_t)t * (uint32_t)a.NX + (uint32_t)(c0 - u0));
   xchg_t<FA>* lline = lds + cw * GR * LINE;
 
   float2 v[G][P];
+  const float2* const in = BIG ? big_at() : nullptr;
 #pragma unroll
   for (int m = 0; m < P; ++m) {
-    if constexpr (WIDE) {
+    if constexpr (BIG) {
 #pragma unroll
-      for (int g = 0; g < G; ++g) v[g][m] = A0[(int64_t)(t + m * T) * a.NX + (c0 - u0) + g * CS];
+      for (int g = 0; g < G; ++g) v[g][m] = in[(int64_t)(m * T) * a.NX + g * CS];
     } else if constexpr (PAIRED) {
       const float4 q = AB.load<float4>(d, m * rs);
       v[0][m] = make_float2(q.x, q.y);
@@ -340,55 +356,38 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
   const Twid<N, P> W = load_twiddles<N, P>(tw, t);
 
   constexpr int PADSH = 3;
-  if constexpr (PK >= 0 && PK != PK_NONE && PK != PROP_KREAL) {
+  if constexpr (PK != PK_NONE && PK != PROP_KREAL) {
     // F_y, propagator, I_y; with a complex128 propagator the field stays in
     // FP64 from the last forward stage to the first inverse one
     prop_t<PK> w[G][P];
     fft_line_io<N, P, G, false, GR, PADSH, FA, SYNC_BLOCK>(v, w, t, W, tw, lline, LINE);
     const int comp = (int)(slab % (uint32_t)a.ncomp);
-    col_prop<N, P, G, CS, PK>(a, w, comp, t, c0);
+    if constexpr (PK == PROP_C64) {
+      col_prop_dense<P, G, WT, PAIRED>(Buf(a.ptab + (int64_t)comp * N * a.NX + u0), w, d, rs, a.scale);
+    } else {
+      col_prop<N, P, G, CS, PK>(a, w, comp, t, c0);
+    }
     fft_line_io<N, P, G, true, GR, PADSH, FA, SYNC_BLOCK>(w, v, t, W, tw, lline, LINE);
   } else {
     if (a.do_fwd) fft_line<N, P, G, false, GR, PADSH, FA>(v, t, W, tw, lline, LINE);
-    if (PK != PK_NONE && a.do_prop) {
-      const int comp = (int)(slab % (uint32_t)a.ncomp);
-      if (PK == PROP_KREAL || a.pkind == PROP_KREAL) {
-        // even real spectrum: entry (ky, kx) of the quadrant table at
-        // (min(ky, N-ky), min(kx, NX-kx))
-        const int hx = a.NX / 2 + 1;
-        int kx[G];
+    if (PK == PROP_KREAL && a.do_prop) {
+      // even real spectrum: entry (ky, kx) of the quadrant table at
+      // (min(ky, N-ky), min(kx, NX-kx))
+      const int hx = a.NX / 2 + 1;
+      int kx[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const int col = c0 + g * CS;
+        kx[g] = col <= a.NX / 2 ? col : a.NX - col;
+      }
+#pragma unroll
+      for (int m = 0; m < P; ++m) {
+        const int ky = t + m * T;
+        const int kyq = ky <= N / 2 ? ky : N - ky;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-          const int col = c0 + g * CS;
-          kx[g] = col <= a.NX / 2 ? col : a.NX - col;
-        }
-#pragma unroll
-        for (int m = 0; m < P; ++m) {
-          const int ky = t + m * T;
-          const int kyq = ky <= N / 2 ? ky : N - ky;
-#pragma unroll
-          for (int g = 0; g < G; ++g) {
-            const float f = a.kq[kyq * hx + kx[g]] * a.scale;
-            v[g][m] = make_float2(v[g][m].x * f, v[g][m].y * f);
-          }
-        }
-      } else if constexpr (PK < 0) {
-        if (a.pkind == PROP_SEP64) {
-          col_prop<N, P, G, CS, PROP_SEP64>(a, v, comp, t, c0);
-        } else if (a.pkind == PROP_C64) {
-          col_prop<N, P, G, CS, PROP_C64>(a, v, comp, t, c0);
-        } else {
-          double2 w[G][P];
-#pragma unroll
-          for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int m = 0; m < P; ++m) w[g][m] = to_f64(v[g][m]);
-          if (a.pkind == PROP_SEP3D) col_prop<N, P, G, CS, PROP_SEP3D>(a, w, comp, t, c0);
-          else col_prop<N, P, G, CS, PROP_C128>(a, w, comp, t, c0);
-#pragma unroll
-          for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int m = 0; m < P; ++m) v[g][m] = to_f32(w[g][m]);
+          const float f = a.kq[kyq * hx + kx[g]] * a.scale;
+          v[g][m] = make_float2(v[g][m].x * f, v[g][m].y * f);
         }
       }
     }
@@ -403,11 +402,12 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
   }
   auto put = [&](auto st) {
     constexpr int ST = decltype(st)::value;
+    float2* const out = BIG ? big_at() : nullptr;
 #pragma unroll
     for (int m = 0; m < P; ++m) {
-      if constexpr (WIDE) {
+      if constexpr (BIG) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) A0[(int64_t)(t + m * T) * a.NX + (c0 - u0) + g * CS] = v[g][m];
+        for (int g = 0; g < G; ++g) out[(int64_t)(m * T) * a.NX + g * CS] = v[g][m];
       } else if constexpr (PAIRED) {
         AB.template store<ST>(make_float4(v[0][m].x, v[0][m].y, v[1][m].x, v[1][m].y), d, m * rs);
       } else {
@@ -416,12 +416,11 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
       }
     }
   };
-  if (!WIDE && a.through >= through_need(8 * TILE)) put(std::integral_constant<int, ST_THROUGH>{});
+  if (!BIG && a.through >= through_need(8 * TILE)) put(std::integral_constant<int, ST_THROUGH>{});
   else put(std::integral_constant<int, ST_BACK>{});
 }
 
-// PK: the propagator kind compiled in (-1: any kind, chosen at run time).
-template <int N, int P, int WT, int G, int GR, int PK = -1, int FA = F64>
+template <int N, int P, int WT, int G, int GR, int PK, int FA = F64, bool BIG = false>
 __global__ __launch_bounds__(WT*(N / P)) void k_col(ColArgs a) {
   __shared__ xchg_t<FA> lds[col_lds_size<N, WT, GR, xchg_t<FA>>()];
   // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs,
@@ -430,7 +429,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_col(ColArgs a) {
   // by neighbouring tiles on the same XCD (one L2 fill instead of two)
   const int64_t nblk = (int64_t)gridDim.x;
   const int64_t b = (nblk % 8 == 0) ? (int64_t)(blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8 : blockIdx.x;
-  col_body<N, P, WT, G, GR, PK, FA>(a, b, lds);
+  col_body<N, P, WT, G, GR, PK, FA, BIG>(a, b, lds);
 }
 
 // Intensity convolution over the full NY-row torus (a response given by

@@ -230,3 +230,52 @@ def test_stores_back_or_through(gpu, ny, nx, counts, comp):
             want = o.out_field(E * scale[:3], 1.5 * DZ, normalize=False)
             assert rel_l2(ref, want) < C64
         assert np.array_equal(out[:3], ref), k
+
+
+def _sized(sim, prop):
+    sim.propagator = prop.copy()
+    return sim
+
+
+# dense propagators: every column tile gives the same bits
+@pytest.mark.parametrize("name,ny,nx", [("NLSE", 16, 64), ("NLSE", 128, 128), ("CNLSE", 512, 32), ("NLSE", 1024, 64),
+                                        ("CNLSE", 2048, 64), ("NLSE", 4096, 32)])
+def test_dense_propagator_tiles(gpu, name, ny, nx):
+    kw = _material(nx, ny, **({"n12": -3e-10} if name == "CNLSE" else {}))
+    comp = (2,) if name == "CNLSE" else ()
+    rng = np.random.default_rng(ny)
+    prop = np.exp(-1j * rng.random(comp + (ny, nx))).astype(np.complex64)
+    E = _beam((2,) + comp, ny, nx, nx)
+    outs = {}
+    for w in (0, 1, 2, 4, 8, 16, 32):
+        g, o = (_sized(s, prop) for s in _pair(name, kw))
+        g.col_width = w
+        out = g.out_field(E, 2.5 * DZ, verbose=False)
+        outs[g._engine.config()[1]] = out
+    err = rel_l2(out, o.out_field(E, 2.5 * DZ))
+    print(name, ny, nx, sorted(outs), f"{err:.2e}")
+    assert err < C64 and len(outs) >= 3
+    for w, x in outs.items():
+        assert np.array_equal(x, out), w
+
+
+# 3-D fields: a dense complex128 table, and its column tiles
+@pytest.mark.parametrize("shape", [(8, 16, 32), (256, 16, 8), (1024, 8, 16)])
+def test_dense_3d_propagator_tiles(gpu, shape):
+    import nlse_amd
+
+    ny, nx, nt = shape
+    kw = dict(alpha=0, energy=1e-9, window=[4e-3, 4e-3, 2e-12], n2=-1e-9, D0=-1e-26, vg=1.0, V=None, L=1.0, NX=nx, NY=ny,
+              NZ=nt, Isat=np.inf)
+    rng = np.random.default_rng(ny)
+    prop = np.exp(-1j * rng.random(shape))
+    E = (1 + 0.1 * rng.standard_normal(shape) + 0.1j * rng.standard_normal(shape)).astype(np.complex64)
+    outs = []
+    for w in (0, 1, 2, 4, 8, 16, 32):
+        g, o = (_sized(getattr(m, "NLSE_3d")(**kw), prop) for m in (nlse_amd, oracle))
+        g.delta_z = o.delta_z = DZ
+        g.col_width = w
+        outs.append(g.out_field(E, 2.5 * DZ, verbose=False))
+    err = rel_l2(outs[0], o.out_field(E, 2.5 * DZ))
+    print(shape, f"{err:.2e}")
+    assert err < C64 and all(np.array_equal(x, outs[0]) for x in outs)
