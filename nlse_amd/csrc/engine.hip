@@ -756,7 +756,7 @@ struct nlse_plan {
   int row_points = 0;             // row kernels' set size (radix plan) if given, else chosen (row_p)
   bool small = false;             // small-field plans (SMALL_FIELD)
   bool large = false;             // a stack of LARGE_STACK points
-  int through = 0;                // level of the field's stores (through_level)
+  int through = 0;                // level of the field's stores (through_level; complex64)
   bool cplx = false;              // any nonlinear record of a complex dz
   bool cplx_slot[3] = {false, false, false};
   int colw = 1;                   // y-column tile
@@ -1757,7 +1757,6 @@ static WRowArgs wrow_args(const nlse_plan* p, void* A) {
   r.drv_r1 = p->fr1;
   r.drv_dz = p->drv_dz;
   r.out_scale = 1.0;
-  r.through = p->through;
   return r;
 }
 
@@ -1776,7 +1775,6 @@ static WColArgs wcol_args(const nlse_plan* p, void* A) {
   c.ptab = p->ptab;
   c.scale = 1.0 / ((double)p->d.nx * (double)p->d.ny);
   c.out_scale = 1.0;
-  c.through = p->through;
   return c;
 }
 
@@ -1849,7 +1847,6 @@ static WColArgs wcolx3d_args(const nlse_plan* p, void* A) {
   c.tw = p->wtwx;
   c.scale = 1.0;
   c.out_scale = 1.0;
-  c.through = p->through;
   return c;
 }
 

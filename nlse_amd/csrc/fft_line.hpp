@@ -118,10 +118,6 @@ struct Buf {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, lane, uni, ST);
   }
-  template <int ST = ST_BACK>
-  __device__ __forceinline__ void store(double2 x, uint32_t lane, uint32_t uni) const {
-    store<ST>(__builtin_bit_cast(float4, x), lane, uni);
-  }
 };
 
 // Padding of the row kernels' LDS lines (one float2 every 2^NLSE_ROW_PADSH

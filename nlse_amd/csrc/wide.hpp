@@ -303,7 +303,6 @@ struct WRowArgs {
   int has_b;
   int loss_sat;
   int write_I;            // store the field and |A|^2 (FP64) after I_x, nothing else
-  int through;            // stores written through (fields of WRITE_THROUGH bytes at most)
   const void* nlp_a;      // WNL1[items] or WNL2[items*2]
   const void* nlp_b;
   const WRabi* rabi;      // [items]
@@ -322,10 +321,10 @@ struct WRowArgs {
 
 // Two waves per SIMD of 1024^2 points load, transform and store in step, so a
 // sweep is the sum of its memory time (5 us), VALU (5 us) and exchanges (3 us)
-// and launch, not their maximum: 18.8 us.  Series instead of library functions,
-// the factored butterflies and stores written through took a 2-D step from
-// 43.3 to 37.6 us (2048^2: 118.7 to 87.5, 256^2: 16.3 to 12.0); 4 points per
-// lane (121 us at 2048^2) and kept twiddles at 1024 points did not help.
+// and launch, not their maximum: 18.8 us.  Series instead of library functions
+// and the factored butterflies took a 2-D step from 43.3 to 37.6 us (2048^2: 118.7
+// to 87.5, 256^2: 16.3 to 12.0); 4 points per lane (121 us at 2048^2) and kept
+// twiddles at 1024 points did not help.
 // Rows of length N (x rows of 2-D fields, t rows of 3-D fields): LPB line
 // groups per block, G components per group.  Dynamic LDS: LPB*G lines.
 template <int N, int P, int LPB, int G>
@@ -365,22 +364,12 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wrow(WRowArgs a) {
 #pragma unroll
   for (int m = 0; m < P; ++m) vf[m] = v_early ? reinterpret_cast<const float*>(a.V)[vbase + m * T] : 0.f;
 
-  // a written-through field is addressed by 32 bits
-  const Buf buf(a.A);
   auto put = [&]() {
     if (!active) return;
-    if (a.through) {
 #pragma unroll
-      for (int g = 0; g < G; ++g)
+    for (int g = 0; g < G; ++g)
 #pragma unroll
-        for (int m = 0; m < P; ++m)
-          buf.store<ST_THROUGH>(v[g][m], 16u * (uint32_t)(off[g] + t), 16u * (uint32_t)(m * T));
-    } else {
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int m = 0; m < P; ++m) a.A[off[g] + t + m * T] = v[g][m];
-    }
+      for (int m = 0; m < P; ++m) a.A[off[g] + t + m * T] = v[g][m];
   };
 
   if (a.inverse_first) wfft_line<N, P, G, true, SYNC>(v, t, W, tw, lline);
@@ -476,7 +465,6 @@ struct WColArgs {
   int nt;
   double scale;
   double out_scale;
-  int through;         // as in WRowArgs
 };
 
 // Columns of length N: WT adjacent columns per block, one per thread column.
@@ -550,15 +538,8 @@ __global__ __launch_bounds__(WT*(N / P)) void k_wcol(WColArgs a) {
 #pragma unroll
     for (int m = 0; m < P; ++m) v[0][m] = make_double2(v[0][m].x * a.out_scale, v[0][m].y * a.out_scale);
   }
-  if (a.through) {
-    const Buf buf(a.A);
 #pragma unroll
-    for (int m = 0; m < P; ++m)
-      buf.store<ST_THROUGH>(v[0][m], 16u * (uint32_t)(base + t * a.NX), 16u * (uint32_t)(m * T * a.NX));
-  } else {
-#pragma unroll
-    for (int m = 0; m < P; ++m) a.A[base + (int64_t)(t + m * T) * a.NX] = v[0][m];
-  }
+  for (int m = 0; m < P; ++m) a.A[base + (int64_t)(t + m * T) * a.NX] = v[0][m];
 }
 
 // ------------------------------------------------- nonlocal response (2-D)
