@@ -234,9 +234,10 @@ __device__ __forceinline__ void bf2(double2 e, double2 o, bool mi, double2& x0, 
 template <int R, int K>
 constexpr double2 const_ct() {
   static_assert(K > 0 && K < R / 4 && R <= 16, "W8, W16, W16^3");
+  // (the tangents of the rounded cosines, as in the tables)
   constexpr double c = R == 8 || K == 2 ? K_R2 : (K == 1 ? K_C8 : K_S8);
-  constexpr double s = R == 8 || K == 2 ? -K_R2 : (K == 1 ? -K_S8 : -K_C8);
-  return double2{c, s / c};
+  constexpr double t = R == 8 || K == 2 ? 0.9999999999999999 : (K == 1 ? 0.41421356237309503 : 2.414213562373095);
+  return double2{c, -t};
 }
 
 template <int R, bool TW, int K = 0>

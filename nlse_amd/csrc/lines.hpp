@@ -43,7 +43,9 @@ struct LineOps {
 
 // Ratio pairs {c, s/c} of the stages of Plan<N, P> (rt_offset): for the levels r
 // = R, R/2, .., 2 of a stage of radix R, w^(R/r) W_r^k with k < max(1, r/4) and
-// w = exp(-2 pi i jm / (Ns R)), entry [i * Ns + jm] for the i-th pair.
+// w = exp(-2 pi i jm / (Ns R)), entry [i * Ns + jm] for the i-th pair.  The ratio
+// is that of the exact sine to the rounded cosine, which the butterfly multiplies
+// by: each part of a twiddle is rounded once.
 template <int N, int P>
 void build_ratio_twiddles(double2* rt) {
   if constexpr (P <= N) {
@@ -56,9 +58,11 @@ void build_ratio_twiddles(double2* rt) {
         for (int k = 0; k < (r >= 4 ? r / 4 : 1); ++k, ++i)
           for (int jm = 0; jm < NS; ++jm) {
             // angle / (-2 pi) = jm / (NS r) + k / r, in lowest terms of NS r
-            const double ang = -2.0 * M_PI * (double)(jm + (long)k * NS) / ((double)NS * r);
-            const double c = std::cos(ang), sn = std::sin(ang);
-            out[i * NS + jm] = make_double2(c, sn / c);
+            const long double pi = 3.14159265358979323846264338327950288L;
+            const long double ang = -2 * pi * (long double)(jm + (long)k * NS) / ((long double)NS * r);
+            double c = (double)cosl(ang);
+            if (std::fabs(c) < 1e-17) c = 6e-17;  // (a quarter turn: see bf2)
+            out[i * NS + jm] = make_double2(c, (double)(sinl(ang) / (long double)c));
           }
     }
   }

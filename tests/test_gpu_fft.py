@@ -102,3 +102,23 @@ def test_fft_roundtrip_unbiased(gpu):
         bias = np.real(np.vdot(x64, e)) / np.real(np.vdot(x64, x64))
         print(f"n={n} round-trip rel err {np.linalg.norm(e) / np.linalg.norm(x64):.3e} gain bias {bias:.3e}")
         assert abs(bias) < 1e-8
+
+
+@pytest.mark.parametrize("n", [8, 64, 256, 512, 1024, 2048, 4096])
+def test_complex128_error_against_80_bits(gpu, n):
+    """A butterfly layer of two roundings and twiddles rounded once leave no more
+    error than numpy's FP64 transform, which has as many layers and roundings."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((256, n)) + 1j * rng.standard_normal((256, n))
+    ref = np.fft.fft(x.astype(np.clongdouble), axis=-1)
+
+    def err(y):
+        return float(np.linalg.norm(y - ref) / np.linalg.norm(ref))
+
+    t = torch.from_numpy(x.copy()).to(gpu)
+    from nlse_amd.fft import HipFFTPlan
+
+    HipFFTPlan(x.shape, np.complex128, 1).fft(t)
+    got, bound = err(t.cpu().numpy()), err(np.fft.fft(x, axis=-1))
+    print(f"{n} points: {got:.3e}, numpy {bound:.3e}")
+    assert got < 1.05 * bound
