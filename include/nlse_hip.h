@@ -373,9 +373,9 @@ int nlse_plan_config(const nlse_plan* plan, int* row_points, int* col_width);
  * Uneven batches (no counterpart in the reference: its batching is the
  * leading-dimension broadcast of one grid, nlse.py:320-327).  Many 2-D
  * single-component NLSE fields of different grids and parameters advance
- * together: one persistent launch per sweep for the whole batch, steady
- * steps replayed from a captured hipGraph.  Grids: powers of two in
- * [128, 2048] on both axes. */
+ * together: one launch per sweep and line length for the whole batch (or one
+ * per sweep), steady steps replayed from a captured hipGraph.  Grids: powers
+ * of two in [128, 2048] on both axes. */
 typedef struct nlse_batch nlse_batch;
 typedef struct {
   int64_t ny, nx;
@@ -388,15 +388,22 @@ typedef struct {
 } nlse_batch_item;
 int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_saturates, nlse_batch** out);
 int nlse_batch_destroy(nlse_batch* batch);
-/* Persistent grid of the batch sweeps: blocks per CU of the row and column
- * kernels (defaults 4 and 2; chosen by the autotuner). */
+/* Grids of the batch sweeps, row and column kernels.  By default the launch of
+ * a line length has a block for every pass of its units (what one block of the
+ * single-field kernels does), and the single launch of all lengths (below) 4 and
+ * 1 blocks per CU that stride over the units.  set_grid: that many blocks per CU
+ * stride over the units in both (1 to 64; where they cover the units of a
+ * length, its launch is the default one).  default_grid: back to the default.
+ * Results are identical; the autotuner times both. */
 int nlse_batch_set_grid(nlse_batch* batch, int row_blocks_per_cu, int col_blocks_per_cu);
+int nlse_batch_default_grid(nlse_batch* batch);
 /* on != 0: every sweep of the batch is ONE persistent launch over the
  * units of all line lengths (each unit's length selects its code path);
- * 0 (default): one persistent launch per line length present.  Results are
+ * 0 (default): one launch per line length present.  Results are
  * identical; the autotuner times both. */
 int nlse_batch_set_single_launch(nlse_batch* batch, int on);
-/* Work units and persistent grid sizes of the row and column sweeps. */
+/* Work units of the row and column sweeps, and how many of them the blocks of a
+ * sweep's launches take at a time (all of them by default). */
 int nlse_batch_config(const nlse_batch* batch, int64_t* row_units, int64_t* col_units, int* row_grid,
                       int* col_grid);
 /* nsteps split steps of every field of the batch buffer `base_dev` (real

@@ -125,6 +125,7 @@ SIGNATURES = {
     "nlse_batch_destroy": (c_int, [c_void_p]),
     "nlse_batch_config": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "nlse_batch_set_grid": (c_int, [c_void_p, c_int, c_int]),
+    "nlse_batch_default_grid": (c_int, [c_void_p]),
     "nlse_batch_set_single_launch": (c_int, [c_void_p, c_int]),
     "nlse_fno_gemm": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_i64, c_i64, c_i64, c_void_p, c_i64, c_i64,
                               c_i64, c_void_p, c_i64, c_i64, c_i64, C.c_float, C.c_float, c_void_p, c_void_p,

@@ -11,8 +11,9 @@ problem shape, flags) on the real tables and remembered in a JSON file:
   stages) and the number of steady steps per captured hipGraph (0: direct
   launches);
 * uneven batches: the launch structure (one persistent launch per sweep for
-  all line lengths, or one per length), the persistent grid of the row and
-  column sweeps (blocks per CU) and the graph chunk.
+  all line lengths, or one per length), the grids of the row and column
+  sweeps (the engine's own, or blocks per CU that stride over the work) and
+  the graph chunk.
 
 Tiles, chunks, grids and launch structures compute bit-identical results;
 the two radix plans round differently (both within the parity bound of the
@@ -34,7 +35,8 @@ import time
 VERSION = 2
 COL_WIDTHS = (1, 2, 4, 8, 16, 32)
 GRAPH_CHUNKS = (0, 8, 16, 32)
-BATCH_GRIDS = ((2, 1), (4, 2), (8, 2), (4, 1), (8, 1), (8, 4), (16, 1))
+DEFAULT_GRID = (0, 0)  # the batch engine's own grids
+BATCH_GRIDS = (DEFAULT_GRID, (2, 1), (4, 2), (8, 2), (4, 1), (8, 1), (8, 4), (16, 1))
 ROW_POINTS = (0, 8, 16)
 
 
@@ -160,21 +162,29 @@ def tune_plan(make_engine, A0, precision: int, nsteps: int = 40) -> dict:
             "graph_chunk_us": {str(k): v * 1e6 for k, v in chunks.items()}}
 
 
+def apply_grid(eng, grid) -> None:
+    """Give a batch engine the grid of a BATCH_GRIDS or cache entry."""
+    if tuple(grid) == DEFAULT_GRID:
+        eng.default_grid()
+    else:
+        eng.set_grid(*grid)
+
+
 def tune_batch(eng, buf, precision: int, nsteps: int = 20) -> dict:
     """Time the launch structure (one persistent launch per sweep for all
-    line lengths, or one per length), the persistent grids and the graph
-    chunks of a batch engine."""
+    line lengths, or one per length), the grids and the graph chunks of a
+    batch engine."""
     grids = {}
     for single in (False, True):
         eng.set_single_launch(single)
         for rb, cb in BATCH_GRIDS:
-            eng.set_grid(rb, cb)
+            apply_grid(eng, (rb, cb))
             eng.graph_chunk = 16
             grids[(single, rb, cb)] = _time_run(lambda A, n: eng.run(A, n, precision), buf, nsteps)
     best = min(grids, key=grids.get)
     eng.set_single_launch(best[0])
     best_g = best[1:]
-    eng.set_grid(*best_g)
+    apply_grid(eng, best_g)
     chunks = {}
     for c in GRAPH_CHUNKS:
         eng.graph_chunk = c

@@ -5,13 +5,15 @@ The reference batches only through leading-dimension broadcasting of one
 grid (nlse.py:320-327); instances of different sizes are separate
 out_field calls.  Here every instance keeps its own NLSE object (grid,
 alpha, n2, I_sat, power, V, delta_z), and NLSEBatch.out_field propagates
-all of them with one persistent launch per sweep for the whole batch:
+all of them with one launch per sweep and line length for the whole batch:
 
     sims = [NLSE(alpha, P_i, window, n2_i, None, L, NX=N_i, NY=N_i, Isat=I_i) ...]
     outs = NLSEBatch(sims).out_field([E_i ...], z)
 
 Each field follows exactly the step sequence of its own out_field (same
-kernels, same arithmetic), so the results equal separate runs.
+kernels, same arithmetic), so the results equal separate runs bit for bit,
+unless a run of its own takes another radix plan (row_points, as set or tuned),
+which rounds differently.
 """
 
 from __future__ import annotations
@@ -78,6 +80,11 @@ class BatchEngine:
         _lib.check(_lib.load().nlse_batch_set_grid(self._h, int(row_blocks_per_cu), int(col_blocks_per_cu)),
                    "batch_set_grid")
 
+    def default_grid(self) -> None:
+        """The engine's own grids: a block per pass of a unit, in one launch
+        per line length (set_grid gives others)."""
+        _lib.check(_lib.load().nlse_batch_default_grid(self._h), "batch_default_grid")
+
     def set_single_launch(self, on: bool) -> None:
         """True: each sweep is one persistent launch over every line length;
         False: one launch per line length present (identical results)."""
@@ -139,7 +146,7 @@ class NLSEBatch:
             raise ValueError("all instances of a batch share the loss semantics")
         self.sims = list(sims)
         self.graph_chunk = 16
-        # one persistent launch per sweep for all line lengths (None: the
+        # True: one persistent launch per sweep for all line lengths (None: the
         # autotuner's choice if cached, else one launch per length)
         self.single_launch = None
 
@@ -178,7 +185,7 @@ class NLSEBatch:
         eng.graph_chunk = self.graph_chunk
         tuned = autotune.lookup(autotune.batch_key([(s.NY, s.NX) for s in self.sims]))
         if tuned is not None:
-            eng.set_grid(tuned["row_blocks_per_cu"], tuned["col_blocks_per_cu"])
+            autotune.apply_grid(eng, (tuned["row_blocks_per_cu"], tuned["col_blocks_per_cu"]))
             eng.graph_chunk = int(tuned["graph_chunk"])
             if self.single_launch is None and "single_launch" in tuned:
                 eng.set_single_launch(bool(tuned["single_launch"]))
@@ -192,8 +199,8 @@ class NLSEBatch:
         return eng, buf, nsteps.pop()
 
     def tune(self, E_list, precision: str = "single") -> dict:
-        """Time the persistent grids and graph chunks of this batch's
-        shapes and cache the fastest (nlse_amd.autotune)."""
+        """Time the grids and graph chunks of this batch's shapes and cache
+        the fastest (nlse_amd.autotune)."""
         eng, buf, _ = self.prepare(E_list, 1e-30, precision)
         res = autotune.tune_batch(eng, buf, self.sims[0]._precision_flag(precision))
         autotune.store(autotune.batch_key([(s.NY, s.NX) for s in self.sims]), res)

@@ -1,18 +1,19 @@
 // Uneven batches of 2-D single-component fields (nlse_batch_*): many NLSE
 // instances of different grid sizes and physical parameters advanced
-// together, one persistent launch per sweep and line length for the whole
-// batch.
+// together, one launch per sweep and line length for the whole batch, or one
+// per sweep.
 //
 // Work units are uniform in size whatever the grid: a row unit is
 // 4096/NX rows of NX points (256 threads) and a column unit is 8192/NY
 // columns of NY points (512 threads).  Every unit therefore moves the same
-// bytes and does the same FFT work per point, and a persistent grid that
-// strides over the unit list is balanced without a work queue.  Each block
-// reads its unit's instance descriptor (field pointer, tables, parameters) and
-// runs the sweep body of that line length, in the plan (points per thread,
-// exchange precision) of the member's own single-field run: small members
-// (SMALL_FIELD) take the small-field plans, so every member gives bit for bit
-// the result of its own run.
+// bytes and does the same FFT work per point.  By default a block takes one
+// pass of a unit; blocks of a smaller grid stride over the unit list, balanced
+// without a work queue.  Each block reads its unit's instance descriptor (field
+// pointer, tables, parameters) and runs the sweep body of that line length, in
+// the plan (points per thread, exchange precision) that the member's own
+// single-field run takes by default: small members (SMALL_FIELD) take the
+// small-field plans, so every member gives bit for bit the result of its own
+// run (row_points as given or tuned for that run aside).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -278,8 +279,9 @@ static BatchFlags row_flags(int precision, int stage) {
   return f;
 }
 
-// Blocks of a per-length launch: one per pass when the grid covers the units
-// (the default), else the grid given per CU (nlse_batch_set_grid).
+// Blocks of a per-length launch: one per pass where the grid covers the units
+// (the default), else the grid given per CU (nlse_batch_set_grid), whose blocks
+// stride over the passes.
 static unsigned pass_grid(int64_t units, int passes, int grid) {
   return (unsigned)(grid >= units ? units * passes : grid);
 }
@@ -303,8 +305,8 @@ static void launch_col_n(nlse_batch* b, int li, const BatchFlags& f, hipStream_t
                      dim3(TH), 0, s, b->d_inst, b->d_col + b->col_off[li], n, f);
 }
 
-// One persistent launch per line length present in the batch, or one for
-// all lengths (b->single).
+// One launch per line length present in the batch, or one for all lengths
+// (b->single).
 static int batch_row(nlse_batch* b, const BatchFlags& f, hipStream_t s) {
   if (b->single) {
     hipLaunchKernelGGL(b->general ? k_batch_row_all<true> : k_batch_row_all<false>, dim3((unsigned)b->row_grid_all),
@@ -378,6 +380,25 @@ static int batch_bind(nlse_batch* b, void* base, hipStream_t s) {
   return NLSE_OK;
 }
 
+static int64_t batch_cus() {
+  int dev = 0, ncu = 256;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  return ncu;
+}
+
+// All units at once: a block per pass (pass_grid).  64 fields of 256^2 to 1024^2
+// (7168 and 3584 units at 1024 points): 366 us a step by 8 and 1 blocks per CU that
+// stride over the units, 282 by a block per pass.
+static void batch_default_grid(nlse_batch* b) {
+  const int64_t ncu = batch_cus();
+  for (int li = 0; li < NLEN; ++li) {
+    b->row_grid[li] = (int)(b->row_off[li + 1] - b->row_off[li]);
+    b->col_grid[li] = (int)(b->col_off[li + 1] - b->col_off[li]);
+  }
+  b->row_grid_all = (int)std::min<int64_t>(b->n_row, ncu * 4);
+  b->col_grid_all = (int)std::min<int64_t>(b->n_col, ncu * 1);
+}
+
 extern "C" {
 
 int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_saturates, nlse_batch** out) {
@@ -395,9 +416,7 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
   nlse_batch* b = new nlse_batch();
   b->count = count;
   int rc = NLSE_OK;
-  int dev = 0, ncu = 256;
   int64_t total = 0;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   std::vector<BatchUnit> rows_n[NLEN], cols_n[NLEN];
   for (int64_t i = 0; i < count && !rc; ++i) {
     const nlse_batch_item& it = items[i];
@@ -467,9 +486,6 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
     b->col_off[li] = (int64_t)cols.size();
     rows.insert(rows.end(), rows_n[li].begin(), rows_n[li].end());
     cols.insert(cols.end(), cols_n[li].begin(), cols_n[li].end());
-    // a block per pass
-    b->row_grid[li] = (int)rows_n[li].size();
-    b->col_grid[li] = (int)cols_n[li].size();
   }
   b->row_off[NLEN] = (int64_t)rows.size();
   b->col_off[NLEN] = (int64_t)cols.size();
@@ -482,8 +498,7 @@ int nlse_batch_create(const nlse_batch_item* items, int64_t count, int loss_satu
   }
   b->n_row = (int64_t)rows.size();
   b->n_col = (int64_t)cols.size();
-  b->row_grid_all = (int)std::min<int64_t>(b->n_row, (int64_t)ncu * 4);
-  b->col_grid_all = (int)std::min<int64_t>(b->n_col, (int64_t)ncu * 1);
+  batch_default_grid(b);
   *out = b;
   return NLSE_OK;
 }
@@ -500,15 +515,21 @@ int nlse_batch_destroy(nlse_batch* b) {
 int nlse_batch_set_grid(nlse_batch* b, int row_blocks_per_cu, int col_blocks_per_cu) {
   if (!b || row_blocks_per_cu < 1 || col_blocks_per_cu < 1 || row_blocks_per_cu > 64 || col_blocks_per_cu > 64)
     return fail(NLSE_ERR_ARG, "bad batch grid (%d, %d blocks per CU)", row_blocks_per_cu, col_blocks_per_cu);
-  int dev = 0, ncu = 256;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  const int64_t ncu = batch_cus();
   for (int li = 0; li < NLEN; ++li) {
-    b->row_grid[li] = (int)std::min<int64_t>(b->row_off[li + 1] - b->row_off[li], (int64_t)ncu * row_blocks_per_cu);
-    b->col_grid[li] = (int)std::min<int64_t>(b->col_off[li + 1] - b->col_off[li], (int64_t)ncu * col_blocks_per_cu);
+    b->row_grid[li] = (int)std::min<int64_t>(b->row_off[li + 1] - b->row_off[li], ncu * row_blocks_per_cu);
+    b->col_grid[li] = (int)std::min<int64_t>(b->col_off[li + 1] - b->col_off[li], ncu * col_blocks_per_cu);
   }
-  b->row_grid_all = (int)std::min<int64_t>(b->n_row, (int64_t)ncu * row_blocks_per_cu);
-  b->col_grid_all = (int)std::min<int64_t>(b->n_col, (int64_t)ncu * col_blocks_per_cu);
+  b->row_grid_all = (int)std::min<int64_t>(b->n_row, ncu * row_blocks_per_cu);
+  b->col_grid_all = (int)std::min<int64_t>(b->n_col, ncu * col_blocks_per_cu);
   batch_graph_free(b);  // the captured launches bake in the grid
+  return NLSE_OK;
+}
+
+int nlse_batch_default_grid(nlse_batch* b) {
+  if (!b) return fail(NLSE_ERR_ARG, "null batch");
+  batch_default_grid(b);
+  batch_graph_free(b);
   return NLSE_OK;
 }
 
@@ -532,7 +553,7 @@ int nlse_batch_config(const nlse_batch* b, int64_t* row_units, int64_t* col_unit
     rg = b->row_grid_all;
     cg = b->col_grid_all;
   }
-  if (row_grid) *row_grid = rg;  // blocks over the launches of one sweep
+  if (row_grid) *row_grid = rg;  // units taken at a time over the launches of one sweep
   if (col_grid) *col_grid = cg;
   return NLSE_OK;
 }

@@ -40,3 +40,48 @@ def test_enabled_flag(monkeypatch):
     assert not autotune.enabled()
     monkeypatch.setenv("NLSE_AMD_AUTOTUNE", "1")
     assert autotune.enabled()
+
+
+class _Batch:
+    """A batch engine whose step takes the time given for its grid."""
+
+    def __init__(self, times):
+        self.times, self.grid, self.single, self.seen = times, None, False, []
+
+    def set_grid(self, rb, cb):
+        assert rb >= 1 and cb >= 1  # refused by the library
+        self.grid = (rb, cb)
+
+    def default_grid(self):
+        self.grid = autotune.DEFAULT_GRID
+
+    def set_single_launch(self, on):
+        self.single = on
+
+    def run(self, A, n, precision):
+        pass
+
+
+def _tune(monkeypatch, times):
+    eng = _Batch(times)
+
+    def time_run(run, A0, nsteps, reps=2):
+        eng.seen.append((eng.single, eng.grid))
+        return times.get(eng.grid, 2.0) + (0.5 if eng.single else 0.0)
+
+    monkeypatch.setattr(autotune, "_time_run", time_run)
+    return eng, autotune.tune_batch(eng, None, 0)
+
+
+def test_batch_tuner_times_the_default_grid(monkeypatch):
+    """The engine's own grid is a candidate, in both launch structures, and is
+    what the engine and the cache entry hold when it is the fastest."""
+    eng, res = _tune(monkeypatch, {autotune.DEFAULT_GRID: 1.0})
+    assert {(False, autotune.DEFAULT_GRID), (True, autotune.DEFAULT_GRID)} <= set(eng.seen)
+    assert eng.grid == autotune.DEFAULT_GRID and eng.single is False
+    assert (res["row_blocks_per_cu"], res["col_blocks_per_cu"]) == autotune.DEFAULT_GRID
+    fresh = _Batch({})
+    autotune.apply_grid(fresh, [res["row_blocks_per_cu"], res["col_blocks_per_cu"]])
+    assert fresh.grid == autotune.DEFAULT_GRID
+    eng, res = _tune(monkeypatch, {(8, 4): 1.0})
+    assert eng.grid == (8, 4) and (res["row_blocks_per_cu"], res["col_blocks_per_cu"]) == (8, 4)

@@ -83,3 +83,35 @@ def test_batch_config_balanced_units(gpu):
     P = sum(ny * nx for ny, nx in SHAPES)
     assert cfg["row_units"] * 4096 == P and cfg["col_units"] * 8192 == P
     assert 0 < cfg["row_grid"] <= cfg["row_units"] and 0 < cfg["col_grid"] <= cfg["col_units"]
+
+
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("precision", ["single", "double"])
+def test_grids_bit_identical(gpu, single, precision):
+    """Blocks that stride over more units than there are CUs (rows and columns
+    of every length, with several passes a unit) and the default grid give the
+    same bits, and default_grid restores the default."""
+    from nlse_amd import NLSE
+    from nlse_amd.batch import NLSEBatch
+
+    shapes = [(128, 128)] * 40 + [(256, 256)] * 40 + [(512, 512)] * 18 + [(1024, 1024)] * 3 + [(2048, 512)] * 2
+    sims, fields = _instances(NLSE, shapes)
+    eng, buf, _ = NLSEBatch(sims).prepare(fields, 1e-5, precision)
+    eng.set_single_launch(single)
+    A0, flag = buf.clone(), int(precision == "double")
+    default = eng.config()
+    eng.run(buf, 3, flag)
+    want = buf.clone()
+    for grid in ((1, 1), (2, 1), (16, 4), (64, 64)):
+        eng.set_grid(*grid)
+        cfg = eng.config()
+        if grid == (1, 1):
+            assert cfg["row_grid"] < cfg["row_units"] and cfg["col_grid"] < cfg["col_units"]
+        buf.copy_(A0)
+        eng.run(buf, 3, flag)
+        assert torch.equal(torch.view_as_real(buf), torch.view_as_real(want)), grid
+    eng.default_grid()
+    assert eng.config() == default
+    buf.copy_(A0)
+    eng.run(buf, 3, flag)
+    assert torch.equal(torch.view_as_real(buf), torch.view_as_real(want))
