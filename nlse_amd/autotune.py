@@ -20,7 +20,7 @@ the two radix plans round differently (both within the parity bound of the
 complex64 oracle), which is why the radix choice is part of the cached
 entry rather than a free run-time switch.
 
-Cache: $NLSE_AMD_TUNE_CACHE, else ~/.cache/nlse_amd/tune-v2.json.  With
+Cache: $NLSE_AMD_TUNE_CACHE, else ~/.cache/nlse_amd/tune-v3.json.  With
 NLSE_AMD_AUTOTUNE=1 the engine tunes a shape on first use; otherwise a
 shape is tuned by NLSE.tune(E) / NLSEBatch.tune(E_list) and cached entries
 are used whenever present.
@@ -32,7 +32,9 @@ import json
 import os
 import time
 
-VERSION = 2
+# raised whenever the kernels or defaults that the stored choices were timed
+# against, or what a stored choice means, change: older files are not read
+VERSION = 3
 COL_WIDTHS = (1, 2, 4, 8, 16, 32)
 GRAPH_CHUNKS = (0, 8, 16, 32)
 DEFAULT_GRID = (0, 0)  # the batch engine's own grids

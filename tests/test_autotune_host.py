@@ -85,3 +85,17 @@ def test_batch_tuner_times_the_default_grid(monkeypatch):
     assert fresh.grid == autotune.DEFAULT_GRID
     eng, res = _tune(monkeypatch, {(8, 4): 1.0})
     assert eng.grid == (8, 4) and (res["row_blocks_per_cu"], res["col_blocks_per_cu"]) == (8, 4)
+
+
+def test_entries_of_earlier_kernels_are_not_read(tmp_path, monkeypatch):
+    """Choices timed before the small-field plans, the 4-column tiles and the
+    block-per-pass grids (version 2) would override those defaults."""
+    path = tmp_path / "tune.json"
+    monkeypatch.setenv("NLSE_AMD_TUNE_CACHE", str(path))
+    path.write_text(json.dumps({"version": 2, "entries": {"plan|gfx950|a": {"col_width": 8, "row_points": 16,
+                                                                             "graph_chunk": 16}}}))
+    assert autotune.lookup("plan|gfx950|a") is None
+    autotune.store("plan|gfx950|b", {"col_width": 4, "graph_chunk": 0})
+    assert set(autotune.load()) == {"plan|gfx950|b"}
+    monkeypatch.delenv("NLSE_AMD_TUNE_CACHE")
+    assert "tune-v2" not in autotune.cache_path()
