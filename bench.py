@@ -388,9 +388,9 @@ def _timed(fn, *a) -> float:
 
 def bench_batch(args) -> int:
     """Uneven batch: 64 fields of 256^2/512^2/1024^2 with random n2, power,
-    Isat, one persistent launch per sweep for the whole batch, steady steps
-    replayed from a captured graph.  Compared with the same fields run one
-    after the other through their own plans."""
+    Isat, one launch per sweep and line length for the whole batch (or one per
+    sweep), steady steps replayed from a captured graph.  Compared with the
+    same fields run one after the other through their own plans."""
     import torch
 
     from nlse_amd import NLSE, NLSEBatch

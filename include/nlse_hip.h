@@ -244,7 +244,9 @@ typedef struct nlse_plan_desc {
   int ndim;          /* 1: (items, [2,] NX); 2: (items, [2,] NY, NX); 3: (items, NY, NX, NT) */
   int64_t ny, nx;    /* transform sizes (ny ignored for ndim 1) */
   int64_t nt;        /* third (fastest) axis of ndim 3 */
-  int64_t items;     /* leading (broadcast) items */
+  int64_t items;     /* leading (broadcast) items; the kernels chosen depend on the points
+                        (lines of ndim 1) of all items: the same field rounds differently, within
+                        the parity bounds, in stacks of other sizes */
   int ncomp;         /* 1, or 2 for CNLSE / DDGPE layouts (..., 2, NY, NX) */
   int loss_saturates;
   int row_points;    /* points per thread of the x-row kernels (radix plan): 0 = default for

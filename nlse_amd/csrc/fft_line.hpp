@@ -203,7 +203,9 @@ __device__ __forceinline__ C from_f64(double2 a) {
   else return a;
 }
 
-// Radix-R butterfly in FP64 as log2 R layers of radix-2 ones: X[k] = E[k] +
+// Radix-R butterfly in FP64 as log2 R layers of radix-2 ones, in the factored form
+// for fused multiply-adds of E. Linzer and E. Feig (IEEE Trans. Signal Processing
+// 41, 93, 1993): X[k] = E[k] +
 // w W_R^k O[k], X[k + R/2] = E[k] - w W_R^k O[k] with E, O the transforms of
 // the even and odd points for w^2.  A twiddle c + i s is applied as c (1 + i
 // s/c), the c inside the additions: a butterfly is 6 FMAs where a complex
@@ -213,7 +215,7 @@ __device__ __forceinline__ C from_f64(double2 a) {
 // a stage: w W_R^k for k < R/4 (the others are -i times these), then the same
 // for w^2 and R/2, and so on.  Where c is nearly zero s/c is as large and the
 // product keeps its relative precision; c is never exactly zero (the table
-// holds cos(pi/2) as the FP64 cosine, 6e-17).
+// holds 6e-17 for a quarter turn).
 __device__ __forceinline__ void bf2(double2 e, double2 o, double2 ct, bool mi, double2& x0, double2& x1) {
   const double vr = fma(-ct.y, o.y, o.x), vi = fma(ct.y, o.x, o.y);
   if (!mi) {

@@ -114,15 +114,19 @@ constexpr int lines_per_block(int threads, int t) { return threads / t >= 1 ? th
 // Fields of at most this many points (all items and components) take the
 // small-field plans of LineCfg: their sweeps are a few waves per CU, bound by
 // the length of one lane's work.  One step (row + column sweep) of a local
-// field, default against small-field plan: 256^2 14.0 -> 7.8 us, 512^2 12.7 ->
-// 10.6 us; 18 fields of 256^2 (1.2 M points) 19.0 -> 20.2 us.
+// field, default against small-field plan: 256^2 14.0 -> 7.8 us; at the limit 4 x
+// 256^2 11.0 -> 9.0, 16 x 128^2 10.6 -> 8.8, 64 x 64^2 11.8 -> 7.5, 512^2 11.5 ->
+// 10.3.  Past it the plans cross at other sizes for each grid (24 x 128^2 11.2 /
+// 9.8, 5 x 256^2 11.1 / 10.8, 4 x 512^2 14.9 / 14.1, but 3 x 512^2 14.1 / 15.1, 24 x
+// 256^2 17.8 / 19.2): the line lies where all of them still gain.
 constexpr int64_t SMALL_FIELD = 1 << 18;
 
 // Fields of at most this many bytes are written through to memory: a kernel's
 // end then has no dirty L2 lines left to write back before the next sweep,
 // whose reads come from other XCDs, may start.  Step of a local field, stores
 // back / through: 1024^2 25.2 -> 21.0 us, 2 x 1024^2 46.2 -> 31.8 us, 2048^2
-// 59.7 -> 56.4 us; 28 x 1024^2 (235 MB) 280 -> 298 us.
+// 59.7 -> 56.4 us, 6 x 1024^2 (48 MiB) 62.7 / 61.4; beyond the limit 7 x 1024^2
+// 69.1 / 74.5, 12 x 1024^2 109 / 112, 28 x 1024^2 (235 MB) 280 / 298 us.
 // Stores of fewer contiguous bytes than a line leave in as many pieces: 64 bytes
 // (rows of 8 lanes, tiles of 8 columns) go through up to WRITE_THROUGH, 16 and 32
 // up to WRITE_THROUGH_NARROW, single points never.  Whole calls with all stores
@@ -170,8 +174,11 @@ struct LineCfg {
   // or two lines, take the small plan: few points per lane, FP64 exchanges
   // up to 1024 points, twiddles kept.  Per step, default against small plan:
   // 250 lines of 1024 4.2 -> 3.0 us (pairs 11.3 -> 5.9), 200 of 256 3.1 ->
-  // 1.25, of 512 3.9 -> 2.0, of 2048 4.9 -> 3.7 us; 2000 lines of 1024 9.8 ->
-  // 12.8, 400 of 2048 5.2 -> 7.1 us
+  // 1.25, of 512 3.9 -> 2.0, of 2048 4.9 -> 3.7 us.  300 steps at and past the
+  // limits, default / small plan, ms: 64 points 8192 lines 1.35 / 0.93, 12000 1.44 /
+  // 1.32; 256: 2048 1.26 / 0.97, 2500 1.27 / 1.38; 512: 1024 1.52 / 1.05, 2048
+  // 1.57 / 1.84, 2500 2.79 / 2.57; 1024: 512 1.57 / 1.43, 600 1.56 / 2.12; 2048: 256
+  // 1.88 / 1.33, 300 1.88 / 2.39
   static constexpr int P1 = N >= 16 ? 16 : N;
   static constexpr int LPB1D1 = lines_per_block(256, N / P1);
   static constexpr int LPB1D2 = lines_per_block(128, N / P1);
@@ -305,7 +312,7 @@ static int nlc_launch(int stage, const NlcArgs& a, hipStream_t s) {
 }
 
 // The default tile: at most the widest of one column per thread (4096^2, tile of 8
-// columns, four per thread, against 4: column sweep 144 -> 131 us).
+// columns, four per thread, against 4: column sweep 144 -> 115 us).
 template <int N>
 constexpr int col_width_default() {
   int w = LineCfg<N>::WDEF;
