@@ -239,11 +239,11 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_nlc_nl(NlcArgs a) {
   }
 
   float vr[P], vi[P];
-  auto load_row_v = [&](uint32_t y) {
+  auto load_row_v = [&](uint32_t y) __attribute__((always_inline)) {
     load_v_set<P, T, GEN>(a.V, a.vkind, L.item0 * a.v_item_stride + (int64_t)L.yp0 * N,
                      (L.item - L.item0) * (uint32_t)a.v_item_stride + (y - L.yp0) * N + t, vr, vi);
   };
-  auto finish_line = [&](float2 (&w)[1][P], uint32_t c1) {
+  auto finish_line = [&](float2 (&w)[1][P], uint32_t c1) __attribute__((always_inline)) {
     if (a.forward_last) fft_line<N, P, 1, false, 1, NLSE_ROW_PADSH, F64, SYNC>(w, t, W, tw, lline, LINE);
     if (a.out_scale != 1.f) {
 #pragma unroll

@@ -400,7 +400,7 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
 #pragma unroll
       for (int m = 0; m < P; ++m) v[g][m] = make_float2(v[g][m].x * a.out_scale, v[g][m].y * a.out_scale);
   }
-  auto put = [&](auto st) {
+  auto put = [&](auto st) __attribute__((always_inline)) {
     constexpr int ST = decltype(st)::value;
     float2* const out = BIG ? big_at() : nullptr;
 #pragma unroll
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(WT*(N / P)) void k_colu(ColArgs a) {
     bool act, two;
     uint32_t da, db;
   };
-  auto unit = [&]() {
+  auto unit = [&]() __attribute__((always_inline)) {
     const uint32_t id = opaque(threadIdx.x);
     Unit u;
     const int j0 = jt + (int)(id % WT);
@@ -634,7 +634,11 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_line1d(Line1DArgs a) {
   RabiParams rb{};
   if (has_rabi) rb = a.rabi[item];
 
-  auto apply_nl = [&](const NL (&p)[G]) {
+  // Always inlined: left to the compiler, pairs of lines of 16 points per lane had
+  // it as a function of its own, on a line in memory, and took twice as long (600
+  // pairs of 1024, 200 steps: 2.8 -> 5.1 ms).  Two copies, for the local and the
+  // convolved intensities: one for both took 5-8 % longer at 4 points per lane.
+  auto apply_nl = [&](const NL (&p)[G]) __attribute__((always_inline)) {
     if (a.nlk != nullptr) {
       // nonlocal response: convolved intensities (nlse_1d.py:65-66 kernel)
       float I[G][P];

@@ -364,7 +364,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wrow(WRowArgs a) {
 #pragma unroll
   for (int m = 0; m < P; ++m) vf[m] = v_early ? reinterpret_cast<const float*>(a.V)[vbase + m * T] : 0.f;
 
-  auto put = [&]() {
+  auto put = [&]() __attribute__((always_inline)) {
     if (!active) return;
 #pragma unroll
     for (int g = 0; g < G; ++g)
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wrow(WRowArgs a) {
   // nonlinear application with the records `nlp`: intensities from the
   // convolved buffer (nonlocal response) or |A|^2, V' rounded per record
   const bool has_vi = a.vkind == V_CPLX || a.vkind == V_CPLX128;
-  auto nl_pass = [&](const void* nlp, bool use_ic) {
+  auto nl_pass = [&](const void* nlp, bool use_ic) __attribute__((always_inline)) {
     double I[G][P], vr[P], vi[P];
 #pragma unroll
     for (int g = 0; g < G; ++g)
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(LPB*(N / P)) void k_wline1d(WLine1DArgs a) {
 #pragma unroll
   for (int m = 0; m < P; ++m) vf[m] = a.vkind == V_REAL ? reinterpret_cast<const float*>(a.V)[t + m * T] : 0.f;
 
-  auto apply_nl = [&](const void* prm) {
+  auto apply_nl = [&](const void* prm) __attribute__((always_inline)) {
     double I[G][P];
     if (a.nlk != nullptr) {
       // convolved intensities (nlse_1d.py:65-66 kernel), FP64
