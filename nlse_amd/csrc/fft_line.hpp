@@ -236,9 +236,10 @@ __device__ __forceinline__ void bf2(double2 e, double2 o, bool mi, double2& x0, 
 template <int R, int K>
 constexpr double2 const_ct() {
   static_assert(K > 0 && K < R / 4 && R <= 16, "W8, W16, W16^3");
-  // (the tangents of the rounded cosines, as in the tables)
+  // (the tangents of the rounded cosines, as in the tables; 1 for W8, whose parts
+  // then have one rounding in common and whose products are additions)
   constexpr double c = R == 8 || K == 2 ? K_R2 : (K == 1 ? K_C8 : K_S8);
-  constexpr double t = R == 8 || K == 2 ? 0.9999999999999999 : (K == 1 ? 0.41421356237309503 : 2.414213562373095);
+  constexpr double t = R == 8 || K == 2 ? 1.0 : (K == 1 ? 0.41421356237309503 : 2.414213562373095);
   return double2{c, -t};
 }
 

@@ -326,15 +326,16 @@ __device__ __forceinline__ void col_body(const ColArgs& a, int64_t b, xchg_t<FA>
   constexpr bool PAIRED = G == 2 && NLSE_COL_PAIRED;
   constexpr int CS = PAIRED ? 1 : WT;
   const int u0 = (int)((uint32_t)b - slab * tiles) * TILE;  // uniform: first column of the tile
-  const int c0 = u0 + (PAIRED ? G * cw : cw);
+  const int cl = PAIRED ? G * cw : cw;  // this thread's first column in the tile
+  const int c0 = u0 + cl;
   // slabs below 4 GiB are addressed from a uniform descriptor (the launcher
   // chooses)
   float2* const A0 = a.A + (int64_t)slab * N * a.NX + u0;
   // (BIG: the lane's 64-bit address, found again for the stores)
-  auto big_at = [&]() { return A0 + (int64_t)opaque((uint32_t)t) * a.NX + (c0 - u0); };
+  auto big_at = [&]() { return A0 + (int64_t)opaque((uint32_t)t) * a.NX + cl; };
   const Buf AB(A0), tw(a.tw);
   const uint32_t rs = 8u * (uint32_t)T * (uint32_t)a.NX;
-  const uint32_t d = 8u * ((uint32_t)t * (uint32_t)a.NX + (uint32_t)(c0 - u0));
+  const uint32_t d = 8u * ((uint32_t)t * (uint32_t)a.NX + (uint32_t)cl);
   xchg_t<FA>* lline = lds + cw * GR * LINE;
 
   float2 v[G][P];
